@@ -532,7 +532,7 @@ int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu
     const int segs[] = {8, 16, 32};
     double ms[K_NKINDS];
     double bj = 1e300, bk = 1e300;
-    int sj = PSWEEP_SEG_DEFAULT, sk = PSWEEP_SEG_DEFAULT;
+    int sj = segs[0], sk = segs[0];
     for (int sgm : segs) {
       if (raishin_model_set_sweep_tiles(m, 0, sgm, sgm) != 0 || !time_kinds(m, uri, uu, time, steps, ms)) return -1;
       if (ms[K_SWEEP2] < bj) { bj = ms[K_SWEEP2]; sj = sgm; }

@@ -148,56 +148,69 @@ __global__ void __launch_bounds__(1024) k_sum_counters(unsigned long long* __res
 // Shape coefficients of the cell: flattening f2 (rec.f90:1736-1858) and the
 // contact-steepening eta of the density (rec.f90:1537-1629).  R is the
 // arithmetic type (double: the reference's; float: the mixed-precision form).
+// One cell's shock indicator (flaten, rec.f90:1736-1830) from the pressure at
+// +-1 and +-2 and the velocity along D at +-1.
+template <class R>
+RH_DEV R ppm_f1(R pm2, R pm1, R pp1, R pp2, R vm1, R vp1) {
+  const R t3a = absr(pp1 - pm1);
+  const R t1 = R(1) * fminf_(pp1, pm1) - t3a;
+  const R t2 = vp1 - vm1;
+  const R omg1 = (t1 < R(0) && t2 < R(0)) ? R(1) : R(0);
+  const R t3b = (pp2 - pm2);
+  R t4;
+  if (t3b == R(0)) t4 = (t3a == R(0)) ? R(-0.52) : R(1.0) - R(0.52);
+  else t4 = (t3a / t3b) - R(0.52);
+  return fminf_(R(1), omg1 * fmaxf_(R(0), t4 * R(10.0)));
+}
+
+// f2 of a cell from the indicators of its neighbours and its own
+// (rec.f90:1831-1858).
+template <class R>
+RH_DEV R ppm_f2(R f1m, R f10, R f1p, R p5m, R p5p) {
+  const R f1b = (p5p - p5m < R(0)) ? f1p : f1m;
+  return fmaxf_(f10, f1b);
+}
+
+// Steepening eta of the density (detect, rec.f90:1537-1629) from the second
+// differences of the two neighbouring cells; xm, x0, xp: cell positions.
+template <class R>
+RH_DEV R ppm_eta(R ddm, R ddp, R um1, R up1, R p5m, R p5p, R xm, R x0, R xp, R gam) {
+  const R t1 = ddp * ddm;
+  const R t2 = mad_(-R(0.1), fminf_(absr(up1), absr(um1)), absr(up1 - um1));
+  R etatil;
+  if (t1 >= R(0) && t2 <= R(0)) etatil = R(0);
+  else {
+    const R t2a = -(ddp - ddm) / (xp - xm);
+    const R dl = x0 - xm, dr = xp - x0;
+    const R t2b = mad_(dr * dr, dr, dl * dl * dl) / (up1 - um1);
+    etatil = t2a * t2b;
+  }
+  R eta = fmaxf_(R(0), fminf_(R(5.0) * (etatil - R(0.05)), R(1)));
+  const R t3 = absr(up1 - um1) / fminf_(up1, um1);
+  const R t4 = absr(p5p - p5m) / fminf_(p5p, p5m);
+  if (gam * R(1) * t3 < t4) eta = R(0);
+  return eta;
+}
+
 template <int D, class R>
 RH_DEV void ppm_shape(const double* __restrict__ W, long long N, long long c, long long s, int p,
                       const double* __restrict__ dxs, const double* __restrict__ xs, R gam, R& f2_out, R& eta_out) {
   const R dm2 = R(dxs[p - 2]), dm1 = R(dxs[p - 1]), d0 = R(dxs[p]), dp1 = R(dxs[p + 1]), dp2 = R(dxs[p + 2]);
-  // --- flattening coefficient f2 of this cell ---
   const int VEL = D;  // velocity component along D is variable D+1 (0-based D)
   const double* P5 = W + 4 * N + c;
   const double* PV = W + (long long)VEL * N + c;
   R f1[3];
 #pragma unroll
-  for (int q = -1; q <= 1; q++) {
-    const R pp1 = R(P5[(q + 1) * s]), pm1 = R(P5[(q - 1) * s]), pp2 = R(P5[(q + 2) * s]), pm2 = R(P5[(q - 2) * s]);
-    const R t3a = absr(pp1 - pm1);
-    const R t1 = R(1) * fminf_(pp1, pm1) - t3a;
-    const R t2 = R(PV[(q + 1) * s]) - R(PV[(q - 1) * s]);
-    const R omg1 = (t1 < R(0) && t2 < R(0)) ? R(1) : R(0);
-    const R t3b = (pp2 - pm2);
-    R t4;
-    if (t3b == R(0)) t4 = (t3a == R(0)) ? R(-0.52) : R(1.0) - R(0.52);
-    else t4 = (t3a / t3b) - R(0.52);
-    f1[q + 1] = fminf_(R(1), omg1 * fmaxf_(R(0), t4 * R(10.0)));
-  }
+  for (int q = -1; q <= 1; q++)
+    f1[q + 1] = ppm_f1<R>(R(P5[(q - 2) * s]), R(P5[(q - 1) * s]), R(P5[(q + 1) * s]), R(P5[(q + 2) * s]),
+                          R(PV[(q - 1) * s]), R(PV[(q + 1) * s]));
   const R p5p = R(P5[s]), p5m = R(P5[-s]);
-  const R f1b = (p5p - p5m < R(0)) ? f1[2] : f1[0];
-  f2_out = fmaxf_(f1[1], f1b);
-
-  // --- contact steepening parameter eta (density only) ---
-  R eta;
-  {
-    const double* P1 = W + c;
-    const R um2 = R(P1[-2 * s]), um1 = R(P1[-s]), u0 = R(P1[0]), up1 = R(P1[s]), up2 = R(P1[2 * s]);
-    const R ddm = (R(1) / (dm2 + dm1 + d0)) * ((u0 - um1) / (d0 + dm1) - (um1 - um2) / (dm1 + dm2));
-    const R ddp = (R(1) / (d0 + dp1 + dp2)) * ((up2 - up1) / (dp2 + dp1) - (up1 - u0) / (dp1 + d0));
-    const R t1 = ddp * ddm;
-    const R t2 = mad_(-R(0.1), fminf_(absr(up1), absr(um1)), absr(up1 - um1));
-    R etatil;
-    if (t1 >= R(0) && t2 <= R(0)) etatil = R(0);
-    else {
-      const R xm = R(xs[p - 2]), x0 = R(xs[p - 1]), xp = R(xs[p]);
-      const R t2a = -(ddp - ddm) / (xp - xm);
-      const R dl = x0 - xm, dr = xp - x0;
-      const R t2b = mad_(dr * dr, dr, dl * dl * dl) / (up1 - um1);
-      etatil = t2a * t2b;
-    }
-    eta = fmaxf_(R(0), fminf_(R(5.0) * (etatil - R(0.05)), R(1)));
-    const R t3 = absr(up1 - um1) / fminf_(up1, um1);
-    const R t4 = absr(p5p - p5m) / fminf_(p5p, p5m);
-    if (gam * R(1) * t3 < t4) eta = R(0);
-  }
-  eta_out = eta;
+  f2_out = ppm_f2<R>(f1[0], f1[1], f1[2], p5m, p5p);
+  const double* P1 = W + c;
+  const R um2 = R(P1[-2 * s]), um1 = R(P1[-s]), u0 = R(P1[0]), up1 = R(P1[s]), up2 = R(P1[2 * s]);
+  const R ddm = (R(1) / (dm2 + dm1 + d0)) * ((u0 - um1) / (d0 + dm1) - (um1 - um2) / (dm1 + dm2));
+  const R ddp = (R(1) / (d0 + dp1 + dp2)) * ((up2 - up1) / (dp2 + dp1) - (up1 - u0) / (dp1 + d0));
+  eta_out = ppm_eta<R>(ddm, ddp, um1, up1, p5m, p5p, R(xs[p - 2]), R(xs[p - 1]), R(xs[p]), gam);
 }
 
 // interp's width-only coefficients of a cell at index p (ppm_coefficients on
@@ -229,35 +242,32 @@ RH_DEV void ppm_coef(const double* __restrict__ pc, long long npc, int p, PpmCoe
 // u = (u(p-2) .. u(p+2)): interp (rec.f90:1309-1476), steepening of the
 // density (rec.f90:1661-1677), flattening and monoto (rec.f90:1887-2056).
 // l = uri*r(c-1), r = uri*l(c).
+// dma of a cell (rec.f90:1338-1414): the limited slope from its neighbours.
 template <int D, class R>
-RH_DEV void ppm_var(const R u[5], const PpmCoef<R>& k, int n, R f2, R eta, R& l_out, R& r_out) {
-  auto dma_of = [&](R um, R u0, R up, int o) -> R {
-    const R t1a = k.ta[o], t1b = k.tb[o], t1c = k.tc[o];
-    const R sp1 = (up - u0);
-    const R sm1 = (u0 - um);
-    const R spm1 = sp1 * sm1;
-    const R da = t1a * mad_(t1b, sp1, t1c * sm1);
-    if (spm1 <= R(0)) return R(0);
-    const R t1 = (da < R(0)) ? R(-1) : R(1);
-    const R t1d = fminf_(absr(sm1), absr(sp1));
-    if (D == 3) return t1 * fminf_(absr(da), t1d);   // rec.f90:1414
-    return t1 * fminf_(absr(da), R(2.0) * t1d);
-  };
-  auto eq51 = [&](R uq, R uq1, R dmq, R dmq1, int o) -> R {
-    // uq + t2 + t3 - e4 dmq1 + e5 dmq with t2 = e2 (uq1 - uq), t3 = e3 (uq1 - uq)
-    const R du = uq1 - uq;
-    return mad_(k.e5[o], dmq, mad_(-k.e4[o], dmq1, mad_(k.e3[o], du, mad_(k.e2[o], du, uq))));
-  };
-  const R um2 = u[0], um1 = u[1], u0 = u[2], up1 = u[3], up2 = u[4];
-  const R dmm1 = dma_of(um2, um1, u0, 0);
-  const R dm0 = dma_of(um1, u0, up1, 1);
-  const R dmp1 = dma_of(u0, up1, up2, 2);
-  R r = eq51(u0, up1, dm0, dmp1, 0);          // value at p+1/2
-  R l = eq51(um1, u0, dmm1, dm0, 1);          // value at p-1/2
-  if (n == 0) {
-    r = mad_(r, R(1) - eta, mad_(-R(0.5), dmp1, up1) * eta);
-    l = mad_(l, R(1) - eta, mad_(R(0.5), dmm1, um1) * eta);
-  }
+RH_DEV R ppm_dma(R um, R u0, R up, R t1a, R t1b, R t1c) {
+  const R sp1 = (up - u0);
+  const R sm1 = (u0 - um);
+  const R spm1 = sp1 * sm1;
+  const R da = t1a * mad_(t1b, sp1, t1c * sm1);
+  if (spm1 <= R(0)) return R(0);
+  const R t1 = (da < R(0)) ? R(-1) : R(1);
+  const R t1d = fminf_(absr(sm1), absr(sp1));
+  if (D == 3) return t1 * fminf_(absr(da), t1d);   // rec.f90:1414
+  return t1 * fminf_(absr(da), R(2.0) * t1d);
+}
+
+// Equation (51) (rec.f90:1427-1476): the value at the face between the cells
+// q and q+1, uq + t2 + t3 - e4 dmq1 + e5 dmq with t2 = e2 (uq1 - uq),
+// t3 = e3 (uq1 - uq).
+template <class R>
+RH_DEV R ppm_eq51(R uq, R uq1, R dmq, R dmq1, R e2, R e3, R e4, R e5) {
+  const R du = uq1 - uq;
+  return mad_(e5, dmq, mad_(-e4, dmq1, mad_(e3, du, mad_(e2, du, uq))));
+}
+
+// Flattening and monoto (rec.f90:1887-2056) of a cell's two face values.
+template <class R>
+RH_DEV void ppm_monoto(R u0, R f2, R& l, R& r) {
   r = mad_(u0, f2, r * (R(1) - f2));
   l = mad_(u0, f2, l * (R(1) - f2));
   if ((r - u0) * (l - u0) >= R(0)) { r = u0; l = u0; }            // equation (73)
@@ -265,6 +275,21 @@ RH_DEV void ppm_var(const R u[5], const PpmCoef<R>& k, int n, R f2, R eta, R& l_
   const R t4 = (r - l) * (r - l);
   if (t3 > t4) l = mad_(R(3.0), u0, -(R(2.0) * r));
   if (-t3 > t4) r = mad_(R(3.0), u0, -(R(2.0) * l));
+}
+
+template <int D, class R>
+RH_DEV void ppm_var(const R u[5], const PpmCoef<R>& k, int n, R f2, R eta, R& l_out, R& r_out) {
+  const R um2 = u[0], um1 = u[1], u0 = u[2], up1 = u[3], up2 = u[4];
+  const R dmm1 = ppm_dma<D, R>(um2, um1, u0, k.ta[0], k.tb[0], k.tc[0]);
+  const R dm0 = ppm_dma<D, R>(um1, u0, up1, k.ta[1], k.tb[1], k.tc[1]);
+  const R dmp1 = ppm_dma<D, R>(u0, up1, up2, k.ta[2], k.tb[2], k.tc[2]);
+  R r = ppm_eq51<R>(u0, up1, dm0, dmp1, k.e2[0], k.e3[0], k.e4[0], k.e5[0]);   // value at p+1/2
+  R l = ppm_eq51<R>(um1, u0, dmm1, dm0, k.e2[1], k.e3[1], k.e4[1], k.e5[1]);   // value at p-1/2
+  if (n == 0) {
+    r = mad_(r, R(1) - eta, mad_(-R(0.5), dmp1, up1) * eta);
+    l = mad_(l, R(1) - eta, mad_(R(0.5), dmm1, um1) * eta);
+  }
+  ppm_monoto<R>(u0, f2, l, r);
   l_out = l;
   r_out = r;
 }
@@ -363,8 +388,8 @@ RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, long long blk) {
 // Face physics and HLLE of interface c+1/2 along D from its two face states
 // (wl: the left cell's right edge, wr: the right cell's left edge):
 // caluu3 -> calflx3 -> calcha -> hlle, written to F (and the transverse B
-// fluxes to their CTsrc planes).
-template <int D, class R, int ICHA>
+// fluxes to their CTsrc planes).  SAME: the two face states are the same.
+template <int D, class R, int ICHA, bool SAME = false>
 RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, long long c, int i, int j, int k,
                        const Met& M, R gam, const R wl[9], const R wr[9]) {
   const long long N = G.N;
@@ -378,8 +403,11 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
     tmunu_row<R>(sl, D, detg, pw, Fl);
     face_speed<R, ICHA>(sl, D, gam, M, vpl, vml);
   }
-  R Ur[9], Fr[9], vpr, vmr;
-  {
+  R Ur[9], Fr[9], vpr = vpl, vmr = vml;
+  if constexpr (SAME) {
+#pragma unroll
+    for (int n = 0; n < 9; n++) { Ur[n] = Ul[n]; Fr[n] = Fl[n]; }
+  } else {
     PrelT<R> sr;
     prelude<R>(wr, gam, M, sr);
     const R pw = powr(sr.de, gam);
@@ -480,114 +508,189 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
 }
 
 // ------------------------------------------------------------------------
-// PPM direction sweep with its face values computed in the same kernel:
-// each cell's edges (interp, detect, flaten, monoto; rec.f90:1261-2056) are
-// written to LDS and the interface physics (caluu3 -> calflx3 -> calcha ->
-// hlle) reads them there, so the 18 edge planes never reach HBM.
-//  D = 1: a wave takes 64 consecutive cells of an i row; lane l's interface
-//         (the right face of its cell) takes the left edges of lane l+1's
-//         cell from LDS.  Consecutive waves of a row overlap by one cell.
-//  D = 2, 3: a wave holds 64 / A.seg consecutive i by A.seg consecutive
-//         cells along D; lane l's interface takes the left edges of the
-//         cell A.seg lanes further along D.  Waves overlap by one cell along D.
-// The arithmetic is that of k_ppm_edges followed by k_sweep (the same
-// functions), so the fluxes are the same bit for bit.
+// PPM direction sweep with its face values computed in the same kernel
+// (interp, detect, flaten, monoto; rec.f90:1261-2056, then caluu3 -> calflx3
+// -> calcha -> hlle), through LDS, so the 18 edge planes never reach HBM.
+//
+// A workgroup holds a tile of A.tp cells along D by blockDim.x / A.tp lines
+// across (D = 1: rows; D = 2, 3: consecutive i, so every load instruction
+// reads runs of contiguous values).  Everything that belongs to a cell or to
+// a face is computed by one lane and passed to the lanes beside it:
+//   1. each cell's limited slope of every variable, its shock indicator f1
+//      and its second difference of the density, from its +-1 (+-2) cells;
+//   2. the face value of equation (51) between the lane's cell and the next;
+//   3. the cell's two face values after steepening, flattening and monoto;
+//   4. the interface between the lane's cell and the next: own right edge,
+//      the next lane's left edge.
+// A tile of tp cells gives tp - 3 interfaces (the first cell lacks the face
+// below it, the last two the face above them or above the next cell), so
+// tiles overlap by three cells.  The lane's arithmetic is that of
+// k_ppm_edges followed by k_sweep on the same values (the pieces above), so
+// the fluxes are the same bit for bit; what a cell alone would compute three
+// times (slopes, indicators) or twice (face values) is computed once.
+// The entropy variable (plane 5) is not reconstructed: no flux reads its
+// face value.
+//
+// D = 0: the j sweep of a collapsed model.  Its one phi row is its own
+// neighbour, so every slope is zero, the face values are the cell's own
+// (not a number where the cell's value is infinite, as inf - inf makes the
+// slopes) and the two sides of each interface are the same state.
 // ------------------------------------------------------------------------
-// Edges of the cell at c (index p along D): left edges to lds[n*ld], right
-// edges to lds[(9+n)*ld].
-template <int D, class R>
-RH_DEV void ppm_edges_lds(const double* __restrict__ W, long long N, long long c, long long s, int p,
-                          const double* __restrict__ dxs, const double* __restrict__ xs,
-                          const double* __restrict__ pc, long long npc, R gam, R* lds, int ld) {
-  PpmCoef<R> kc;
-  ppm_coef<R>(pc, npc, p, kc);
-  R f2, eta;
-  ppm_shape<D, R>(W, N, c, s, p, dxs, xs, gam, f2, eta);
-  R cur[5], nxt[5];
-#pragma unroll
-  for (int o = 0; o < 5; o++) cur[o] = R(W[c + (o - 2) * s]);
-#pragma unroll 1
-  for (int n = 0; n < 9; n++) {
-    if (n < 8) {
-      const double* Pn = W + (long long)(n + 1) * N + c;
-#pragma unroll
-      for (int o = 0; o < 5; o++) nxt[o] = R(Pn[(o - 2) * s]);
-    }
-    R l, r;
-    ppm_var<D, R>(cur, kc, n, f2, eta, l, r);
-    lds[n * ld] = l;
-    lds[(9 + n) * ld] = r;
-#pragma unroll
-    for (int o = 0; o < 5; o++) cur[o] = nxt[o];
-  }
-}
+constexpr int PS_NV = 8;                                     // reconstructed variables
+RH_DEV constexpr int ps_plane(int q) { return q < 5 ? q : q + 1; }
 
 template <int D, class R, int ICHA>
 RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
-  extern __shared__ unsigned char rh_dyn_lds[];  // 18 planes of blockDim.x values of R
-  R* const L = reinterpret_cast<R*>(rh_dyn_lds);
-  const int bt = blockDim.x, tid = threadIdx.x, lane = tid & 63;
+  const int bt = blockDim.x, tid = threadIdx.x;
   const long long N = G.N;
   const double* __restrict__ W = A.W;
   R* __restrict__ F = (R*)A.F;
   R* __restrict__ CTsrc = (R*)A.CTsrc;
   const R gam = R(A.gam);
-  const int lj = jlo(G, G.nm0), hj = jhi(G, G.nj - G.nm0);
-  const long long wv = (blk * bt + tid) >> 6;
-  if (D == 1) {
-    const long long nic = (G.ni - 2 * G.nm0 + 1 + 62) / 63, cj = hj - lj + 1, ck = G.nk - 2 * G.nm0 + 1;
-    const long long ic = wv % nic, r = wv / nic;
-    const int j = lj + (int)(r % cj);
-    const long long kk = r / cj;
-    const int k = G.nm0 + (int)kk;
-    const int i = G.nm0 + (int)(ic * 63) + lane;
-    const bool cell_in = kk < ck && i <= G.ni - G.nm0 + 1;
-    const long long c = cell_in ? cidx(i, j, k, G) : 0;
-    if (cell_in) ppm_edges_lds<1, R>(W, N, c, 1, i, A.dxs, A.xs, A.pc, G.ni + 2, gam, L + tid, bt);
-    __syncthreads();  // every thread of the block reaches it: no early exit above
-    if (cell_in && lane < 63 && i <= G.ni - G.nm0) {
-      R wl[9], wr[9];
+  const unsigned nif_i = (unsigned)(G.ni - 2 * G.nm0 + 1), nif_k = (unsigned)(G.nk - 2 * G.nm0 + 1);
+  const int ihi = G.ni - G.nm0, jl = jlo(G, G.nm0), jh = jhi(G, G.nj - G.nm0);
+  if constexpr (D == 0) {
+    const unsigned t = (unsigned)blk * (unsigned)bt + (unsigned)tid;
+    const unsigned kk = t / nif_i;
+    if (kk >= nif_k) return;
+    const int i = G.nm0 + (int)(t - kk * nif_i), k = G.nm0 + (int)kk;
+    const long long c = cidx(i, jl, k, G);
+    R w[9];
 #pragma unroll
-      for (int n = 0; n < 9; n++) { wl[n] = L[(9 + n) * bt + tid]; wr[n] = L[n * bt + tid + 1]; }
-      const Met M{A.metF, G.P2, q2(i, k, G)};
-      sweep_face<1, R, ICHA>(G, F, CTsrc, c, i, j, k, M, gam, wl, wr);
+    for (int n = 0; n < 9; n++) {
+      const R u = n == 5 ? R(0) : R(W[(long long)n * N + c]);
+      w[n] = absr(u) == R(__builtin_inf()) ? R(__builtin_nan("")) : u;
     }
+    const Met M{A.metF, G.P2, q2(i, k, G)};
+    sweep_face<2, R, ICHA, true>(G, F, CTsrc, c, i, jl, k, M, gam, w, w);
     return;
   }
-  // D = 2, 3: a wave holds TI consecutive i (fastest) by TP = 64 / TI
-  // consecutive cells along D, so each load instruction reads TP runs of TI
-  // contiguous values; lane l's interface takes the left edges of lane
-  // l + TI's cell.  A wave's TP cells give TP - 1 interfaces (consecutive
-  // waves along D overlap by one cell).  A collapsed model's one phi row is
-  // its own neighbour along j (stride 0): there a wave holds 64 i of that
-  // row, and each interface takes both edges of its own cell.
-  const bool self = D == 2 && G.jfix;
-  const int TP = self ? 1 : A.seg, TI = 64 / TP, IPW = self ? 1 : TP - 1;
-  const int il = lane % TI, pl = lane / TI;
-  const int plo = (D == 2) ? lj : G.nm0, phi = (D == 2) ? hj : G.nk - G.nm0;
-  const int tlo = (D == 2) ? G.nm0 : lj, thi = (D == 2) ? G.nk - G.nm0 : hj;
-  const long long nig = (G.ni - 2 * G.nm0 + 1 + TI - 1) / TI;
-  const long long ndc = (phi - plo + 1 + IPW - 1) / IPW, ct = thi - tlo + 1;
-  // consecutive waves along i (a workgroup's waves share cache lines), then
-  // along D, then across (measured fastest for both directions: along k,
-  // walking j before the chunks keeps the face metric in L2 but loses more
-  // to the stencil rows)
-  const long long ig = wv % nig, r = wv / nig, dc = r % ndc, tt = r / ndc;
-  const int i = G.nm0 + (int)ig * TI + il;
-  const int p = plo + (int)dc * IPW + pl;
-  const int t = tlo + (int)tt;
-  const bool cell_in = tt < ct && dc < ndc && i <= G.ni - G.nm0 && p <= phi + (self ? 0 : 1);
-  const long long s = (D == 2) ? jstride(G) : kstride(G);
-  const long long npc = ((D == 2) ? G.nj : G.nk) + 2;
-  const long long c = cell_in ? ((D == 2) ? cidx(i, p, t, G) : cidx(i, t, p, G)) : 0;
-  if (cell_in) ppm_edges_lds<D, R>(W, N, c, s, p, A.dxs, A.xs, A.pc, npc, gam, L + tid, bt);
-  __syncthreads();  // every thread of the block reaches it: no early exit above
-  if (cell_in && (self || pl < TP - 1) && p <= phi) {
-    const int nb = self ? tid : tid + TI;
-    R wl[9], wr[9];
+  extern __shared__ unsigned char rh_dyn_lds[];  // 18 planes of blockDim.x values of R
+  R* const L = reinterpret_cast<R*>(rh_dyn_lds) + tid;
+  R* const Lv = L + 8 * bt;   // slopes, then left edges (L: cell values, then those of equation (51))
+  R* const Ls = L + 16 * bt;  // f1, second difference of the density
+  const int TP = A.tp, IPT = TP - 3;
+  const int phi = D == 1 ? ihi : D == 2 ? jh : G.nk - G.nm0;
+  // place in the tile: pl along D, il across; a step along D is `st` lanes
+  const int pl = D == 1 ? tid & ((1 << A.sh) - 1) : tid >> A.sh;
+  const int il = D == 1 ? tid >> A.sh : tid & ((1 << A.sh) - 1);
+  const int st = D == 1 ? 1 : 1 << A.sh;
+  const unsigned b = (unsigned)blk;
+  // the lane's cell (p: its index along D); lanes past the last line or the
+  // last cell that a needed slope reads (phi + 3, the grid's last but one)
+  // are clamped to it and write nothing
+  int i, j, k, p;
+  bool in;
+  if constexpr (D == 1) {
+    const unsigned rt = b / (unsigned)A.ndc, dc = b - rt * (unsigned)A.ndc;
+    const unsigned cj = (unsigned)(jh - jl + 1), rows = cj * nif_k;
+    unsigned row = rt * (unsigned)(bt / TP) + (unsigned)il;
+    in = row < rows;
+    row = in ? row : rows - 1;
+    const unsigned kk = row / cj;
+    j = jl + (int)(row - kk * cj);
+    k = G.nm0 + (int)kk;
+    p = G.nm0 - 1 + (int)dc * IPT + pl;
+    in = in && p <= phi;
+    if (p > phi + 3) p = phi + 3;
+    i = p;
+  } else {
+    // consecutive workgroups along i (their lines share cache lines); then,
+    // along j, the tiles of a k row; along k, the j of one k range, which
+    // share that range's face metric
+    const int TI = 1 << A.sh;
+    const unsigned r = b / (unsigned)A.nig, ig = b - r * (unsigned)A.nig;
+    const unsigned nin = D == 2 ? (unsigned)A.ndc : (unsigned)(jh - jl + 1), ro = r / nin, ri = r - ro * nin;
+    const unsigned tt = D == 2 ? ro : ri, dc = D == 2 ? ri : ro;
+    i = G.nm0 + (int)ig * TI + il;
+    in = i <= ihi;
+    if (!in) i = ihi;
+    p = (D == 2 ? jl : G.nm0) - 1 + (int)dc * IPT + pl;
+    in = in && p <= phi;
+    if (p > phi + 3) p = phi + 3;
+    j = D == 2 ? p : jl + (int)tt;
+    k = D == 2 ? G.nm0 + (int)tt : p;
+  }
+  const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
+  const long long c = cidx(i, j, k, G);
+  // the lane's own cell from memory, its neighbours from the lanes beside it
+  // (the tile's first and last cells read theirs)
+  const int nx = pl < TP - 1 ? st : 0, pv = pl > 0 ? -st : 0;
+  R um[PS_NV], u0[PS_NV], up[PS_NV], ue[PS_NV];
 #pragma unroll
-    for (int n = 0; n < 9; n++) { wl[n] = L[(9 + n) * bt + tid]; wr[n] = L[n * bt + nb]; }
-    const int j = (D == 2) ? p : t, k = (D == 2) ? t : p;
+  for (int q = 0; q < PS_NV; q++) u0[q] = R(W[(long long)ps_plane(q) * N + c]);
+  const bool edge = pl == 0 || pl == TP - 1;
+  if (edge) {
+    const long long ce = c + (pl == 0 ? -s : s);
+#pragma unroll
+    for (int q = 0; q < PS_NV; q++) ue[q] = R(W[(long long)ps_plane(q) * N + ce]);
+  }
+  // (the cell at phi + 3 has no second neighbour and needs no indicator)
+  const R pm2 = R(W[4 * N + c - 2 * s]), pp2 = R(W[4 * N + c + (p < phi + 3 ? 2 : 1) * s]);
+  const long long npc = ((D == 1) ? G.ni : (D == 2) ? G.nj : G.nk) + 2;
+  const double* __restrict__ pc = A.pc + p;
+#pragma unroll
+  for (int q = 0; q < PS_NV; q++) L[q * bt] = u0[q];
+  __syncthreads();  // every thread of the block reaches each of the four
+#pragma unroll
+  for (int q = 0; q < PS_NV; q++) {
+    um[q] = L[q * bt + pv];
+    up[q] = L[q * bt + nx];
+    if (pl == 0) um[q] = ue[q];
+    if (pl == TP - 1) up[q] = ue[q];
+  }
+  // 1. slopes, shock indicator, second difference of the density
+  R dm[PS_NV];
+  {
+    const R ta = R(pc[0]), tb = R(pc[npc]), tc = R(pc[2 * npc]);
+#pragma unroll
+    for (int q = 0; q < PS_NV; q++) {
+      dm[q] = ppm_dma<D, R>(um[q], u0[q], up[q], ta, tb, tc);
+      Lv[q * bt] = dm[q];
+    }
+    Ls[0] = ppm_f1<R>(pm2, um[4], up[4], pp2, um[D], up[D]);
+    const R dl = R(A.dxs[p - 1]), d0 = R(A.dxs[p]), dr = R(A.dxs[p + 1]);
+    Ls[bt] = (R(1) / (dl + d0 + dr)) * ((up[0] - u0[0]) / (dr + d0) - (u0[0] - um[0]) / (d0 + dl));
+  }
+  __syncthreads();
+  // 2. face value between this cell and the next
+  R V[PS_NV], dmp0 = R(0);
+  {
+    const R e2 = R(pc[3 * npc]), e3 = R(pc[4 * npc]), e4 = R(pc[5 * npc]), e5 = R(pc[6 * npc]);
+#pragma unroll
+    for (int q = 0; q < PS_NV; q++) {
+      const R dmp = Lv[q * bt + nx];
+      if (q == 0) dmp0 = dmp;
+      V[q] = ppm_eq51<R>(u0[q], up[q], dm[q], dmp, e2, e3, e4, e5);
+      L[q * bt] = V[q];
+    }
+  }
+  const R dmm0 = Lv[pv], f1m = Ls[pv], f10 = Ls[0], f1p = Ls[nx], ddm = Ls[bt + pv], ddp = Ls[bt + nx];
+  __syncthreads();
+  // 3. the cell's face values: left edges to LDS, right edges kept
+  R wl[9], wr[9];
+  {
+    const R f2 = ppm_f2<R>(f1m, f10, f1p, um[4], up[4]);
+    const R eta = ppm_eta<R>(ddm, ddp, um[0], up[0], um[4], up[4], R(A.xs[p - 2]), R(A.xs[p - 1]),
+                             R(A.xs[p]), gam);
+#pragma unroll
+    for (int q = 0; q < PS_NV; q++) {
+      R l = L[q * bt + pv], r = V[q];
+      if (q == 0) {
+        r = mad_(r, R(1) - eta, mad_(-R(0.5), dmp0, up[0]) * eta);
+        l = mad_(l, R(1) - eta, mad_(R(0.5), dmm0, um[0]) * eta);
+      }
+      ppm_monoto<R>(u0[q], f2, l, r);
+      Lv[q * bt] = l;
+      wl[ps_plane(q)] = r;
+    }
+  }
+  __syncthreads();
+  // 4. the interface
+  if (in && pl >= 1 && pl <= IPT) {
+#pragma unroll
+    for (int q = 0; q < PS_NV; q++) wr[ps_plane(q)] = Lv[q * bt + st];
+    wl[5] = wr[5] = R(0);
     const Met M{A.metF, G.P2, q2(i, k, G)};
     sweep_face<D, R, ICHA>(G, F, CTsrc, c, i, j, k, M, gam, wl, wr);
   }
@@ -2137,7 +2240,8 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const 
   return hipGetLastError();
 }
 
-// Fused PPM sweeps: variant = dir + 4*mixed + 64*icha (as the sweeps').
+// Fused PPM sweeps: variant = dir + 4*mixed + 64*icha (as the sweeps'), dir 0
+// the j sweep of a collapsed model.
 static int psweep_variant(int dir, bool mixed, int icha) { return dir + 4 * (int)mixed + 64 * icha; }
 
 template <class F>
@@ -2149,35 +2253,63 @@ static void with_psweep(int variant, F&& f) {
       if (mx) f(D, TypeTag<float>{}, C);
       else f(D, TypeTag<double>{}, C);
     };
-    if (d == 1) t(IC<1>{});
+    if (d == 0) t(IC<0>{});
+    else if (d == 1) t(IC<1>{});
     else if (d == 2) t(IC<2>{});
     else t(IC<3>{});
   });
 }
 
-// Waves of one fused PPM sweep (per model): D = 1, 64-cell chunks of the i
-// rows (63 interfaces each) over (j, k); D = 2, 3, tiles of 64 / seg i by
-// seg cells along D (seg - 1 interfaces) over the transverse axis.
-static long long psweep_waves(const Geo& G, int D, int seg) {
-  const long long nj = G.jfix ? 1 : (long long)(G.nj - 2 * G.nm0 + 1);
-  const long long ni = G.ni - 2 * G.nm0 + 1, nk = G.nk - 2 * G.nm0 + 1;
-  if (ni <= 0 || nj <= 0 || nk <= 0) return 0;
-  if (D == 1) return ((ni + 62) / 63) * nj * nk;
-  if (D == 2 && G.jfix) return ((ni + 63) / 64) * nk;  // one stored row: 64 i per wave
-  const long long along = D == 2 ? nj : nk, across = D == 2 ? nk : nj, ti = 64 / seg;
-  return ((along + seg - 2) / (seg - 1)) * ((ni + ti - 1) / ti) * across;
+// Interfaces of a fused PPM sweep along dir and the lines across it (D = 1:
+// rows; D = 2, 3: the i of one transverse index, and those indices).
+static void psweep_extent(const Geo& G, int dir, long long& along, long long& lines, long long& across) {
+  const long long ni = box(G.nm0, G.ni - G.nm0), nj = jbox(G, G.nm0, G.nj - G.nm0), nk = box(G.nm0, G.nk - G.nm0);
+  along = dir == 1 ? ni : dir == 2 ? nj : nk;
+  lines = dir == 1 ? nj * nk : ni;
+  across = dir == 1 ? 1 : dir == 2 ? nk : nj;
 }
 
-// The tile height in use along dir: the chosen one (or the default), but no
-// taller than the axis needs (the smallest power of two above its interface
-// count), so short axes (Riemann tubes' transverse axes) waste no lanes.
+// Tile of a fused PPM sweep along dir in workgroups of bt threads: tp cells
+// along the axis (3 of them overlap the next tile) by bt / tp lines.
+//  D = 1: the whole workgroup along the row, or 16, 32 or 64 cells of several
+//  rows, whichever leaves the fewest idle or overlapping lanes.
+//  D = 2, 3: a wave holds seg cells along the axis by 64 / seg consecutive i
+//  and the workgroup's waves are stacked along the axis.  seg as set by the
+//  caller, else the one with the fewest such lanes among runs of at least 4
+//  consecutive i along j and 16 along k (along j a tile's cells share their
+//  face metric; along k every (i, k) has its own, 33 values read in runs of
+//  64 / seg: 256x128x128 at seg 4, 8, 16 0.374, 0.377, 0.329 ms along j and
+//  0.396, 0.446, 0.444 ms along k); never taller than the axis needs (Riemann
+//  tubes' four transverse interfaces), never below the 4 cells that give an
+//  interface.
+static int psweep_tp(const Geo& G, int dir, int bt) {
+  long long along, lines, across;
+  psweep_extent(G, dir, along, lines, across);
+  auto lanes = [&](long long tp, long long ti) {
+    return ((along + tp - 4) / (tp - 3)) * tp * ((lines + ti - 1) / ti) * ti;
+  };
+  if (dir == 1) {
+    int best = bt;
+    for (int tp : {64, 32, 16})
+      if (tp < bt && lanes(tp, bt / tp) < lanes(best, bt / best)) best = tp;
+    return best;
+  }
+  const int nw = bt / 64;
+  int seg = G.seg[dir - 2];
+  if (!seg) {
+    seg = dir == 2 ? 16 : 4;
+    for (int sg : {8, 4, 2})
+      if (sg < seg && sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
+  }
+  while (seg > 1 && seg * nw / 2 >= 4 && seg * nw / 2 - 3 >= along) seg /= 2;
+  while (seg * nw < 4) seg *= 2;
+  return seg * nw;
+}
+
+// Cells along j or k that a wave of the sweep's tile holds.
 int psweep_segment(const Geo& G, int dir) {
-  const int want = (dir == 2 ? G.seg[0] : dir == 3 ? G.seg[1] : 0);
-  int s = want > 0 ? want : PSWEEP_SEG_DEFAULT;
-  const int n = dir == 2 ? (G.jfix ? 1 : G.nj - 2 * G.nm0 + 1) : dir == 3 ? G.nk - 2 * G.nm0 + 1 : 0;
-  int cap = 2;
-  while (cap < 64 && cap - 1 < n) cap *= 2;
-  return s < cap ? s : cap;
+  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
+  return psweep_tp(G, dir, bt) / (bt / 64);
 }
 
 size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads * (mixed ? sizeof(float) : sizeof(double)); }
@@ -2185,20 +2317,34 @@ size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads *
 hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* metF, const double* dxs,
                          const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,
                          hipStream_t st) {
-  const int seg = psweep_segment(G, dir);
-  const long long waves = psweep_waves(G, dir, seg);
-  PSweepArgs A{W, metF, dxs, xs, pc, gam, F, CTsrc, seg};
   const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
-  const unsigned nb = nblk(waves * 64, bt);
-  const int variant = psweep_variant(dir, mixed, G.icha);
+  long long along, lines, across;
+  psweep_extent(G, dir, along, lines, across);
+  const bool self = dir == 2 && G.jfix;  // one stored phi row: its own neighbour
+  PSweepArgs A{W, metF, dxs, xs, pc, gam, F, CTsrc, 0, 0, 0, 0};
+  long long n = 0;  // workgroups
+  if (self) {
+    n = (lines * across + bt - 1) / bt;
+  } else if (along > 0 && lines > 0 && across > 0) {
+    A.tp = psweep_tp(G, dir, bt);
+    const int ti = bt / A.tp;
+    // log2 of the lanes that vary fastest (D = 1 with the whole workgroup on one row: all)
+    const int fast = dir == 1 ? A.tp : ti;
+    A.sh = dir == 1 && ti == 1 ? 30 : __builtin_ctz((unsigned)fast);
+    A.nig = (int)((lines + ti - 1) / ti);
+    A.ndc = (int)((along + A.tp - 4) / (A.tp - 3));
+    n = (long long)A.nig * A.ndc * across;
+  }
+  const unsigned nb = (unsigned)n;
+  const int variant = psweep_variant(self ? 0 : dir, mixed, G.icha);
   if (g_rec) {
     AnyArgs a{};
     a.ps = A;
     record(LK_PSWEEP, variant, bt, nb, G, a);
     return hipSuccess;
   }
-  if (waves == 0) return hipSuccess;
-  const size_t lds = psweep_lds_bytes(bt, mixed);
+  if (n == 0) return hipSuccess;
+  const size_t lds = self ? 0 : psweep_lds_bytes(bt, mixed);
   with_psweep(variant, [&](auto D, auto T, auto C) {
     hipLaunchKernelGGL((k_psweep<D.value, typename decltype(T)::type, C.value>), dim3(nb), dim3(bt), lds, st, G, A);
   });
@@ -2344,7 +2490,7 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       });
       break;
     case LK_PSWEEP: {
-      const size_t lds = psweep_lds_bytes(threads, (variant & 4) != 0);
+      const size_t lds = (variant & 3) ? psweep_lds_bytes(threads, (variant & 4) != 0) : 0;
       with_psweep(variant, [&](auto D, auto T, auto C) {
         hipLaunchKernelGGL((kb_psweep<D.value, typename decltype(T)::type, C.value>), g, b, lds, st, it, n);
       });

@@ -80,7 +80,10 @@ struct PSweepArgs {
   const double *W, *metF, *dxs, *xs, *pc;  // pc: PPM width coefficients of the direction
   double gam;
   void *F, *CTsrc;  // element type: the sweep's arithmetic type
-  int seg;          // interfaces per lane along j or k
+  // tile: tp cells along the sweep's axis per workgroup, 2^sh lanes in the
+  // fastest direction (D = 1: along the row; else consecutive i); nig tiles
+  // across (D = 1: of rows, else of i), ndc along the axis
+  int tp, sh, nig, ndc;
 };
 
 struct CtArgs {
@@ -174,8 +177,8 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const 
 // kernel (through LDS): reads W and the direction's PPM width coefficients
 // pc, writes what launch_edges + launch_sweep write to F and CTsrc.
 // seg: cells along j or k per wave of the fused sweep (64 / seg consecutive
-// i per wave), a power of two from 2 to 64
-constexpr int PSWEEP_SEG_DEFAULT = 16;
+// i per wave; a workgroup's waves are stacked along the axis), a power of two
+// from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
 hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* metF, const double* dxs,
                          const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,

@@ -111,3 +111,21 @@ def test_autotuner_picks_tiles():
     same(ref, mod, "tuned")
     ref.close()
     mod.close()
+
+
+@pytest.mark.parametrize("threads", [64, 128, 192, 256])
+@pytest.mark.parametrize("ni,nj,nk,seg,mixed", [(17, 11, 12, 0, False), (72, 13, 30, 0, True), (75, 16, 71, 8, False)])
+def test_workgroup_tiles_equal_split(threads, ni, nj, nk, seg, mixed):
+    """The sweeps' workgroup tiles (rows of a workgroup or of 16, 32, 64
+    lanes along i; stacked waves along j and k) at extents one below, at and
+    above what a tile covers, against the split form."""
+    p = configs.Pram("tile", ni, nj, nk, irec=5, irkt=3, cfl=0.4)
+    a, b = make(p, mixed), make(p, mixed)
+    a.set_sweep_tiles(1, 0, 0)
+    b.set_block_sizes([threads] * 8)
+    b.set_sweep_tiles(0, seg, seg)
+    for s in range(2):
+        assert a.step(1) == b.step(1), s
+    same(a, b, threads)
+    a.close()
+    b.close()
