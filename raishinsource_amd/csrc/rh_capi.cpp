@@ -159,7 +159,7 @@ bool model_set_state(raishin_model* m, const double* uri, const double* uu, doub
       if (!upload(m->stage_aos, src(uu), 9 * N, m->st)) return false;
       HIPCHK(launch_aos_to_soa(m->stage_aos, m->Ucur, N, m->st));
     } else {
-      HIPCHK(launch_caluu1(m->G, m->W, m->met[0], m->p.gam, m->Ucur, m->st));  // main.f90:530
+      HIPCHK(launch_caluu1(m->G, m->W, m->metric_centre(), m->p.gam, m->Ucur, m->st));  // main.f90:530
     }
     double tdt[2] = {time, 0.0};
     HIPCHK(hipMemcpyAsync(m->tdt, tdt, 16, hipMemcpyHostToDevice, m->st));

@@ -8,6 +8,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #define RH_DEV __device__ __forceinline__
 
@@ -61,31 +62,83 @@ struct Geo {
   // reference's arithmetic: its HLLE keeps a dissipative normal-B flux that
   // flux-CT leaves alone); flux-CT then keeps div B at round-off
   unsigned short divb0;
+  unsigned short mk;       // 1: the metric pointers of the launches are compact tables (MetK)
 };
 
-// One metric location (centre or a face) from the (i,k) tables:
-// planes 0..15 gcov(m,n) at m+4n, 16..31 gcon, 32 sqrt(-g).
-struct Met {
+// One metric location (centre or a face) at one (i,k), in one of two table
+// forms (the model's: Geo::mk).  R is the arithmetic type the values are used
+// in.  Both give: g, gi (gcov, gcon), detg, the lapse alpha and its
+// reciprocal, the shift beta, and the spatial gcon3a's diagonal gi3 (cal3met,
+// coord.f90:970-1013; the spatial gcov3a is gcov itself).
+//
+// General tables: planes 0..15 gcov(m,n) at m+4n, 16..31 gcon, 32 sqrt(-g),
+// in double; what derives from them is computed where it is used.
+template <class R>
+struct MetG {
   const double* __restrict__ b;
   long long P2, q;
-  RH_DEV double g(int m, int n) const { return b[(long long)(m + 4 * n) * P2 + q]; }
-  RH_DEV double gi(int m, int n) const { return b[(long long)(16 + m + 4 * n) * P2 + q]; }
-  RH_DEV double detg() const { return b[32LL * P2 + q]; }
+  RH_DEV MetG(const void* tab, long long P2_, long long q_) : b((const double*)tab), P2(P2_), q(q_) {}
+  RH_DEV R g(int m, int n) const { return R(b[(long long)(m + 4 * n) * P2 + q]); }
+  RH_DEV R gi(int m, int n) const { return R(b[(long long)(16 + m + 4 * n) * P2 + q]); }
+  RH_DEV R detg() const { return R(b[32LL * P2 + q]); }
+  RH_DEV R alpha() const { return R(1) / sqrtr(-gi(0, 0)); }
+  RH_DEV R ralpha() const { return R(1) / alpha(); }
+  RH_DEV R beta(int n) const { const R a = alpha(); return a * a * gi(0, n); }
+  RH_DEV R gi3(int d) const { const R on = beta(d) / alpha(); return mad_(on, on, gi(d, d)); }
 };
+
+// Compact tables (k_compact_metric), for a metric that is symmetric bit for
+// bit, couples theta to nothing (g_t3 = g_13 = g_23 = 0, the same and the
+// t-phi entry of gcon zero) -- Kerr-Schild and Minkowski: the entries that
+// are left and the derived values, in the arithmetic type R.  The zeros stay
+// in the arithmetic as constants (a product with an infinity is still not a
+// number), so results are those of the general tables bit for bit; 13 planes
+// are read where the general form reads 33 and takes a square root and five
+// divisions (256x128x128: i, j, k sweeps 0.306, 0.330, 0.396 -> 0.288, 0.302,
+// 0.374 ms in FP64, 0.166, 0.198, 0.236 -> 0.136, 0.168, 0.202 ms mixed;
+// floors 0.305 -> 0.238, recovery 0.184 -> 0.163 ms).
+enum { MK_G00, MK_G01, MK_G02, MK_G11, MK_G12, MK_G22, MK_G33, MK_DETG, MK_ALPHA, MK_RALPHA, MK_BETA1,
+       MK_GI3_1, MK_GI3_2, MK_GI3_3, MK_FACE_PLANES,
+       MK_GI00 = MK_FACE_PLANES, MK_GI01, MK_GI11, MK_GI12, MK_GI22, MK_GI33, MK_PLANES };
+template <class R>
+struct MetK {
+  const R* __restrict__ b;
+  long long P2, q;
+  RH_DEV MetK(const void* tab, long long P2_, long long q_) : b((const R*)tab), P2(P2_), q(q_) {}
+  RH_DEV R at(int pl) const { return b[(long long)pl * P2 + q]; }
+  RH_DEV R g(int m, int n) const {
+    const int lo = m < n ? m : n, hi = m < n ? n : m;
+    if (hi == 3) return lo == 3 ? at(MK_G33) : R(0);
+    return at(lo == 0 ? MK_G00 + hi : lo == 1 ? MK_G11 + hi - 1 : MK_G22);
+  }
+  RH_DEV R gi(int m, int n) const {  // centre tables only
+    const int lo = m < n ? m : n, hi = m < n ? n : m;
+    if (hi == 3) return lo == 3 ? at(MK_GI33) : R(0);
+    if (lo == 0) return hi == 2 ? R(0) : at(MK_GI00 + hi);
+    return at(lo == 1 ? MK_GI11 + hi - 1 : MK_GI22);
+  }
+  RH_DEV R detg() const { return at(MK_DETG); }
+  RH_DEV R alpha() const { return at(MK_ALPHA); }
+  RH_DEV R ralpha() const { return at(MK_RALPHA); }
+  RH_DEV R beta(int n) const { return n == 1 ? at(MK_BETA1) : R(0); }
+  RH_DEV R gi3(int d) const { return at(MK_GI3_1 + d - 1); }
+};
+template <bool MK, class R>
+using MetOf = std::conditional_t<MK, MetK<R>, MetG<R>>;
 
 // physfunc.f90 helpers -------------------------------------------------
 // Templated on the arithmetic type R: double reproduces the reference; float
 // is the mixed-precision face arithmetic (metric values rounded to float).
 
 // calgfl: physfunc.f90:2-41
-template <class R>
-RH_DEV R calgfl(const R u1, const R u2, const R u3, const Met& M) {
+template <class R, class MT>
+RH_DEV R calgfl(const R u1, const R u2, const R u3, const MT& M) {
   const R ut[4] = {R(0), u1, u2, u3};
   R utsq = R(0);
 #pragma unroll
   for (int m = 1; m <= 3; m++)
 #pragma unroll
-    for (int n = 1; n <= 3; n++) utsq = mad_(R(M.g(m, n)) * ut[m], ut[n], utsq);
+    for (int n = 1; n <= 3; n++) utsq = mad_(M.g(m, n) * ut[m], ut[n], utsq);
   if (utsq < R(0)) {
     if (absr(utsq) <= R(1.0e-10)) utsq = absr(utsq);
     else utsq = R(1.0e-10);
@@ -95,31 +148,28 @@ RH_DEV R calgfl(const R u1, const R u2, const R u3, const Met& M) {
 }
 
 // calucon: physfunc.f90:44-74
-template <class R>
-RH_DEV void calucon(const R ut[4], R ucon[4], R gfl, const Met& M) {
-  const R alpha1 = R(1) / sqrtr(-R(M.gi(0, 0)));
-  const R b1 = alpha1 * alpha1 * R(M.gi(0, 1));
-  const R b2 = alpha1 * alpha1 * R(M.gi(0, 2));
-  const R b3 = alpha1 * alpha1 * R(M.gi(0, 3));
-  ucon[0] = gfl * (R(1) / alpha1);
-  ucon[1] = mad_(-(gfl * b1), R(1) / alpha1, ut[1]);
-  ucon[2] = mad_(-(gfl * b2), R(1) / alpha1, ut[2]);
-  ucon[3] = mad_(-(gfl * b3), R(1) / alpha1, ut[3]);
+template <class R, class MT>
+RH_DEV void calucon(const R ut[4], R ucon[4], R gfl, const MT& M) {
+  const R ra = M.ralpha();
+  ucon[0] = gfl * ra;
+  ucon[1] = mad_(-(gfl * M.beta(1)), ra, ut[1]);
+  ucon[2] = mad_(-(gfl * M.beta(2)), ra, ut[2]);
+  ucon[3] = mad_(-(gfl * M.beta(3)), ra, ut[3]);
 }
 
 // lower: physfunc.f90:158-192
-template <class R>
-RH_DEV void lower(const R v[4], R w[4], const Met& M) {
+template <class R, class MT>
+RH_DEV void lower(const R v[4], R w[4], const MT& M) {
 #pragma unroll
   for (int m = 0; m < 4; m++)
-    w[m] = mad_(R(M.g(m, 3)), v[3], mad_(R(M.g(m, 2)), v[2], mad_(R(M.g(m, 1)), v[1], R(M.g(m, 0)) * v[0])));
+    w[m] = mad_(M.g(m, 3), v[3], mad_(M.g(m, 2), v[2], mad_(M.g(m, 1), v[1], M.g(m, 0) * v[0])));
 }
 // upper: physfunc.f90:195-230
-template <class R>
-RH_DEV void upper(const R v[4], R w[4], const Met& M) {
+template <class R, class MT>
+RH_DEV void upper(const R v[4], R w[4], const MT& M) {
 #pragma unroll
   for (int m = 0; m < 4; m++)
-    w[m] = mad_(R(M.gi(m, 3)), v[3], mad_(R(M.gi(m, 2)), v[2], mad_(R(M.gi(m, 1)), v[1], R(M.gi(m, 0)) * v[0])));
+    w[m] = mad_(M.gi(m, 3), v[3], mad_(M.gi(m, 2), v[2], mad_(M.gi(m, 1), v[1], M.gi(m, 0) * v[0])));
 }
 
 // calbbcon: physfunc.f90:77-95
@@ -131,29 +181,6 @@ RH_DEV void calbbcon(const R bcon[4], R bb[4], const R ucov[4], const R ucon[4])
   bb[3] = mad_(bb[0], ucon[3], bcon[3]) * (R(1) / ucon[0]);
 }
 
-// cal3met: coord.f90:970-1013; g3/gi3 hold gcov3a/gcon3a(m,n) at (m-1)+3(n-1)
-template <class R>
-RH_DEV void cal3met(const Met& M, R g3[9], R gi3[9]) {
-  const R alpha1 = R(1) / sqrtr(-R(M.gi(0, 0)));
-  R beta1[4];
-  beta1[1] = alpha1 * alpha1 * R(M.gi(0, 1));
-  beta1[2] = alpha1 * alpha1 * R(M.gi(0, 2));
-  beta1[3] = alpha1 * alpha1 * R(M.gi(0, 3));
-  R oncon[4], oncov[4];
-  oncon[0] = R(1) / alpha1;
-  oncon[1] = beta1[1] / alpha1;
-  oncon[2] = beta1[2] / alpha1;
-  oncon[3] = beta1[3] / alpha1;
-  oncov[0] = -alpha1; oncov[1] = R(0); oncov[2] = R(0); oncov[3] = R(0);
-#pragma unroll
-  for (int m = 1; m <= 3; m++)
-#pragma unroll
-    for (int n = 1; n <= 3; n++) {
-      g3[(m - 1) + 3 * (n - 1)] = mad_(oncov[m], oncov[n], R(M.g(m, n)));
-      gi3[(m - 1) + 3 * (n - 1)] = mad_(oncon[m], oncon[n], R(M.gi(m, n)));
-    }
-}
-
 // Shared prelude of caluu1/caluu3/calflx3*/caltenr/calcha4*:
 // primitives -> enthalpy, Lorentz factor, u^mu, u_mu, b^mu, b_mu, b^2.
 template <class R>
@@ -163,18 +190,18 @@ struct PrelT {
 };
 using Prel = PrelT<double>;
 
-template <class R>
-RH_DEV void prelude(const R w[9], R gam, const Met& M, PrelT<R>& s) {
+template <class R, class MT>
+RH_DEV void prelude(const R w[9], R gam, const MT& M, PrelT<R>& s) {
   s.de = w[0];
   s.ut[0] = R(0); s.ut[1] = w[1]; s.ut[2] = w[2]; s.ut[3] = w[3];
   s.pr = w[4];
   s.bcon[0] = R(0); s.bcon[1] = w[6]; s.bcon[2] = w[7]; s.bcon[3] = w[8];
   s.roh = mad_(gam / (gam - R(1)), s.pr, s.de);   // caluu.f90:52 (ieos=0)
-  s.gfl = calgfl<R>(w[1], w[2], w[3], M);
-  calucon<R>(s.ut, s.ucon, s.gfl, M);
-  lower<R>(s.ucon, s.ucov, M);
+  s.gfl = calgfl(w[1], w[2], w[3], M);
+  calucon(s.ut, s.ucon, s.gfl, M);
+  lower(s.ucon, s.ucov, M);
   calbbcon<R>(s.bcon, s.bb, s.ucov, s.ucon);
-  lower<R>(s.bb, s.bbcov, M);
+  lower(s.bb, s.bbcov, M);
   s.bbsq = mad_(s.bb[3], s.bbcov[3], mad_(s.bb[2], s.bbcov[2], mad_(s.bb[1], s.bbcov[1], s.bb[0] * s.bbcov[0])));
 }
 
@@ -233,24 +260,21 @@ RH_DEV void speed_pair(R vd, R vsq, R omsq, R cssq, R vb, R rohb, R gfl, R gii, 
 }
 
 // v_i B^i with v_i = gcov3a v^j (lower1, physfunc.f90:233-258)
-template <class R>
-RH_DEV R v_dot_b(const R* g3, const R vcon[4], const R bcon[4]) {
+template <class R, class MT>
+RH_DEV R v_dot_b(const MT& M, const R vcon[4], const R bcon[4]) {
   R vcov[4];
 #pragma unroll
   for (int m = 1; m <= 3; m++)
-    vcov[m] = mad_(g3[(m - 1) + 6], vcon[3], mad_(g3[(m - 1) + 3], vcon[2], g3[(m - 1) + 0] * vcon[1]));
+    vcov[m] = mad_(M.g(m, 3), vcon[3], mad_(M.g(m, 2), vcon[2], M.g(m, 1) * vcon[1]));
   return mad_(vcov[3], bcon[3], mad_(vcov[2], bcon[2], vcov[1] * bcon[1]));
 }
 
 // Fast magnetosonic speeds along direction d for a face state:
 // calcha4i/j/k (calcha.f90:370-906).  The three directions write cs^2 and
 // vA^2 differently (calcha.f90:480,648,826 and 486,654,832).
-template <class R, int ICHA>
-RH_DEV void face_speed(const PrelT<R>& s, int d, R gam, const Met& M, R& vfp, R& vfm) {
-  const R alpha1 = R(1) / sqrtr(-R(M.gi(0, 0)));
-  const R beta_d = alpha1 * alpha1 * R(M.gi(0, d));
-  R g3[9], gi3[9];
-  cal3met<R>(M, g3, gi3);
+template <class R, int ICHA, class MT>
+RH_DEV void face_speed(const PrelT<R>& s, int d, R gam, const MT& M, R& vfp, R& vfm) {
+  const R alpha1 = M.alpha(), beta_d = M.beta(d);
   R vcon[4];
   vcon[1] = s.ut[1] * (R(1) / s.gfl);
   vcon[2] = s.ut[2] * (R(1) / s.gfl);
@@ -259,16 +283,16 @@ RH_DEV void face_speed(const PrelT<R>& s, int d, R gam, const Met& M, R& vfp, R&
 #pragma unroll
   for (int m = 1; m <= 3; m++)
 #pragma unroll
-    for (int n = 1; n <= 3; n++) vsq = mad_(g3[(m - 1) + 3 * (n - 1)] * vcon[m], vcon[n], vsq);
+    for (int n = 1; n <= 3; n++) vsq = mad_(M.g(m, n) * vcon[m], vcon[n], vsq);
   R cssq, vasq;
   if (d == 3) cssq = gam * s.pr * (R(1) / s.roh);
   else cssq = gam * s.pr / s.roh;
   if (d == 2) vasq = s.bbsq / (s.roh + s.bbsq);
   else vasq = s.bbsq * (R(1) / (s.roh + s.bbsq));
   const R omsq = mad_(cssq, R(1) - vasq, vasq);
-  const R vb = ICHA == 1 ? v_dot_b<R>(g3, vcon, s.bcon) : R(0);
+  const R vb = ICHA == 1 ? v_dot_b(M, vcon, s.bcon) : R(0);
   R p, m;
-  speed_pair<R, ICHA>(vcon[d], vsq, omsq, cssq, vb, s.roh + s.bbsq, s.gfl, gi3[(d - 1) * 4], p, m);
+  speed_pair<R, ICHA>(vcon[d], vsq, omsq, cssq, vb, s.roh + s.bbsq, s.gfl, M.gi3(d), p, m);
   p = mad_(alpha1, p, -beta_d);
   m = mad_(alpha1, m, -beta_d);
   if (absr(p) > R(1)) p = R(1);
@@ -277,15 +301,9 @@ RH_DEV void face_speed(const PrelT<R>& s, int d, R gam, const Met& M, R& vfp, R&
 }
 
 // Centre speeds for the CFL condition: calcha4 (calcha.f90:129-367).
-template <int ICHA>
-RH_DEV void centre_speeds(const Prel& s, double gam, const Met& M, double vp[4], double vm[4]) {
-  const double alpha1 = 1.0 / sqrtr(-M.gi(0, 0));
-  double beta1[4];
-  beta1[1] = alpha1 * alpha1 * M.gi(0, 1);
-  beta1[2] = alpha1 * alpha1 * M.gi(0, 2);
-  beta1[3] = alpha1 * alpha1 * M.gi(0, 3);
-  double g3[9], gi3[9];
-  cal3met(M, g3, gi3);
+template <int ICHA, class MT>
+RH_DEV void centre_speeds(const Prel& s, double gam, const MT& M, double vp[4], double vm[4]) {
+  const double alpha1 = M.alpha();
   double vcon[4];
   vcon[1] = s.ut[1] * (1.0 / s.gfl);
   vcon[2] = s.ut[2] * (1.0 / s.gfl);
@@ -294,18 +312,18 @@ RH_DEV void centre_speeds(const Prel& s, double gam, const Met& M, double vp[4],
 #pragma unroll
   for (int m = 1; m <= 3; m++)
 #pragma unroll
-    for (int n = 1; n <= 3; n++) vsq = vsq + g3[(m - 1) + 3 * (n - 1)] * vcon[m] * vcon[n];
+    for (int n = 1; n <= 3; n++) vsq = vsq + M.g(m, n) * vcon[m] * vcon[n];
   const double cssq = gam * s.pr / s.roh;
   const double vasq = s.bbsq * (1.0 / (s.roh + s.bbsq));
   const double omsq = vasq + cssq * (1.0 - vasq);
-  const double vb = ICHA == 1 ? v_dot_b<double>(g3, vcon, s.bcon) : 0.0;
+  const double vb = ICHA == 1 ? v_dot_b(M, vcon, s.bcon) : 0.0;
 #pragma unroll
   for (int d = 1; d <= 3; d++)
-    speed_pair<double, ICHA>(vcon[d], vsq, omsq, cssq, vb, s.roh + s.bbsq, s.gfl, gi3[(d - 1) * 4], vp[d], vm[d]);
+    speed_pair<double, ICHA>(vcon[d], vsq, omsq, cssq, vb, s.roh + s.bbsq, s.gfl, M.gi3(d), vp[d], vm[d]);
 #pragma unroll
   for (int d = 1; d <= 3; d++) {
-    vp[d] = alpha1 * vp[d] - beta1[d];
-    vm[d] = alpha1 * vm[d] - beta1[d];
+    vp[d] = alpha1 * vp[d] - M.beta(d);
+    vm[d] = alpha1 * vm[d] - M.beta(d);
     if (absr(vp[d]) > 1.0) vp[d] = 1.0;
     if (absr(vm[d]) > 1.0) vm[d] = -1.0;
   }

@@ -389,15 +389,15 @@ RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, long long blk) {
 // (wl: the left cell's right edge, wr: the right cell's left edge):
 // caluu3 -> calflx3 -> calcha -> hlle, written to F (and the transverse B
 // fluxes to their CTsrc planes).  SAME: the two face states are the same.
-template <int D, class R, int ICHA, bool SAME = false>
+template <int D, class R, int ICHA, bool SAME = false, class MT>
 RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, long long c, int i, int j, int k,
-                       const Met& M, R gam, const R wl[9], const R wr[9]) {
+                       const MT& M, R gam, const R wl[9], const R wr[9]) {
   const long long N = G.N;
-  const R detg = R(M.detg());
+  const R detg = M.detg();
   R Ul[9], Fl[9], vpl, vml;
   {
     PrelT<R> sl;
-    prelude<R>(wl, gam, M, sl);
+    prelude(wl, gam, M, sl);
     const R pw = powr(sl.de, gam);
     tmunu_row<R>(sl, 0, detg, pw, Ul);
     tmunu_row<R>(sl, D, detg, pw, Fl);
@@ -409,7 +409,7 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
     for (int n = 0; n < 9; n++) { Ur[n] = Ul[n]; Fr[n] = Fl[n]; }
   } else {
     PrelT<R> sr;
-    prelude<R>(wr, gam, M, sr);
+    prelude(wr, gam, M, sr);
     const R pw = powr(sr.de, gam);
     tmunu_row<R>(sr, 0, detg, pw, Ur);
     tmunu_row<R>(sr, D, detg, pw, Fr);
@@ -459,10 +459,9 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
 // averaging); inside the CT box fluxct then writes F itself.
 //
 // PPM's face values come from k_ppm_edges (E); MP5 and WENO5 reconstruct here.
-template <int D, int IREC, class R, int ICHA>
+template <int D, int IREC, class R, int ICHA, bool MK>
 RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
   const double* __restrict__ W = A.W;
-  const double* __restrict__ metF = A.metF;
   const R* __restrict__ E = (const R*)A.E;
   R* __restrict__ F = (R*)A.F;
   R* __restrict__ CTsrc = (R*)A.CTsrc;
@@ -503,7 +502,7 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
       }
     }
   }
-  const Met M{metF, G.P2, q2(i, k, G)};
+  const MetOf<MK, R> M(A.metF, G.P2, q2(i, k, G));
   sweep_face<D, R, ICHA>(G, F, CTsrc, c, i, j, k, M, gam, wl, wr);
 }
 
@@ -539,7 +538,7 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
 constexpr int PS_NV = 8;                                     // reconstructed variables
 RH_DEV constexpr int ps_plane(int q) { return q < 5 ? q : q + 1; }
 
-template <int D, class R, int ICHA>
+template <int D, class R, int ICHA, bool MK>
 RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
   const int bt = blockDim.x, tid = threadIdx.x;
   const long long N = G.N;
@@ -561,7 +560,7 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
       const R u = n == 5 ? R(0) : R(W[(long long)n * N + c]);
       w[n] = absr(u) == R(__builtin_inf()) ? R(__builtin_nan("")) : u;
     }
-    const Met M{A.metF, G.P2, q2(i, k, G)};
+    const MetOf<MK, R> M(A.metF, G.P2, q2(i, k, G));
     sweep_face<2, R, ICHA, true>(G, F, CTsrc, c, i, jl, k, M, gam, w, w);
     return;
   }
@@ -691,7 +690,7 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
 #pragma unroll
     for (int q = 0; q < PS_NV; q++) wr[ps_plane(q)] = Lv[q * bt + st];
     wl[5] = wr[5] = R(0);
-    const Met M{A.metF, G.P2, q2(i, k, G)};
+    const MetOf<MK, R> M(A.metF, G.P2, q2(i, k, G));
     sweep_face<D, R, ICHA>(G, F, CTsrc, c, i, j, k, M, gam, wl, wr);
   }
 }
@@ -753,7 +752,8 @@ RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, long long blk) {
 // ------------------------------------------------------------------------
 struct RecovOut { double w[9]; int fallback, fail, negrho, negp, vsqgt1, det0, guard, indep; };
 
-RH_DEV void recov_cell(const double u[9], const double wold[9], const Met& M, double gam, double dmin,
+template <class MT>
+RH_DEV void recov_cell(const double u[9], const double wold[9], const MT& M, double gam, double dmin,
                        double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool& carry,
                        RecovOut& o, double& wg_out) {
   const double safty = 1.0e-4, saftybig = 1.0e5, dv = 1.0e-2;
@@ -762,7 +762,7 @@ RH_DEV void recov_cell(const double u[9], const double wold[9], const Met& M, do
   o.fallback = o.fail = o.negrho = o.negp = o.vsqgt1 = o.det0 = o.guard = 0;
   double delta = 1.0, deltaend = 1.0e-7;
   int irecov = 0;
-  const double alpha1 = 1.0 / sqrt(-M.gi(0, 0));
+  const double alpha1 = M.alpha();
   const double detg1 = M.detg();
   const double dro = alpha1 * u[0] * (1.0 / detg1);
   double qcov[4], qcon[4], bcon[4], bcov[4], oncov[4], oncon[4];
@@ -981,7 +981,8 @@ RH_DEV void recov_cell(const double u[9], const double wold[9], const Met& M, do
 // quadratic has no admissible root is the previous cell's final W.  recov2
 // prints "vsq > 1.0" at every trip that clamps v^2; vsqgt1 counts them.
 // ------------------------------------------------------------------------
-RH_DEV void recov2_cell(const double u[9], const double wold[9], const Met& M, double gam, double dmin,
+template <class MT>
+RH_DEV void recov2_cell(const double u[9], const double wold[9], const MT& M, double gam, double dmin,
                         double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool& carry,
                         RecovOut& o, double& wg_out) {
   const double safty = 1.0e-5, dv = 1.0e-4;
@@ -991,7 +992,7 @@ RH_DEV void recov2_cell(const double u[9], const double wold[9], const Met& M, d
   double delta = 1.0;
   const double deltaend = 1.0e-8;
   int irecov = 0;
-  const double alpha1 = 1.0 / sqrt(-M.gi(0, 0));
+  const double alpha1 = M.alpha();
   const double detg1 = M.detg();
   const double dro = alpha1 * u[0] / detg1;
   double qcov[4], qcon[4], bcon[4], bcov[4], oncov[4], oncon[4];
@@ -1148,8 +1149,8 @@ RH_DEV void recov2_cell(const double u[9], const double wold[9], const Met& M, d
 }
 
 // one cell of the recovery iwvec selects
-template <int IW>
-RH_DEV void recov_any(const double u[9], const double wold[9], const Met& M, double gam, double dmin, double pmin,
+template <int IW, class MT>
+RH_DEV void recov_any(const double u[9], const double wold[9], const MT& M, double gam, double dmin, double pmin,
                       int iter, double x1pow15, double x1pow25, double wg_in, bool& carry, RecovOut& o,
                       double& wg_out) {
   if constexpr (IW == 2) recov2_cell(u, wold, M, gam, dmin, pmin, iter, x1pow15, x1pow25, wg_in, carry, o, wg_out);
@@ -1171,7 +1172,7 @@ RH_DEV long long chr_plane(int l, int a, int b) {
   return (long long)(l + 4 * a + 16 * b);
 }
 
-template <int STAGE, bool SYM, class FT>
+template <int STAGE, bool SYM, class FT, bool MK>
 RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
   const FT* __restrict__ F1 = (const FT*)A.F1;
   const FT* __restrict__ F2 = (const FT*)A.F2;
@@ -1194,7 +1195,7 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
     dt = A.cfl * dtcfl;
     a1 = dt / A.dx1b[i - 1]; a2 = dt / A.dx2b[j - 1]; a3 = dt / A.dx3b[k - 1];
   }
-  const Met M{A.metC, G.P2, q2(i, k, G)};
+  const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
 
   double w[9];
 #pragma unroll
@@ -1259,7 +1260,7 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
 // recov1a (recov.f90:578-1228) or recov2 (recov.f90:1919-2454) on every
 // interior cell from the stage's RK result; cells whose initial W is
 // inherited are flagged for k_recov_carry.
-template <int IW>
+template <int IW, bool MK>
 RH_DEV void b_recov(const Geo& G, const StageArgs& A, long long blk) {
   int i, j, k;
   const long long t = blk * blockDim.x + threadIdx.x;
@@ -1267,7 +1268,7 @@ RH_DEV void b_recov(const Geo& G, const StageArgs& A, long long blk) {
                  k))
     return;
   const long long N = G.N, c = cidx(i, j, k, G);
-  const Met M{A.metC, G.P2, q2(i, k, G)};
+  const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
   double w[9], u[9];
 #pragma unroll
   for (int n = 0; n < 9; n++) {
@@ -1452,18 +1453,20 @@ RH_DEV void b_bnd(const Geo& G, const PostArgs& A, long long blk) {
 // through, so its values are loaded again (from cache) in the next phase
 // instead of being held in registers across phases.  k_post's three phases
 // each read the 32 metric values; holding them costs two waves per SIMD.
-RH_DEV Met reload_met(const double* metC, const Geo& G, int i, int k) {
+template <bool MK>
+RH_DEV MetOf<MK, double> reload_met(const void* metC, const Geo& G, int i, int k) {
   asm volatile("" : "+s"(metC));
-  return Met{metC, G.P2, q2(i, k, G)};
+  return MetOf<MK, double>(metC, G.P2, q2(i, k, G));
 }
 
+template <bool MK>
 RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
   const long long t = blk * blockDim.x + threadIdx.x;
   int i, j, k;
   if (!box_index(t, 1, G.ni, jlo(G, 1), jhi(G, G.nj), 1, G.nk, i, j, k)) return;
   const long long N = G.N, c = cidx(i, j, k, G);
   const double gam = A.gam;
-  const Met M{A.metC, G.P2, q2(i, k, G)};
+  const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
   double w[9];
 #pragma unroll
   for (int n = 0; n < 9; n++) w[n] = A.Wpre[(long long)n * N + c];
@@ -1475,9 +1478,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
     vel[2] = w[2] * (1.0 / gfl);
     vel[3] = w[3] * (1.0 / gfl);
     if (vel[1] < 0.0) {
-      const double alpha1 = 1.0 / sqrt(-M.gi(0, 0));
-      const double beta1 = alpha1 * alpha1 * M.gi(0, 1);
-      vel[1] = beta1 * (1.0 / alpha1);
+      vel[1] = M.beta(1) * M.ralpha();
       double vsq = 0.0;
 #pragma unroll
       for (int m = 1; m <= 3; m++)
@@ -1517,10 +1518,8 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
   // pminmax2b: correction.f90:808-961
   bool scaled = false, hit = false;
   {
-    const Met M = reload_met(A.metC, G, i, k);
+    const auto M = reload_met<MK>(A.metC, G, i, k);
     const double gflmax = 20.0;
-    double g3[9], gi3[9];
-    cal3met(M, g3, gi3);
     double gfl = calgfl(w[1], w[2], w[3], M);
     double vel[4];
     vel[1] = w[1] * (1.0 / gfl);
@@ -1530,7 +1529,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
 #pragma unroll
     for (int m = 1; m <= 3; m++)
 #pragma unroll
-      for (int nn = 1; nn <= 3; nn++) vsq = vsq + g3[(m - 1) + 3 * (nn - 1)] * vel[m] * vel[nn];
+      for (int nn = 1; nn <= 3; nn++) vsq = vsq + M.g(m, nn) * vel[m] * vel[nn];
     if (vsq >= 1.0 || gfl > gflmax) vsq = 1.0 - 1.0 / (gflmax * gflmax);
     gfl = 1.0 / sqrt(1.0 - vsq);
     Prel s;
@@ -1568,7 +1567,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
   for (int n = 0; n < 9; n++) A.Wout[(long long)n * N + c] = w[n];
   // caluu1 (caluu.f90:2-126): conserved variables of the final primitives
   {
-    const Met M = reload_met(A.metC, G, i, k);
+    const auto M = reload_met<MK>(A.metC, G, i, k);
     Prel s2;
     prelude(w, gam, M, s2);
     double u[9];
@@ -1607,7 +1606,7 @@ RH_DEV long long wave_max_ll(long long v) {
   return v;
 }
 
-template <int ICHA>
+template <int ICHA, bool MK>
 RH_DEV void b_cfl(const Geo& G, const CflArgs& A, long long blk) {
   __shared__ long long s_last[4][4];
   __shared__ double s_min[4][4];
@@ -1617,7 +1616,7 @@ RH_DEV void b_cfl(const Geo& G, const CflArgs& A, long long blk) {
   bool valid = box_index(t, 2, G.ni - 1, jlo(G, 2), jhi(G, G.nj - 1), 2, G.nk - 1, i, j, k);
   if (valid) {
     const long long N = G.N, c = cidx(i, j, k, G);
-    const Met M{A.metC, G.P2, q2(i, k, G)};
+    const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
     double w[9];
 #pragma unroll
     for (int n = 0; n < 9; n++) w[n] = A.W[(long long)n * N + c];
@@ -1786,10 +1785,10 @@ RH_DEV long long carry_pred(const Geo& G, long long c, int& i, int& k) {
   return pk >= G.nm1 + 1 ? cidx(pi, pj, pk, G) : -1;
 }
 
-template <int IW>
+template <int IW, bool MK>
 RH_DEV void carry_cell(const Geo& G, const FixArgs& A, long long c, int i, int k, double wg_prev) {
   const long long N = G.N;
-  const Met M{A.metC, G.P2, q2(i, k, G)};
+  const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
   double u[9], w[9];
   for (int m = 0; m < 9; m++) { u[m] = A.Ustage[(long long)m * N + c]; w[m] = A.W[(long long)m * N + c]; }
   RecovOut ro;
@@ -1812,7 +1811,7 @@ RH_DEV void carry_cell(const Geo& G, const FixArgs& A, long long c, int i, int k
 // Pass -1 takes the chain heads (pend 2 = resolved, 1 = waits for its
 // predecessor); passes 0, 1, ... (last workgroup) take the links.  One loop
 // body, so the recovery is compiled once.
-template <int IW>
+template <int IW, bool MK>
 RH_DEV void b_recov_carry(const Geo& G, const FixArgs& A, int grp, int ngrp) {
   __shared__ int s_progress, s_left, s_last;
   unsigned long long n = A.carry[0];
@@ -1838,7 +1837,7 @@ RH_DEV void b_recov_carry(const Geo& G, const FixArgs& A, int grp, int ngrp) {
         else s_left = 1;
         continue;
       }
-      carry_cell<IW>(G, A, c, i, k, pc >= 0 ? A.wgout[pc] : 0.0);
+      carry_cell<IW, MK>(G, A, c, i, k, pc >= 0 ? A.wgout[pc] : 0.0);
       pend[e] = 2;
       if (!heads) s_progress = 1;
     }
@@ -1913,6 +1912,50 @@ __global__ void __launch_bounds__(256) k_metric_tables(int ni, int nk, int metri
   if (!s) atomicAnd(sym, 0);
 }
 
+// Compact tables (MetK) of the four locations from the general ones, in
+// double and, for the three faces, in float (the derived values formed in
+// float from float-rounded entries, as the mixed form forms them), one
+// thread per (i,k).  *ok is cleared where the metric does not have the
+// structure the compact form assumes (the caller sets it to 1 first).
+template <class R>
+RH_DEV void put_compact(const double* met, long long P2, long long q, R* out, bool centre) {
+  const MetG<R> M(met, P2, q);
+  auto put = [&](int pl, R v) { out[(long long)pl * P2 + q] = v; };
+  put(MK_G00, M.g(0, 0)); put(MK_G01, M.g(0, 1)); put(MK_G02, M.g(0, 2));
+  put(MK_G11, M.g(1, 1)); put(MK_G12, M.g(1, 2)); put(MK_G22, M.g(2, 2)); put(MK_G33, M.g(3, 3));
+  put(MK_DETG, M.detg()); put(MK_ALPHA, M.alpha()); put(MK_RALPHA, M.ralpha()); put(MK_BETA1, M.beta(1));
+  put(MK_GI3_1, M.gi3(1)); put(MK_GI3_2, M.gi3(2)); put(MK_GI3_3, M.gi3(3));
+  if (centre) {
+    put(MK_GI00, M.gi(0, 0)); put(MK_GI01, M.gi(0, 1)); put(MK_GI11, M.gi(1, 1));
+    put(MK_GI12, M.gi(1, 2)); put(MK_GI22, M.gi(2, 2)); put(MK_GI33, M.gi(3, 3));
+  }
+}
+
+__global__ void __launch_bounds__(256) k_compact_metric(CompactArgs A, long long P2, int* ok) {
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= P2) return;
+  bool fine = true;
+  for (int a = 0; a < 4; a++) {
+    const double* met = A.met[a];
+    auto bits = [&](int e) { return __double_as_longlong(met[(long long)e * P2 + q]); };
+    for (int h = 0; h < 2; h++)
+      for (int m = 0; m < 4; m++)
+        for (int n = m + 1; n < 4; n++) {
+          fine = fine && bits(16 * h + m + 4 * n) == bits(16 * h + n + 4 * m);
+          if (n == 3 || (h == 1 && m == 0 && n == 2)) fine = fine && bits(16 * h + m + 4 * n) == 0;
+        }
+    put_compact<double>(met, P2, q, A.mk[a], a == 0);
+    if (a > 0) put_compact<float>(met, P2, q, A.mkf[a - 1], false);
+  }
+  if (!fine) atomicAnd(ok, 0);
+}
+
+hipError_t launch_compact_metric(const CompactArgs& A, long long P2, int* ok, hipStream_t st) {
+  if (P2 <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_compact_metric, dim3((unsigned)((P2 + 255) / 256)), dim3(256), 0, st, A, P2, ok);
+  return hipGetLastError();
+}
+
 hipError_t launch_metric_tables(int ni, int nk, int metric, double akm, const double* x1, const double* x1a,
                                 const double* x3, double ph, const double* tr, double* const met[4], double* chr,
                                 int* sym, hipStream_t st) {
@@ -1924,13 +1967,14 @@ hipError_t launch_metric_tables(int ni, int nk, int metric, double akm, const do
 }
 
 // caluu1 (caluu.f90:2-126) on every cell: conserved variables from primitives.
-__global__ void __launch_bounds__(256) k_caluu1(Geo G, const double* __restrict__ W, const double* __restrict__ metC,
+template <bool MK>
+__global__ void __launch_bounds__(256) k_caluu1(Geo G, const double* __restrict__ W, const void* __restrict__ metC,
                                                 double gam, double* __restrict__ U) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   int i, j, k;
   if (!box_index(t, 1, G.ni, jlo(G, 1), jhi(G, G.nj), 1, G.nk, i, j, k)) return;
   const long long N = G.N, c = cidx(i, j, k, G);
-  const Met M{metC, G.P2, q2(i, k, G)};
+  const MetOf<MK, double> M(metC, G.P2, q2(i, k, G));
   double w[9], u[9];
 #pragma unroll
   for (int n = 0; n < 9; n++) w[n] = W[(long long)n * N + c];
@@ -2013,26 +2057,27 @@ __global__ void __launch_bounds__(256) k_mc_edges(Geo G, EdgeArgs A) { b_mc_edge
 // MP5 and WENO5 are left to the compiler
 template <class R, int IREC>
 constexpr int sweep_waves = (IREC == 5 || IREC == 1) ? (sizeof(R) == 4 ? 5 : 3) : 1;
-template <int D, int IREC, class R, int ICHA>
+template <int D, int IREC, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, IREC>)))
-k_sweep(Geo G, SweepArgs A) { b_sweep<D, IREC, R, ICHA>(G, A, xcd_block()); }
-template <int D, class R, int ICHA>
+k_sweep(Geo G, SweepArgs A) { b_sweep<D, IREC, R, ICHA, MK>(G, A, xcd_block()); }
+template <int D, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
-k_psweep(Geo G, PSweepArgs A) { b_psweep<D, R, ICHA>(G, A, xcd_block()); }
+k_psweep(Geo G, PSweepArgs A) { b_psweep<D, R, ICHA, MK>(G, A, xcd_block()); }
 template <class FT>
 __global__ void __launch_bounds__(256) k_fluxct(Geo G, CtArgs A) { b_fluxct<FT>(G, A, xcd_block()); }
-template <int STAGE, bool SYM, class FT>
-__global__ void __launch_bounds__(256) k_rk(Geo G, StageArgs A) { b_rk<STAGE, SYM, FT>(G, A, xcd_block()); }
-template <int IW>
-__global__ void __launch_bounds__(256) k_recov(Geo G, StageArgs A) { b_recov<IW>(G, A, xcd_block()); }
-template <int IW>
+template <int STAGE, bool SYM, class FT, bool MK>
+__global__ void __launch_bounds__(256) k_rk(Geo G, StageArgs A) { b_rk<STAGE, SYM, FT, MK>(G, A, xcd_block()); }
+template <int IW, bool MK>
+__global__ void __launch_bounds__(256) k_recov(Geo G, StageArgs A) { b_recov<IW, MK>(G, A, xcd_block()); }
+template <int IW, bool MK>
 __global__ void __launch_bounds__(1024) k_recov_carry(Geo G, FixArgs A) {
-  b_recov_carry<IW>(G, A, blockIdx.x, gridDim.x);
+  b_recov_carry<IW, MK>(G, A, blockIdx.x, gridDim.x);
 }
 __global__ void __launch_bounds__(256) k_bnd(Geo G, PostArgs A) { b_bnd(G, A, blockIdx.x); }
-__global__ void __launch_bounds__(256) k_post(Geo G, PostArgs A) { b_post(G, A, xcd_block()); }
-template <int ICHA>
-__global__ void __launch_bounds__(256) k_cfl(Geo G, CflArgs A) { b_cfl<ICHA>(G, A, blockIdx.x); }
+template <bool MK>
+__global__ void __launch_bounds__(256) k_post(Geo G, PostArgs A) { b_post<MK>(G, A, xcd_block()); }
+template <int ICHA, bool MK>
+__global__ void __launch_bounds__(256) k_cfl(Geo G, CflArgs A) { b_cfl<ICHA, MK>(G, A, blockIdx.x); }
 __global__ void __launch_bounds__(1024) k_cfl_finish(CflArgs A) { b_cfl_finish(A); }
 __global__ void __launch_bounds__(64) k_advance_time(AdvArgs A) { b_advance_time(A); }
 
@@ -2053,19 +2098,19 @@ __global__ void __launch_bounds__(256) kb_mc_edges(const BatchItem* __restrict__
   const EdgeArgs A = it[q].A.e;
   b_mc_edges<D, R>(G, A, blk);
 }
-template <int D, int IREC, class R, int ICHA>
+template <int D, int IREC, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, IREC>)))
 kb_sweep(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const SweepArgs A = it[q].A.s;
-  b_sweep<D, IREC, R, ICHA>(G, A, blk);
+  b_sweep<D, IREC, R, ICHA, MK>(G, A, blk);
 }
-template <int D, class R, int ICHA>
+template <int D, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
 kb_psweep(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const PSweepArgs A = it[q].A.ps;
-  b_psweep<D, R, ICHA>(G, A, blk);
+  b_psweep<D, R, ICHA, MK>(G, A, blk);
 }
 template <class FT>
 __global__ void __launch_bounds__(256) kb_fluxct(const BatchItem* __restrict__ it, int n) {
@@ -2073,33 +2118,34 @@ __global__ void __launch_bounds__(256) kb_fluxct(const BatchItem* __restrict__ i
   const CtArgs A = it[q].A.c;
   b_fluxct<FT>(G, A, blk);
 }
-template <int STAGE, bool SYM, class FT>
+template <int STAGE, bool SYM, class FT, bool MK>
 __global__ void __launch_bounds__(256) kb_rk(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const StageArgs A = it[q].A.st;
-  b_rk<STAGE, SYM, FT>(G, A, blk);
+  b_rk<STAGE, SYM, FT, MK>(G, A, blk);
 }
-template <int IW>
+template <int IW, bool MK>
 __global__ void __launch_bounds__(256) kb_recov(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const StageArgs A = it[q].A.st;
-  b_recov<IW>(G, A, blk);
+  b_recov<IW, MK>(G, A, blk);
 }
 __global__ void __launch_bounds__(256) kb_bnd(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const PostArgs A = it[q].A.p;
   b_bnd(G, A, blk);
 }
+template <bool MK>
 __global__ void __launch_bounds__(256) kb_post(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const PostArgs A = it[q].A.p;
-  b_post(G, A, blk);
+  b_post<MK>(G, A, blk);
 }
-template <int ICHA>
+template <int ICHA, bool MK>
 __global__ void __launch_bounds__(256) kb_cfl(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const CflArgs A = it[q].A.cf;
-  b_cfl<ICHA>(G, A, blk);
+  b_cfl<ICHA, MK>(G, A, blk);
 }
 __global__ void __launch_bounds__(256) kb_copy(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
@@ -2109,12 +2155,12 @@ __global__ void __launch_bounds__(256) kb_copy(const BatchItem* __restrict__ it,
 }
 #undef RH_BATCH_PROLOGUE
 // one workgroup per model
-template <int IW>
+template <int IW, bool MK>
 __global__ void __launch_bounds__(1024) kb_recov_carry(const BatchItem* __restrict__ it, int n) {
   if ((int)blockIdx.x >= n) return;
   const Geo G = it[blockIdx.x].G;
   const FixArgs A = it[blockIdx.x].A.fx;
-  b_recov_carry<IW>(G, A, 0, 1);
+  b_recov_carry<IW, MK>(G, A, 0, 1);
 }
 __global__ void __launch_bounds__(1024) kb_cfl_finish(const BatchItem* __restrict__ it, int n) {
   if ((int)blockIdx.x >= n) return;
@@ -2186,27 +2232,68 @@ hipError_t launch_edges(const Geo& G, int dir, int irec, const double* W, const 
 // Sweep kernels are instantiated per (direction, reconstruction, arithmetic
 // type, wave-speed formula); the variant number packs the four so that batch
 // plans group launches of the same kernel:
-//   dir + 4*mixed + 8*irec + 64*icha.
+//   dir + 4*mixed + 8*irec + 64*icha + 256*compact (metric tables).
 template <int V> using IC = std::integral_constant<int, V>;
 template <class T> struct TypeTag { using type = T; };
 
-static int sweep_variant(int dir, bool mixed, int irec, int icha) { return dir + 4 * (int)mixed + 8 * irec + 64 * icha; }
+static int sweep_variant(int dir, bool mixed, int irec, const Geo& G) {
+  return dir + 4 * (int)mixed + 8 * irec + 64 * G.icha + 256 * G.mk;
+}
 
+// f(compact metric tables?)
 template <class F>
-static void with_icha(int icha, F&& f) {
-  if (icha == 2) f(IC<2>{});
-  else if (icha == 1) f(IC<1>{});
-  else f(IC<0>{});
+static void with_mk(bool mk, F&& f) {
+  if (mk) f(std::true_type{});
+  else f(std::false_type{});
+}
+
+// f(wave-speed formula, compact metric tables?)
+template <class F>
+static void with_icha(int icha, bool mk, F&& f) {
+  with_mk(mk, [&](auto K) {
+    if (icha == 2) f(IC<2>{}, K);
+    else if (icha == 1) f(IC<1>{}, K);
+    else f(IC<0>{}, K);
+  });
+}
+
+// f(primitive recovery, compact metric tables?) for a variant iwvec + 4*compact
+template <class F>
+static void with_recov(int variant, F&& f) {
+  with_mk((variant & 4) != 0, [&](auto K) {
+    if ((variant & 3) == 2) f(IC<2>{}, K);
+    else f(IC<1>{}, K);
+  });
+}
+
+// f(stage, symmetric Christoffel tables?, stored flux type, compact metric
+// tables?) for a variant stage + 8*sym + 16*float + 32*compact
+template <class F>
+static void with_rk(int variant, F&& f) {
+  with_mk((variant & 32) != 0, [&](auto K) {
+    with_mk((variant & 8) != 0, [&](auto Y) {
+      auto t = [&](auto S) {
+        if (variant & 16) f(S, Y, TypeTag<float>{}, K);
+        else f(S, Y, TypeTag<double>{}, K);
+      };
+      switch (variant & 7) {
+        case 1: t(IC<1>{}); break;
+        case 2: t(IC<2>{}); break;
+        case 3: t(IC<3>{}); break;
+        default: t(IC<4>{}); break;
+      }
+    });
+  });
 }
 
 template <class F>
 static void with_sweep(int variant, F&& f) {
   const int d = variant & 3, irec = (variant >> 3) & 7;
   const bool mx = (variant & 4) != 0;
-  with_icha(variant >> 6, [&](auto C) {
+  with_icha((variant >> 6) & 3, (variant & 256) != 0, [&](auto C, auto K) {
     auto t = [&](auto D, auto I) {
-      if (mx) f(D, I, TypeTag<float>{}, C);
-      else f(D, I, TypeTag<double>{}, C);
+      if (mx) f(D, I, TypeTag<float>{}, C, K);
+      else f(D, I, TypeTag<double>{}, C, K);
     };
     auto r = [&](auto I) {
       if (d == 1) t(IC<1>{}, I);
@@ -2220,7 +2307,7 @@ static void with_sweep(int variant, F&& f) {
   });
 }
 
-hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const double* metF, const void* E,
+hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
                         double gam, void* F, void* CTsrc, bool mixed, hipStream_t st) {
   const long long n = box(G.nm0, G.ni - G.nm0) * jbox(G, G.nm0, G.nj - G.nm0) * box(G.nm0, G.nk - G.nm0);
   SweepArgs A{W, metF, E, gam, F, CTsrc};
@@ -2229,29 +2316,29 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const 
   if (g_rec) {
     AnyArgs a{};
     a.s = A;
-    record(LK_SWEEP, sweep_variant(dir, mixed, irec, G.icha), bt, nb, G, a);
+    record(LK_SWEEP, sweep_variant(dir, mixed, irec, G), bt, nb, G, a);
     return hipSuccess;
   }
   if (n == 0) return hipSuccess;
-  with_sweep(sweep_variant(dir, mixed, irec, G.icha), [&](auto D, auto I, auto T, auto C) {
-    hipLaunchKernelGGL((k_sweep<D.value, I.value, typename decltype(T)::type, C.value>), dim3(nb), dim3(bt), 0, st,
+  with_sweep(sweep_variant(dir, mixed, irec, G), [&](auto D, auto I, auto T, auto C, auto K) {
+    hipLaunchKernelGGL((k_sweep<D.value, I.value, typename decltype(T)::type, C.value, K.value>), dim3(nb), dim3(bt), 0, st,
                        G, A);
   });
   return hipGetLastError();
 }
 
-// Fused PPM sweeps: variant = dir + 4*mixed + 64*icha (as the sweeps'), dir 0
+// Fused PPM sweeps: variant as the sweeps' without irec, dir 0
 // the j sweep of a collapsed model.
-static int psweep_variant(int dir, bool mixed, int icha) { return dir + 4 * (int)mixed + 64 * icha; }
+static int psweep_variant(int dir, bool mixed, const Geo& G) { return sweep_variant(dir, mixed, 0, G); }
 
 template <class F>
 static void with_psweep(int variant, F&& f) {
   const int d = variant & 3;
   const bool mx = (variant & 4) != 0;
-  with_icha(variant >> 6, [&](auto C) {
+  with_icha((variant >> 6) & 3, (variant & 256) != 0, [&](auto C, auto K) {
     auto t = [&](auto D) {
-      if (mx) f(D, TypeTag<float>{}, C);
-      else f(D, TypeTag<double>{}, C);
+      if (mx) f(D, TypeTag<float>{}, C, K);
+      else f(D, TypeTag<double>{}, C, K);
     };
     if (d == 0) t(IC<0>{});
     else if (d == 1) t(IC<1>{});
@@ -2314,7 +2401,7 @@ int psweep_segment(const Geo& G, int dir) {
 
 size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads * (mixed ? sizeof(float) : sizeof(double)); }
 
-hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* metF, const double* dxs,
+hipError_t launch_psweep(const Geo& G, int dir, const double* W, const void* metF, const double* dxs,
                          const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,
                          hipStream_t st) {
   const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
@@ -2336,7 +2423,7 @@ hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* m
     n = (long long)A.nig * A.ndc * across;
   }
   const unsigned nb = (unsigned)n;
-  const int variant = psweep_variant(self ? 0 : dir, mixed, G.icha);
+  const int variant = psweep_variant(self ? 0 : dir, mixed, G);
   if (g_rec) {
     AnyArgs a{};
     a.ps = A;
@@ -2345,8 +2432,8 @@ hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* m
   }
   if (n == 0) return hipSuccess;
   const size_t lds = self ? 0 : psweep_lds_bytes(bt, mixed);
-  with_psweep(variant, [&](auto D, auto T, auto C) {
-    hipLaunchKernelGGL((k_psweep<D.value, typename decltype(T)::type, C.value>), dim3(nb), dim3(bt), lds, st, G, A);
+  with_psweep(variant, [&](auto D, auto T, auto C, auto K) {
+    hipLaunchKernelGGL((k_psweep<D.value, typename decltype(T)::type, C.value, K.value>), dim3(nb), dim3(bt), lds, st, G, A);
   });
   return hipGetLastError();
 }
@@ -2367,42 +2454,38 @@ hipError_t launch_update(const Geo& G, int stage, const StageArgs& A, hipStream_
   const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
   const int bt = slot_threads(G, TS_RK);
   const unsigned nb = nblk(n, bt);
+  const int variant = stage + 8 * (int)A.chr_sym + 16 * (int)A.f32flux + 32 * G.mk;
   if (g_rec) {
     AnyArgs a{};
     a.st = A;
-    record(LK_RK, stage + 8 * (int)A.chr_sym + 16 * (int)A.f32flux, bt, nb, G, a);
+    record(LK_RK, variant, bt, nb, G, a);
     return hipSuccess;
   }
   if (n == 0) return hipSuccess;
-#define LT(S, Y) \
-  do { if (A.f32flux) hipLaunchKernelGGL((k_rk<S, Y, float>), dim3(nb), dim3(bt), 0, st, G, A); \
-       else hipLaunchKernelGGL((k_rk<S, Y, double>), dim3(nb), dim3(bt), 0, st, G, A); } while (0)
-#define L(S) do { if (A.chr_sym) LT(S, true); else LT(S, false); } while (0)
-  if (stage == 1) L(1);
-  else if (stage == 2) L(2);
-  else if (stage == 3) L(3);
-  else L(4);
-#undef L
-#undef LT
+  with_rk(variant, [&](auto S, auto Y, auto T, auto K) {
+    hipLaunchKernelGGL((k_rk<S.value, Y.value, typename decltype(T)::type, K.value>), dim3(nb), dim3(bt), 0, st, G, A);
+  });
   return hipGetLastError();
 }
 
 hipError_t launch_recov(const Geo& G, const StageArgs& A, hipStream_t st) {
   const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
   const int bt = slot_threads(G, TS_RECOV);
-  if (g_rec) { AnyArgs a{}; a.st = A; record(LK_RECOV, G.iwvec, bt, nblk(n, bt), G, a); return hipSuccess; }
+  if (g_rec) { AnyArgs a{}; a.st = A; record(LK_RECOV, G.iwvec + 4 * G.mk, bt, nblk(n, bt), G, a); return hipSuccess; }
   if (n == 0) return hipSuccess;
-  if (G.iwvec == 2) hipLaunchKernelGGL(k_recov<2>, dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
-  else hipLaunchKernelGGL(k_recov<1>, dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
+  with_recov(G.iwvec + 4 * G.mk, [&](auto I, auto K) {
+    hipLaunchKernelGGL((k_recov<I.value, K.value>), dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
+  });
   return hipGetLastError();
 }
 
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st) {
-  if (g_rec) { AnyArgs a{}; a.fx = A; record(LK_CARRY, G.iwvec, 1024, 1, G, a); return hipSuccess; }
+  if (g_rec) { AnyArgs a{}; a.fx = A; record(LK_CARRY, G.iwvec + 4 * G.mk, 1024, 1, G, a); return hipSuccess; }
   // workgroups sharing the chain heads: one per 1024 flaggable cells, at most 64
   const int ng = (int)std::min<long long>(64, std::max<long long>(1, (A.carry_cap + 1023) / 1024));
-  if (G.iwvec == 2) hipLaunchKernelGGL(k_recov_carry<2>, dim3(ng), dim3(1024), 0, st, G, A);
-  else hipLaunchKernelGGL(k_recov_carry<1>, dim3(ng), dim3(1024), 0, st, G, A);
+  with_recov(G.iwvec + 4 * G.mk, [&](auto I, auto K) {
+    hipLaunchKernelGGL((k_recov_carry<I.value, K.value>), dim3(ng), dim3(1024), 0, st, G, A);
+  });
   return hipGetLastError();
 }
 
@@ -2414,11 +2497,13 @@ hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st) {
     AnyArgs a{};
     a.p = A;
     record(LK_BND, 0, bt, ng > 0 ? nblk(ng, bt) : 0, G, a);
-    record(LK_POST, 0, bt, nblk(G.N, bt), G, a);
+    record(LK_POST, G.mk, bt, nblk(G.N, bt), G, a);
     return hipSuccess;
   }
   if (ng > 0) hipLaunchKernelGGL(k_bnd, dim3(nblk(ng, bt)), dim3(bt), 0, st, G, A);
-  hipLaunchKernelGGL(k_post, dim3(nblk(G.N, bt)), dim3(bt), 0, st, G, A);
+  with_mk(G.mk, [&](auto K) {
+    hipLaunchKernelGGL(k_post<K.value>, dim3(nblk(G.N, bt)), dim3(bt), 0, st, G, A);
+  });
   return hipGetLastError();
 }
 
@@ -2439,11 +2524,13 @@ hipError_t launch_cfl(const Geo& G, const CflArgs& A0, hipStream_t st) {
   if (g_rec) {
     AnyArgs a{};
     a.cf = A;
-    record(LK_CFL, G.icha, 256, nb, G, a);
+    record(LK_CFL, G.icha + 4 * G.mk, 256, nb, G, a);
     record(LK_CFL_FINISH, 0, 1024, 1, G, a);
     return hipSuccess;
   }
-  with_icha(G.icha, [&](auto C) { hipLaunchKernelGGL((k_cfl<C.value>), dim3(nb), dim3(256), 0, st, G, A); });
+  with_icha(G.icha, G.mk, [&](auto C, auto K) {
+    hipLaunchKernelGGL((k_cfl<C.value, K.value>), dim3(nb), dim3(256), 0, st, G, A);
+  });
   hipLaunchKernelGGL(k_cfl_finish, dim3(1), dim3(1024), 0, st, A);
   return hipGetLastError();
 }
@@ -2485,14 +2572,14 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       break;
     }
     case LK_SWEEP:
-      with_sweep(variant, [&](auto D, auto I, auto T, auto C) {
-        hipLaunchKernelGGL((kb_sweep<D.value, I.value, typename decltype(T)::type, C.value>), g, b, 0, st, it, n);
+      with_sweep(variant, [&](auto D, auto I, auto T, auto C, auto K) {
+        hipLaunchKernelGGL((kb_sweep<D.value, I.value, typename decltype(T)::type, C.value, K.value>), g, b, 0, st, it, n);
       });
       break;
     case LK_PSWEEP: {
       const size_t lds = (variant & 3) ? psweep_lds_bytes(threads, (variant & 4) != 0) : 0;
-      with_psweep(variant, [&](auto D, auto T, auto C) {
-        hipLaunchKernelGGL((kb_psweep<D.value, typename decltype(T)::type, C.value>), g, b, lds, st, it, n);
+      with_psweep(variant, [&](auto D, auto T, auto C, auto K) {
+        hipLaunchKernelGGL((kb_psweep<D.value, typename decltype(T)::type, C.value, K.value>), g, b, lds, st, it, n);
       });
       break;
     }
@@ -2500,34 +2587,28 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       if (variant == 1) hipLaunchKernelGGL(kb_fluxct<float>, g, b, 0, st, it, n);
       else hipLaunchKernelGGL(kb_fluxct<double>, g, b, 0, st, it, n);
       break;
-    case LK_RK: {
-      const int stg = variant & 7;
-      const bool sym = (variant & 8) != 0, f32 = (variant & 16) != 0;
-#define LT(S, Y) \
-  do { if (f32) hipLaunchKernelGGL((kb_rk<S, Y, float>), g, b, 0, st, it, n); \
-       else hipLaunchKernelGGL((kb_rk<S, Y, double>), g, b, 0, st, it, n); } while (0)
-#define L(S) do { if (sym) LT(S, true); else LT(S, false); } while (0)
-      if (stg == 1) L(1);
-      else if (stg == 2) L(2);
-      else if (stg == 3) L(3);
-      else L(4);
-#undef L
-#undef LT
+    case LK_RK:
+      with_rk(variant, [&](auto S, auto Y, auto T, auto K) {
+        hipLaunchKernelGGL((kb_rk<S.value, Y.value, typename decltype(T)::type, K.value>), g, b, 0, st, it, n);
+      });
       break;
-    }
     case LK_RECOV:
-      if (variant == 2) hipLaunchKernelGGL(kb_recov<2>, g, b, 0, st, it, n);
-      else hipLaunchKernelGGL(kb_recov<1>, g, b, 0, st, it, n);
+      with_recov(variant, [&](auto I, auto K) { hipLaunchKernelGGL((kb_recov<I.value, K.value>), g, b, 0, st, it, n); });
       break;
     case LK_BND: hipLaunchKernelGGL(kb_bnd, g, b, 0, st, it, n); break;
-    case LK_POST: hipLaunchKernelGGL(kb_post, g, b, 0, st, it, n); break;
+    case LK_POST:
+      with_mk(variant != 0, [&](auto K) { hipLaunchKernelGGL(kb_post<K.value>, g, b, 0, st, it, n); });
+      break;
     case LK_CFL:
-      with_icha(variant, [&](auto C) { hipLaunchKernelGGL((kb_cfl<C.value>), g, b, 0, st, it, n); });
+      with_icha(variant & 3, (variant & 4) != 0, [&](auto C, auto K) {
+        hipLaunchKernelGGL((kb_cfl<C.value, K.value>), g, b, 0, st, it, n);
+      });
       break;
     case LK_COPY: hipLaunchKernelGGL(kb_copy, g, b, 0, st, it, n); break;
     case LK_CARRY:
-      if (variant == 2) hipLaunchKernelGGL(kb_recov_carry<2>, dim3(n), dim3(1024), 0, st, it, n);
-      else hipLaunchKernelGGL(kb_recov_carry<1>, dim3(n), dim3(1024), 0, st, it, n);
+      with_recov(variant, [&](auto I, auto K) {
+        hipLaunchKernelGGL((kb_recov_carry<I.value, K.value>), dim3(n), dim3(1024), 0, st, it, n);
+      });
       break;
     case LK_CFL_FINISH: hipLaunchKernelGGL(kb_cfl_finish, dim3(n), dim3(1024), 0, st, it, n); break;
     case LK_ADVANCE: hipLaunchKernelGGL(kb_advance_time, dim3(n), dim3(64), 0, st, it, n); break;
@@ -2547,8 +2628,9 @@ hipError_t launch_gather_first(const double* const* src, double* dst, int n, hip
   return hipGetLastError();
 }
 
-hipError_t launch_caluu1(const Geo& G, const double* W, const double* metC, double gam, double* U, hipStream_t st) {
-  hipLaunchKernelGGL(k_caluu1, dim3(nblk(G.N, 256)), dim3(256), 0, st, G, W, metC, gam, U);
+hipError_t launch_caluu1(const Geo& G, const double* W, const void* metC, double gam, double* U, hipStream_t st) {
+  if (G.mk) hipLaunchKernelGGL(k_caluu1<true>, dim3(nblk(G.N, 256)), dim3(256), 0, st, G, W, metC, gam, U);
+  else hipLaunchKernelGGL(k_caluu1<false>, dim3(nblk(G.N, 256)), dim3(256), 0, st, G, W, metC, gam, U);
   return hipGetLastError();
 }
 

@@ -10,7 +10,8 @@ struct StageArgs {
   const double *W;                 // primitives at stage start (9 planes)
   const double *Ua, *Ub;           // RK inputs: stage1 uu; stage2 uo,uh; stage3 uo,us
   const void *F1, *F2, *F3;        // ww(1..3,:,...) after ct (9 planes each; float when f32flux)
-  const double *metC, *chr;        // centre metric tables, Christoffel tables
+  const void *metC;                // centre metric tables (compact when Geo::mk)
+  const double *chr;               // Christoffel tables
   const double *dx1b, *dx2b, *dx3b;
   const double *r15, *r25;         // x1(i)**(-3/2), x1(i)**(-5/2) from the host libm
   const unsigned long long *dtbits;
@@ -36,7 +37,8 @@ struct StageArgs {
 struct PostArgs {
   const double *Wpre, *Wold, *Wo;
   double *Wghost;                  // = Wpre: k_bnd writes its ghost slots
-  const double *metC, *r15, *r25;
+  const void *metC;
+  const double *r15, *r25;
   const int *bc;                   // boundary codes [axis*2+side][9]
   double *Wout, *Uout;
   unsigned long long *cnt, *cpart;
@@ -45,7 +47,9 @@ struct PostArgs {
 };
 
 struct CflArgs {
-  const double *W, *metC, *dx1b, *dx2b, *dx3b;
+  const double *W;
+  const void *metC;
+  const double *dx1b, *dx2b, *dx3b;
   unsigned long long *dtbits;      // [0] dtcfl [1..3] dt1..dt3 (bit patterns of the doubles)
   long long *blast;                // per block and accumulator: position of the last NaN
   double *bmin;                    // per block and accumulator: minimum after it
@@ -54,7 +58,9 @@ struct CflArgs {
 };
 
 struct FixArgs {
-  const double *W, *Ustage, *metC, *r15, *r25;
+  const double *W, *Ustage;
+  const void *metC;
+  const double *r15, *r25;
   double *Wpre, *wgout;
   unsigned long long *carry, *cnt;
   unsigned char *cflag, *pend;
@@ -70,14 +76,17 @@ struct EdgeArgs {
 };
 
 struct SweepArgs {
-  const double *W, *metF;
+  const double *W;
+  const void *metF;                // face metric tables: doubles, or (compact and mixed) floats
   const void *E;
   double gam;
   void *F, *CTsrc;  // element type: the sweep's arithmetic type (double, or float when mixed)
 };
 
 struct PSweepArgs {
-  const double *W, *metF, *dxs, *xs, *pc;  // pc: PPM width coefficients of the direction
+  const double *W;
+  const void *metF;
+  const double *dxs, *xs, *pc;  // pc: PPM width coefficients of the direction
   double gam;
   void *F, *CTsrc;  // element type: the sweep's arithmetic type
   // tile: tp cells along the sweep's axis per workgroup, 2^sh lanes in the
@@ -171,7 +180,7 @@ hipError_t launch_edges(const Geo& G, int dir, int irec, const double* W, const 
 // Fluxes at the interfaces along dir; E = the PPM edges (irec 5), unused otherwise.
 // F and CTsrc take doubles, or floats when mixed (every value the float
 // arithmetic produced, so storing it in float loses nothing).
-hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const double* metF, const void* E,
+hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
                         double gam, void* F, void* CTsrc, bool mixed, hipStream_t st);
 // PPM (irec 5) sweep along dir with the face values computed in the same
 // kernel (through LDS): reads W and the direction's PPM width coefficients
@@ -180,7 +189,7 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const 
 // i per wave; a workgroup's waves are stacked along the axis), a power of two
 // from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
-hipError_t launch_psweep(const Geo& G, int dir, const double* W, const double* metF, const double* dxs,
+hipError_t launch_psweep(const Geo& G, int dir, const double* W, const void* metF, const double* dxs,
                          const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,
                          hipStream_t st);
 int psweep_segment(const Geo& G, int dir);
@@ -208,8 +217,17 @@ hipError_t launch_advance_time(const Geo& G, const unsigned long long* dtbits, d
 hipError_t launch_metric_tables(int ni, int nk, int metric, double akm, const double* x1, const double* x1a,
                                 const double* x3, double ph, const double* tr, double* const met[4], double* chr,
                                 int* sym, hipStream_t st);
+// The compact metric tables of the four locations (centre: MK_PLANES planes,
+// faces: MK_FACE_PLANES) and the faces' float ones from the general tables;
+// *ok is cleared where the metric has not the structure they assume.
+struct CompactArgs {
+  const double* met[4];
+  double* mk[4];
+  float* mkf[3];
+};
+hipError_t launch_compact_metric(const CompactArgs& A, long long P2, int* ok, hipStream_t st);
 hipError_t launch_copy(const Geo& G, double* dst, const double* src, long long n, hipStream_t st);
-hipError_t launch_caluu1(const Geo& G, const double* W, const double* metC, double gam, double* U, hipStream_t st);
+hipError_t launch_caluu1(const Geo& G, const double* W, const void* metC, double gam, double* U, hipStream_t st);
 hipError_t launch_aos_to_soa(const double* aos, double* soa, long long N, hipStream_t st);
 hipError_t launch_soa_to_aos(const double* soa, double* aos, long long N, hipStream_t st);
 hipError_t launch_ww_to_planes(const double* ww, double* F, long long N, hipStream_t st);

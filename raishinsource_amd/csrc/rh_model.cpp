@@ -76,18 +76,17 @@ bool check_pram(const raishin_pram& p) {
 
 void dfree_all(raishin_model* m) {
   double** bufs[] = {&m->W, &m->Wb, &m->Wpre, &m->Wo, &m->Ucur, &m->Uh, &m->Us, &m->Unext, &m->F, &m->CT, &m->E,
-                     &m->wgout, &m->stage_aos, &m->chr, &m->r15, &m->r25, &m->tdt};
+                     &m->wgout, &m->stage_aos, &m->chr, &m->grid, &m->mkall, &m->tdt};
   for (auto b : bufs) if (*b) { (void)hipFree(*b); *b = nullptr; }
-  for (int a = 0; a < 4; a++) if (m->met[a]) { (void)hipFree(m->met[a]); m->met[a] = nullptr; }
-  for (int a = 0; a < 3; a++) {
-    if (m->ppmc[a]) (void)hipFree(m->ppmc[a]);
-    m->ppmc[a] = nullptr;
-    if (m->xs[a]) (void)hipFree(m->xs[a]);
-    if (m->dxb[a]) (void)hipFree(m->dxb[a]);
-    if (m->dxs[a]) (void)hipFree(m->dxs[a]);
-    if (m->xa[a]) (void)hipFree(m->xa[a]);
-    m->xs[a] = m->dxb[a] = m->dxs[a] = m->xa[a] = nullptr;
+  for (int a = 0; a < 4; a++) {
+    if (m->met[a]) { (void)hipFree(m->met[a]); m->met[a] = nullptr; }
+    m->mk[a] = nullptr;  // parts of mkall
   }
+  for (int a = 0; a < 3; a++) {
+    m->mkf[a] = nullptr;
+    m->ppmc[a] = m->xs[a] = m->dxb[a] = m->dxs[a] = m->xa[a] = nullptr;  // parts of grid
+  }
+  m->r15 = m->r25 = nullptr;
   if (m->bc) (void)hipFree(m->bc);
   if (m->dtbits) (void)hipFree(m->dtbits);
   if (m->cnt) (void)hipFree(m->cnt);
@@ -252,8 +251,7 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
     }
   if (!dalloc(&m->W, 9 * N) || !dalloc(&m->Wb, 9 * N) || !dalloc(&m->Wpre, 9 * N) || !dalloc(&m->Ucur, 9 * N) ||
       !dalloc(&m->Uh, 9 * N) || !dalloc(&m->Us, 9 * N) || !dalloc(&m->Unext, 9 * N) || !dalloc(&m->F, 27 * N) ||
-      !dalloc(&m->CT, 6 * N) || !dalloc(&m->wgout, N) || !dalloc(&m->chr, 64 * G.P2) || !dalloc(&m->r15, G.ni) ||
-      !dalloc(&m->r25, G.ni) || !dalloc(&m->bc, 54) || !dalloc(&m->dtbits, 4) || !dalloc(&m->cnt, NCOUNT) ||
+      !dalloc(&m->CT, 6 * N) || !dalloc(&m->wgout, N) || !dalloc(&m->chr, 64 * G.P2) || !dalloc(&m->bc, 54) || !dalloc(&m->dtbits, 4) || !dalloc(&m->cnt, NCOUNT) ||
       !dalloc(&m->carry, 2 + m->carry_cap) || !dalloc(&m->tdt, 2) || !dalloc(&m->cflag, N) ||
       !dalloc(&m->pend, m->carry_cap) || !dalloc(&m->cfl_last, 4 * cfl_blocks(G)) ||
       !dalloc(&m->cfl_min, 4 * cfl_blocks(G)))
@@ -275,6 +273,8 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
   HIPCHK(hipMemsetAsync(m->Wpre, 0, 9 * N * 8, m->st));
   HIPCHK(hipMemsetAsync(m->cflag, 0, N, m->st));
   // metric tables
+  int flags[2] = {1, 1};  // Christoffel tables symmetric, metric of the compact structure
+  int* flags_d = nullptr;
   if (!gcv) {
     // from the grid on the device (k_metric_tables); its inputs are staged in
     // wgout, which the recovery does not use before the first step
@@ -289,19 +289,20 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
     if (need > N) { set_error("grid too small to stage the metric inputs"); return false; }
     std::vector<double> tr(8 * (size_t)G.nk);
     theta_trig_table(*p, x3, x3a, tr.data());
+    // one upload: x1, x1a, x3, the trigonometric table, then the flags
+    // (Christoffel symmetry, compact structure), both set to start with
+    std::vector<double> in(x1, x1 + G.ni);
+    in.insert(in.end(), x1a, x1a + G.ni);
+    in.insert(in.end(), x3, x3 + G.nk);
+    in.insert(in.end(), tr.begin(), tr.end());
+    in.push_back(0.0);
+    std::memcpy(&in.back(), flags, sizeof flags);
     double* sc = m->wgout;
-    int* sym = reinterpret_cast<int*>(sc + 2LL * G.ni + 9LL * G.nk);
-    const int one = 1;
-    if (!h2d_sync(sc, x1, G.ni * 8, m->st) || !h2d_sync(sc + G.ni, x1a, G.ni * 8, m->st) ||
-        !h2d_sync(sc + 2LL * G.ni, x3, G.nk * 8, m->st) || !h2d_sync(sc + 2LL * G.ni + G.nk, tr.data(), tr.size() * 8, m->st) ||
-        !h2d_sync(sym, &one, 4, m->st))
-      return false;
+    flags_d = reinterpret_cast<int*>(sc + in.size() - 1);
+    HIPCHK(hipMemcpyAsync(sc, in.data(), in.size() * 8, hipMemcpyHostToDevice, m->st));
     HIPCHK(launch_metric_tables(G.ni, G.nk, p->metric, p->akm, sc, sc + G.ni, sc + 2LL * G.ni, x2[0],
-                                sc + 2LL * G.ni + G.nk, m->met, m->chr, sym, m->st));
-    int symh = 0;
-    HIPCHK(hipMemcpyAsync(&symh, sym, 4, hipMemcpyDeviceToHost, m->st));
-    HIPCHK(hipStreamSynchronize(m->st));
-    m->chr_sym = symh != 0;
+                                sc + 2LL * G.ni + G.nk, m->met, m->chr, flags_d, m->st));
+    HIPCHK(hipStreamSynchronize(m->st));  // the upload's source goes out of scope
   } else {
   const char* names[4] = {"centre", "i-face", "j-face", "k-face"};
   std::vector<double> tab;
@@ -332,20 +333,45 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
           m->chr_sym = std::memcmp(&ct[(size_t)(l + 4 * a + 16 * b) * G.P2], &ct[(size_t)(l + 4 * b + 16 * a) * G.P2],
                                    (size_t)G.P2 * 8) == 0;
   }
+  flags[0] = m->chr_sym;
+  flags_d = reinterpret_cast<int*>(m->wgout);
+  HIPCHK(hipMemcpyAsync(flags_d, flags, sizeof flags, hipMemcpyHostToDevice, m->st));
   }
-  // 1D grids; dxs[d] = rec2's dummy dx*b(d) = actual dx*b(d-1) (rec.f90:58), clamped at the ends
+  // the compact tables, where the metric has their structure (the flags are
+  // staged in wgout, which the recovery does not use before the first step)
+  {
+    if (!dalloc(&m->mkall, (MK_PLANES + 3 * MK_FACE_PLANES + 3 * MK_FACE_PLANES / 2) * G.P2)) return false;
+    CompactArgs C{};
+    double* at = m->mkall;
+    for (int a = 0; a < 4; a++) {
+      C.met[a] = m->met[a];
+      C.mk[a] = m->mk[a] = at;
+      at += (a == 0 ? MK_PLANES : MK_FACE_PLANES) * G.P2;
+    }
+    for (int a = 0; a < 3; a++, at += MK_FACE_PLANES / 2 * G.P2) C.mkf[a] = m->mkf[a] = reinterpret_cast<float*>(at);
+    HIPCHK(launch_compact_metric(C, G.P2, flags_d + 1, m->st));
+    HIPCHK(hipMemcpyAsync(flags, flags_d, sizeof flags, hipMemcpyDeviceToHost, m->st));
+    HIPCHK(hipStreamSynchronize(m->st));
+    m->chr_sym = flags[0] != 0;
+    G.mk = flags[1] != 0;
+  }
+  // 1D grids; dxs[d] = rec2's dummy dx*b(d) = actual dx*b(d-1) (rec.f90:58),
+  // clamped at the ends.  Collected here and uploaded in one copy.
+  std::vector<double> one;
+  std::vector<std::pair<double**, size_t>> parts;
+  auto part = [&](double** where, const std::vector<double>& v) {
+    parts.emplace_back(where, one.size());
+    one.insert(one.end(), v.begin(), v.end());
+  };
   const double* xsrc[3] = {x1, x2, x3};
   const double* dsrc[3] = {dx1b, dx2b, dx3b};
   const int nn[3] = {G.ni, G.nj, G.nk};
   for (int a = 0; a < 3; a++) {
     const int n = nn[a];
-    if (!dalloc(&m->xs[a], n) || !dalloc(&m->dxb[a], n) || !dalloc(&m->dxs[a], n + 2) || !dalloc(&m->xa[a], n))
-      return false;
     // x*a(i) = (x*(i) + x*(i+1))/2 as grid.f90 builds it (the last entry is never read)
     std::vector<double> fa(n, 0.0);
     for (int q = 0; q + 1 < n; q++) fa[q] = 0.5 * (xsrc[a][q] + xsrc[a][q + 1]);
     if (n > 1) fa[n - 1] = fa[n - 2] + (xsrc[a][n - 1] - xsrc[a][n - 2]);
-    if (!h2d_sync(m->xa[a], fa.data(), n * 8, m->st)) return false;
     std::vector<double> db(n, 0.0), ds(n + 2, 0.0);
     for (int q = 0; q < n - 1; q++) db[q] = dsrc[a][q];
     for (int d = 0; d <= n + 1; d++) {
@@ -354,20 +380,20 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
       if (q > n - 1) q = n - 1;
       ds[d] = (n > 1) ? dsrc[a][q - 1] : 0.0;
     }
-    if (!h2d_sync(m->xs[a], xsrc[a], n * 8, m->st)) return false;
-    if (!h2d_sync(m->dxb[a], db.data(), n * 8, m->st)) return false;
-    if (!h2d_sync(m->dxs[a], ds.data(), (n + 2) * 8, m->st)) return false;
-    if (p->irec == 5) {
-      const std::vector<double> pc = ppm_coefficients(ds);
-      if (!dalloc(&m->ppmc[a], pc.size())) return false;
-      if (!h2d_sync(m->ppmc[a], pc.data(), pc.size() * 8, m->st)) return false;
-    }
+    part(&m->xs[a], std::vector<double>(xsrc[a], xsrc[a] + n));
+    part(&m->dxb[a], db);
+    part(&m->dxs[a], ds);
+    part(&m->xa[a], fa);
+    if (p->irec == 5) part(&m->ppmc[a], ppm_coefficients(ds));
   }
   // r-power tables from the host libm, as the reference computes them (correction.f90:318-319)
   std::vector<double> r15(G.ni), r25(G.ni);
   for (int i = 0; i < G.ni; i++) { r15[i] = std::pow(x1[i], -1.5); r25[i] = std::pow(x1[i], -2.5); }
-  if (!h2d_sync(m->r15, r15.data(), G.ni * 8, m->st)) return false;
-  if (!h2d_sync(m->r25, r25.data(), G.ni * 8, m->st)) return false;
+  part(&m->r15, r15);
+  part(&m->r25, r25);
+  if (!dalloc(&m->grid, one.size())) return false;
+  for (const auto& q : parts) *q.first = m->grid + q.second;
+  HIPCHK(hipMemcpyAsync(m->grid, one.data(), one.size() * 8, hipMemcpyHostToDevice, m->st));
   int bch[54];
   const int* bsrc[6] = {p->iboux1in, p->iboux1ot, p->iboux2in, p->iboux2ot, p->iboux3in, p->iboux3ot};
   for (int a = 0; a < 6; a++) for (int q = 0; q < 9; q++) bch[a * 9 + q] = bsrc[a][q];
@@ -466,7 +492,7 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F) {
   for (int d = 1; d <= 3; d++) {
     if (irec == 5 && !G.ppm_split) {
       TimedLaunch t(m, K_SWEEP1 + d - 1);
-      HIPCHK(launch_psweep(G, d, W, m->met[d], m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam,
+      HIPCHK(launch_psweep(G, d, W, m->metric_face(d), m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam,
                            flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed, m->st));
       continue;
     }
@@ -476,7 +502,7 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F) {
       HIPCHK(launch_edges(G, d, irec, W, m->dxs[d - 1], m->xs[d - 1], tab, m->p.gam, m->E, m->mixed, m->st));
     }
     TimedLaunch t(m, K_SWEEP1 + d - 1);
-    HIPCHK(launch_sweep(G, d, irec, W, m->met[d], m->E, m->p.gam, flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed,
+    HIPCHK(launch_sweep(G, d, irec, W, m->metric_face(d), m->E, m->p.gam, flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed,
                         m->st));
   }
   return true;
@@ -505,7 +531,7 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
   A.F3 = flux_plane(m, const_cast<double*>(F), 18);
   A.f32flux = m->mixed;
   A.CTd = ct_fp64(m, const_cast<double*>(F));
-  A.metC = m->met[0]; A.chr = m->chr; A.dx1b = m->dxb[0]; A.dx2b = m->dxb[1]; A.dx3b = m->dxb[2];
+  A.metC = m->metric_centre(); A.chr = m->chr; A.dx1b = m->dxb[0]; A.dx2b = m->dxb[1]; A.dx3b = m->dxb[2];
   A.r15 = m->r15; A.r25 = m->r25; A.dtbits = m->dtbits; A.Wpre = m->Wpre; A.wgout = m->wgout; A.Ukeep = Uout;
   A.cnt = m->cnt; A.cpart = m->cpart; A.carry = m->carry; A.cflag = m->cflag; A.carry_cap = m->carry_cap;
   A.gam = m->p.gam; A.cfl = m->p.cfl; A.dmin = m->p.dmin; A.pmin = m->p.pmin; A.iter = m->p.iter;
@@ -514,7 +540,7 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
   { TimedLaunch t(m, K_UPDATE); HIPCHK(launch_update(G, rkstage, A, m->st)); }
   { TimedLaunch t(m, K_RECOV); HIPCHK(launch_recov(G, A, m->st)); }
   FixArgs X{};
-  X.W = W; X.Ustage = Uout; X.metC = m->met[0]; X.r15 = m->r15; X.r25 = m->r25; X.Wpre = m->Wpre;
+  X.W = W; X.Ustage = Uout; X.metC = m->metric_centre(); X.r15 = m->r15; X.r25 = m->r25; X.Wpre = m->Wpre;
   X.wgout = m->wgout; X.carry = m->carry; X.cnt = m->cnt; X.cflag = m->cflag; X.pend = m->pend;
   X.carry_cap = m->carry_cap; X.gam = m->p.gam;
   X.dmin = m->p.dmin; X.pmin = m->p.pmin; X.iter = m->p.iter;
@@ -524,7 +550,7 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
 
 bool stage_post(raishin_model* m, const double* Wold, const double* Wo, double* Wout, double* Uout) {
   PostArgs P{};
-  P.Wpre = m->Wpre; P.Wghost = m->Wpre; P.Wold = Wold; P.Wo = Wo; P.metC = m->met[0]; P.r15 = m->r15;
+  P.Wpre = m->Wpre; P.Wghost = m->Wpre; P.Wold = Wold; P.Wo = Wo; P.metC = m->metric_centre(); P.r15 = m->r15;
   P.r25 = m->r25; P.bc = m->bc; P.Wout = Wout; P.Uout = Uout; P.cnt = m->cnt; P.cpart = m->cpart; P.gam = m->p.gam;
   P.dmin = m->p.dmin; P.pmin = m->p.pmin; P.pmax = m->p.pmax; P.model = m->p.model;
   { TimedLaunch t(m, K_POST); HIPCHK(launch_post(m->G, P, m->st)); }
@@ -556,7 +582,7 @@ bool copy_fluxes_out(raishin_model* m, double* ww, double* ct) {
 
 bool run_cfl(raishin_model* m, const double* W) {
   CflArgs C{};
-  C.W = W; C.metC = m->met[0]; C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
+  C.W = W; C.metC = m->metric_centre(); C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
   C.dtbits = m->dtbits; C.blast = m->cfl_last; C.bmin = m->cfl_min; C.gam = m->p.gam;
   { TimedLaunch t(m, K_CFL); HIPCHK(launch_cfl(m->G, C, m->st)); }
   return true;

@@ -45,10 +45,21 @@ struct raishin_model {
   double* ppmc[3] = {nullptr, nullptr, nullptr};  // PPM width coefficients per direction (irec = 5)
   // geometry
   double *met[4] = {nullptr, nullptr, nullptr, nullptr};  // centre, i-face, j-face, k-face
+  // the same in the compact form, where the metric allows it (Geo::mk), in
+  // double and for the faces in float (the mixed form's sweeps)
+  double *mk[4] = {nullptr, nullptr, nullptr, nullptr};
+  float *mkf[3] = {nullptr, nullptr, nullptr};
+  double* mkall = nullptr;  // the allocation mk and mkf are parts of
+  // the tables the kernels read: centre, and face d = 1..3
+  const void* metric_centre() const { return G.mk ? mk[0] : met[0]; }
+  const void* metric_face(int d) const {
+    return !G.mk ? (const void*)met[d] : mixed ? (const void*)mkf[d - 1] : (const void*)mk[d];
+  }
   double *chr = nullptr;
   double *xs[3] = {nullptr, nullptr, nullptr}, *dxb[3] = {nullptr, nullptr, nullptr}, *dxs[3] = {nullptr, nullptr, nullptr};
   double* xa[3] = {nullptr, nullptr, nullptr};  // cell-face positions x*a (MC reconstruction)
   double *r15 = nullptr, *r25 = nullptr;
+  double* grid = nullptr;  // the allocation ppmc, xs, dxb, dxs, xa, r15, r25 are parts of
   int* bc = nullptr;
   unsigned long long *dtbits = nullptr, *cnt = nullptr, *carry = nullptr;
   unsigned long long* cpart = nullptr;  // per-wavefront event rows, folded into cnt on read

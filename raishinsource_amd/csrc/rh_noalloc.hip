@@ -62,7 +62,7 @@ extern "C" int raishin_model_cdtcfl4_noalloc(raishin_model* m, double* out) {
   // every workgroup writes its partials before the finishing workgroup
   // reads them, so nothing needs clearing between calls
   CflArgs C{};
-  C.W = m->W; C.metC = m->met[0]; C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
+  C.W = m->W; C.metC = m->metric_centre(); C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
   C.dtbits = reinterpret_cast<unsigned long long*>(out);
   C.blast = reinterpret_cast<long long*>(base);
   C.bmin = reinterpret_cast<double*>(base + (size_t)NOALLOC_CFL_BLOCKS * 4 * sizeof(long long));

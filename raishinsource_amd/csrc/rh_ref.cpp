@@ -549,7 +549,7 @@ void raishin_caluu1(double* uri, double* uu, const double* gcov, const double* g
     const double* W = input(uri, MK_STATE);
     double* U = output(uu, MK_STATE);
     if (!W || !U) return;
-    if (launch_caluu1(m->G, W, m->met[0], g.p.gam, U, m->st) != hipSuccess) set_error("caluu1: launch failed");
+    if (launch_caluu1(m->G, W, m->metric_centre(), g.p.gam, U, m->st) != hipSuccess) set_error("caluu1: launch failed");
     return;
   }
   const bool want_inf = g.p.model >= 7 && g.p.model <= 20, want_atm = g.p.model >= 7 && g.p.model <= 15;

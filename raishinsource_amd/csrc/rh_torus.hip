@@ -305,7 +305,7 @@ extern "C" int raishin_model_set_torus(raishin_model* m, const raishin_torus* t)
     HIPCHK(hipGetLastError());
     // the rest as a set_state with uu computed: conserved variables (main.f90:530),
     // time 0, ww from zero (main.f90:374-376)
-    HIPCHK(rh::launch_caluu1(G, m->W, m->met[0], m->p.gam, m->Ucur, m->st));
+    HIPCHK(rh::launch_caluu1(G, m->W, m->metric_centre(), m->p.gam, m->Ucur, m->st));
     const double tdt[2] = {0.0, 0.0};
     HIPCHK(hipMemcpyAsync(m->tdt, tdt, 16, hipMemcpyHostToDevice, m->st));
     HIPCHK(hipMemsetAsync(m->F, 0, (size_t)27 * N * 8, m->st));

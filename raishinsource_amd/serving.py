@@ -89,6 +89,7 @@ def footprint(p):
     b += 2 * 8 * 4 * ncfl                            # CFL per-block results
     b += 8 * 11 * ((n + 255) // 256) * 4             # per-wavefront counter rows
     b += 4 * 8 * 33 * p2                             # metric tables
+    b += 8 * (20 + 3 * 14) * p2 + 4 * 3 * 14 * p2    # compact metric tables, and the faces' in float
     b += sum(8 * (4 * d + 2) for d in (ni, nj, nk))  # xs, dxb, dxs, xa
     if p.irec == 5:
         b += sum(8 * 7 * (d + 2) for d in (ni, nj, nk))

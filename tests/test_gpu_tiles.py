@@ -114,7 +114,7 @@ def test_autotuner_picks_tiles():
 
 
 @pytest.mark.parametrize("threads", [64, 128, 192, 256])
-@pytest.mark.parametrize("ni,nj,nk,seg,mixed", [(17, 11, 12, 0, False), (72, 13, 30, 0, True), (75, 16, 71, 8, False)])
+@pytest.mark.parametrize("ni,nj,nk,seg,mixed", [(17, 11, 15, 0, False), (72, 13, 30, 0, True), (75, 16, 71, 8, False)])
 def test_workgroup_tiles_equal_split(threads, ni, nj, nk, seg, mixed):
     """The sweeps' workgroup tiles (rows of a workgroup or of 16, 32, 64
     lanes along i; stacked waves along j and k) at extents one below, at and
