@@ -36,6 +36,18 @@ RH_DEV float fsign1(float x) { return copysignf(1.0f, x); }
 RH_DEV double mad_(double x, double y, double z) { return x * y + z; }
 RH_DEV float mad_(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
 
+// Element of a plane (an address the whole wave shares) at a lane's 32-bit
+// byte offset, so that the lane keeps one offset for all planes.  A plane is
+// below 4 GiB: 2^29 cells would need more than 400 GB of state.
+template <class T>
+RH_DEV T ld_(const T* plane, unsigned byte) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(plane) + byte);
+}
+template <class T>
+RH_DEV void st_(T* plane, unsigned byte, T v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(plane) + byte) = v;
+}
+
 // Geometry of one model on the device.
 struct Geo {
   int ni, nj, nk;        // imax, jmax, kmax (ghosts included)
@@ -76,11 +88,12 @@ struct Geo {
 template <class R>
 struct MetG {
   const double* __restrict__ b;
-  long long P2, q;
-  RH_DEV MetG(const void* tab, long long P2_, long long q_) : b((const double*)tab), P2(P2_), q(q_) {}
-  RH_DEV R g(int m, int n) const { return R(b[(long long)(m + 4 * n) * P2 + q]); }
-  RH_DEV R gi(int m, int n) const { return R(b[(long long)(16 + m + 4 * n) * P2 + q]); }
-  RH_DEV R detg() const { return R(b[32LL * P2 + q]); }
+  long long P2;
+  unsigned q;
+  RH_DEV MetG(const void* tab, long long P2_, unsigned q_) : b((const double*)tab), P2(P2_), q(q_ * 8u) {}
+  RH_DEV R g(int m, int n) const { return R(ld_(b + (long long)(m + 4 * n) * P2, q)); }
+  RH_DEV R gi(int m, int n) const { return R(ld_(b + (long long)(16 + m + 4 * n) * P2, q)); }
+  RH_DEV R detg() const { return R(ld_(b + 32LL * P2, q)); }
   RH_DEV R alpha() const { return R(1) / sqrtr(-gi(0, 0)); }
   RH_DEV R ralpha() const { return R(1) / alpha(); }
   RH_DEV R beta(int n) const { const R a = alpha(); return a * a * gi(0, n); }
@@ -103,9 +116,11 @@ enum { MK_G00, MK_G01, MK_G02, MK_G11, MK_G12, MK_G22, MK_G33, MK_DETG, MK_ALPHA
 template <class R>
 struct MetK {
   const R* __restrict__ b;
-  long long P2, q;
-  RH_DEV MetK(const void* tab, long long P2_, long long q_) : b((const R*)tab), P2(P2_), q(q_) {}
-  RH_DEV R at(int pl) const { return b[(long long)pl * P2 + q]; }
+  long long P2;
+  unsigned q;
+  RH_DEV MetK(const void* tab, long long P2_, unsigned q_)
+      : b((const R*)tab), P2(P2_), q(q_ * (unsigned)sizeof(R)) {}
+  RH_DEV R at(int pl) const { return ld_(b + (long long)pl * P2, q); }
   RH_DEV R g(int m, int n) const {
     const int lo = m < n ? m : n, hi = m < n ? n : m;
     if (hi == 3) return lo == 3 ? at(MK_G33) : R(0);

@@ -14,9 +14,12 @@
 
 namespace rh {
 
-RH_DEV long long cidx(int i, int j, int k, const Geo& G) {
-  const long long jr = G.jfix ? 0 : (long long)(j - 1);
-  return (long long)(i - 1) + (long long)G.ni * (jr + (long long)G.njs * (long long)(k - 1));
+// Cell and (i,k) indices, thread and workgroup numbers are 32-bit (cells are
+// below 2^29): a 64-bit division, four of which decode a thread's (i,j,k),
+// takes several times the instructions of a 32-bit one.
+RH_DEV unsigned cidx(int i, int j, int k, const Geo& G) {
+  const unsigned jr = G.jfix ? 0u : (unsigned)(j - 1);
+  return (unsigned)(i - 1) + (unsigned)G.ni * (jr + (unsigned)G.njs * (unsigned)(k - 1));
 }
 // j range of a box: the stored row of a collapsed model, else [lo, hi]
 RH_DEV int jlo(const Geo& G, int lo) { return G.jfix ? G.jfix : lo; }
@@ -24,38 +27,32 @@ RH_DEV int jhi(const Geo& G, int hi) { return G.jfix ? G.jfix : hi; }
 // strides of a step in j and in k in the stored planes
 RH_DEV long long jstride(const Geo& G) { return G.jfix ? 0LL : (long long)G.ni; }
 RH_DEV long long kstride(const Geo& G) { return (long long)G.ni * G.njs; }
-RH_DEV long long q2(int i, int k, const Geo& G) { return (long long)(i - 1) + (long long)G.ni * (long long)(k - 1); }
+RH_DEV unsigned q2(int i, int k, const Geo& G) { return (unsigned)(i - 1) + (unsigned)G.ni * (unsigned)(k - 1); }
 
 // 1-based (i,j,k) of linear thread t over a box [lo_a, hi_a] per axis; false if outside.
-RH_DEV bool box_index(long long t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j, int& k) {
-  const long long ci = ihi - ilo + 1, cj = jhi - jlo + 1, ck = khi - klo + 1;
-  if (ci <= 0 || cj <= 0 || ck <= 0 || t >= ci * cj * ck) return false;
-  i = ilo + (int)(t % ci);
-  const long long r = t / ci;
-  j = jlo + (int)(r % cj);
-  k = klo + (int)(r / cj);
+RH_DEV bool box_index(unsigned t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j, int& k) {
+  if (ihi < ilo || jhi < jlo || khi < klo) return false;
+  const unsigned ci = ihi - ilo + 1, cj = jhi - jlo + 1, ck = khi - klo + 1;
+  const unsigned r = t / ci, kk = r / cj;
+  if (kk >= ck) return false;
+  i = ilo + (int)(t - r * ci);
+  j = jlo + (int)(r - kk * cj);
+  k = klo + (int)kk;
   return true;
 }
 
 // Workgroup b is dispatched to XCD b % 8.  Renumbering the workgroups so that
 // each XCD takes one contiguous eighth of the launch keeps neighbouring rows
 // of a stencil in the same L2.  A bijection on [0, gridDim.x).
-RH_DEV long long xcd_block() {
+RH_DEV unsigned xcd_block() {
   const unsigned nb = gridDim.x, b = blockIdx.x, x = b % 8u, idx = b / 8u, q = nb / 8u, r = nb % 8u;
-  return x < r ? (long long)x * (q + 1) + idx : (long long)r * (q + 1) + (long long)(x - r) * q + idx;
+  return x < r ? x * (q + 1) + idx : r * (q + 1) + (x - r) * q + idx;
 }
-RH_DEV long long xcd_thread() { return xcd_block() * blockDim.x + threadIdx.x; }
 
 // As box_index with the j and k axes swapped in the ordering (i fastest, then
 // k, then j): consecutive workgroups step along k, the k sweep's stencil axis.
-RH_DEV bool box_index_ikj(long long t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j, int& k) {
-  const long long ci = ihi - ilo + 1, cj = jhi - jlo + 1, ck = khi - klo + 1;
-  if (ci <= 0 || cj <= 0 || ck <= 0 || t >= ci * cj * ck) return false;
-  i = ilo + (int)(t % ci);
-  const long long r = t / ci;
-  k = klo + (int)(r % ck);
-  j = jlo + (int)(r / ck);
-  return true;
+RH_DEV bool box_index_ikj(unsigned t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j, int& k) {
+  return box_index(t, ilo, ihi, klo, khi, jlo, jhi, i, k, j);
 }
 
 // Waves along the D axis (D = 2 or 3): a lane's i within a 64-wide chunk
@@ -63,28 +60,16 @@ RH_DEV bool box_index_ikj(long long t, int ilo, int ihi, int jlo, int jhi, int k
 // the cell's index along D is the same in every lane of a wave.  Covers
 // 64*ceil(ci/64)*cj*ck indices; lanes past the row's end return false.
 template <int D>
-RH_DEV bool box_index_wave(long long t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j,
+RH_DEV bool box_index_wave(unsigned t, int ilo, int ihi, int jlo, int jhi, int klo, int khi, int& i, int& j,
                            int& k) {
-  const long long ci = ihi - ilo + 1, cj = jhi - jlo + 1, ck = khi - klo + 1;
-  if (ci <= 0 || cj <= 0 || ck <= 0) return false;
-  const long long nic = (ci + 63) / 64;
-  const long long w = t >> 6;
-  long long ic;
-  if (D == 2) {
-    j = jlo + (int)(w % cj);
-    const long long r = w / cj;
-    ic = r % nic;
-    const long long kk = r / nic;
-    if (kk >= ck) return false;
-    k = klo + (int)kk;
-  } else {
-    k = klo + (int)(w % ck);
-    const long long r = w / ck;
-    ic = r % nic;
-    const long long jj = r / nic;
-    if (jj >= cj) return false;
-    j = jlo + (int)jj;
-  }
+  if (ihi < ilo || jhi < jlo || khi < klo) return false;
+  const unsigned ci = ihi - ilo + 1, cj = jhi - jlo + 1, ck = khi - klo + 1;
+  const unsigned nic = (ci + 63) / 64, w = t >> 6;
+  const unsigned n1 = D == 2 ? cj : ck, n2 = D == 2 ? ck : cj;
+  const unsigned r = w / n1, a = w - r * n1, b = r / nic, ic = r - b * nic;
+  if (b >= n2) return false;
+  j = jlo + (int)(D == 2 ? a : b);
+  k = klo + (int)(D == 2 ? b : a);
   i = ilo + (int)(ic * 64 + (t & 63));
   return i <= ihi;
 }
@@ -100,12 +85,12 @@ enum { C_FALLBACK = 0, C_FAIL, C_NEGRHO, C_NEGP, C_VSQGT1, C_DET0, C_WGCARRY, C_
 // writer at a time; k_sum_counters folds the rows when counters are read.
 // (Device-scope atomics on a few addresses from every wave serialise across
 // the XCDs: they cost more than the kernels that raise the events.)
-RH_DEV void count_wave(unsigned long long* cpart, long long blk, int slot, bool flag,
+RH_DEV void count_wave(unsigned long long* cpart, unsigned blk, int slot, bool flag,
                        unsigned long long weight = 1) {
   const unsigned long long b = __ballot(flag);
   if (b && (threadIdx.x % warpSize) == (unsigned)(__ffsll((long long)b) - 1)) {
-    const long long w = (blk * blockDim.x + threadIdx.x) / warpSize;
-    cpart[w * C_NCOUNT + slot] += (unsigned long long)__popcll(b) * weight;
+    const unsigned w = (blk * blockDim.x + threadIdx.x) / warpSize;
+    cpart[(unsigned long long)w * C_NCOUNT + slot] += (unsigned long long)__popcll(b) * weight;
   }
 }
 
@@ -302,7 +287,7 @@ RH_DEV void ppm_var(const R u[5], const PpmCoef<R>& k, int n, R f2, R eta, R& l_
 // sweep's box across.  R: arithmetic and storage type of the edges.
 // ------------------------------------------------------------------------
 template <int D, class R>
-RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, long long blk) {
+RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, unsigned blk) {
   const double* __restrict__ W = A.W;
   const double* __restrict__ dxs = A.dxs;
   const double* __restrict__ xs = A.xs;
@@ -310,7 +295,7 @@ RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, long long blk) {
   const double gam = A.gam;
   R* __restrict__ E = (R*)A.E;
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   const int hi = G.ni - G.nm0 + (D == 1), hj = jhi(G, G.nj - G.nm0 + (D == 2)), hk = G.nk - G.nm0 + (D == 3);
   const int lj = jlo(G, G.nm0);
   const bool in = (D == 1) ? box_index(t, G.nm0, hi, lj, hj, G.nm0, hk, i, j, k)
@@ -318,7 +303,7 @@ RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, long long blk) {
   if (!in) return;
   const long long N = G.N;
   const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
-  const long long c = cidx(i, j, k, G);
+  const unsigned c = cidx(i, j, k, G);
   // along j and k every lane of a wave has the same index along D: its
   // coefficients and widths are loaded once per wave, into scalar registers
   const int p = (D == 1) ? i : __builtin_amdgcn_readfirstlane((D == 2) ? j : k);
@@ -353,13 +338,13 @@ RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, long long blk) {
 // distances (+1e-12), the MC limiter, edges at the cell's faces; stored like
 // the PPM edges.  A.pc holds the face positions x*a of the direction.
 template <int D, class R>
-RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, long long blk) {
+RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, unsigned blk) {
   const double* __restrict__ W = A.W;
   const double* __restrict__ xs = A.xs;
   const double* __restrict__ xa = A.pc;
   R* __restrict__ E = (R*)A.E;
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   const int hi = G.ni - G.nm0 + (D == 1), hj = jhi(G, G.nj - G.nm0 + (D == 2)), hk = G.nk - G.nm0 + (D == 3);
   const int lj = jlo(G, G.nm0);
   const bool in = (D == 3) ? box_index_ikj(t, G.nm0, hi, lj, hj, G.nm0, hk, i, j, k)
@@ -367,7 +352,7 @@ RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, long long blk) {
   if (!in) return;
   const long long N = G.N;
   const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
-  const long long c = cidx(i, j, k, G);
+  const unsigned c = cidx(i, j, k, G);
   const int p = (D == 1) ? i : (D == 2) ? j : k;
   const R small = R(1.0e-12);
   const R xp = R(xs[p]), xc = R(xs[p - 1]), xm = R(xs[p - 2]), xap = R(xa[p - 1]), xam = R(xa[p - 2]);
@@ -390,7 +375,7 @@ RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, long long blk) {
 // caluu3 -> calflx3 -> calcha -> hlle, written to F (and the transverse B
 // fluxes to their CTsrc planes).  SAME: the two face states are the same.
 template <int D, class R, int ICHA, bool SAME = false, class MT>
-RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, long long c, int i, int j, int k,
+RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, unsigned c, int i, int j, int k,
                        const MT& M, R gam, const R wl[9], const R wr[9]) {
   const long long N = G.N;
   const R detg = M.detg();
@@ -418,7 +403,7 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
   const R cmax = fmaxf_(fmaxf_(R(0), vpr), vpl);
   const R cmin = (D == 3) ? fminf_(fminf_(R(0), vpr), vml)   // calcha.f90:107
                           : fminf_(fminf_(R(0), vmr), vml);
-  R* Fo = F + c;
+  const unsigned co = c * (unsigned)sizeof(R);
   // transverse B fluxes of this direction and their CTsrc planes
   // (0 ww(2,7) 1 ww(3,7) 2 ww(1,8) 3 ww(3,8) 4 ww(1,9) 5 ww(2,9))
   constexpr int nA = (D == 1) ? 7 : 6, nB = (D == 3) ? 7 : 8;
@@ -433,17 +418,17 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
       const R c1 = fmaxf_(absr(cmax), absr(cmin));
       o = double(R(0.5) * mad_(-c1, Ur[n] - Ul[n], Fl[n] + Fr[n]));
     } else if (cmax <= R(0)) o = double(Fr[n]);
-    else o = Fo[(long long)n * N];  // unordered (NaN) speeds: hlle keeps ww, then flushes it
+    else o = F[(long long)n * N + c];  // unordered (NaN) speeds: hlle keeps ww, then flushes it
     if (absr(o) < 1.0e-40) o = 0.0;
     // the labelled non-reference form: no flux of the normal field component
     // (the induction flux itself is zero; HLLE's dissipation term is what
     // the reference keeps, hll.f90:109-111), so flux-CT keeps div B
     if (n == 5 + D && G.divb0) o = 0.0;
     if (n == nA || n == nB) {
-      CTsrc[(long long)(n == nA ? pA : pB) * N + c] = R(o);
-      if (!in_ct) Fo[(long long)n * N] = R(o);  // inside the CT box fluxct writes this slot
+      st_(CTsrc + (long long)(n == nA ? pA : pB) * N, co, R(o));
+      if (!in_ct) st_(F + (long long)n * N, co, R(o));  // inside the CT box fluxct writes this slot
     } else {
-      Fo[(long long)n * N] = R(o);
+      st_(F + (long long)n * N, co, R(o));
     }
   }
 }
@@ -460,14 +445,14 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, l
 //
 // PPM's face values come from k_ppm_edges (E); MP5 and WENO5 reconstruct here.
 template <int D, int IREC, class R, int ICHA, bool MK>
-RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
+RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, unsigned blk) {
   const double* __restrict__ W = A.W;
   const R* __restrict__ E = (const R*)A.E;
   R* __restrict__ F = (R*)A.F;
   R* __restrict__ CTsrc = (R*)A.CTsrc;
   const R gam = R(A.gam);
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   const int lj = jlo(G, G.nm0), hj = jhi(G, G.nj - G.nm0);
   // k sweeps that read a stencil along k (MP5, WENO5) walk k before j so
   // neighbouring workgroups share the stencil planes in L2; with the face
@@ -479,18 +464,23 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, long long blk) {
   if (!in) return;
   const long long N = G.N;
   const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
-  const long long c = cidx(i, j, k, G);
+  const unsigned c = cidx(i, j, k, G);
   R wl[9], wr[9];
   if (IREC == 5 || IREC == 1) {
     // right edge of cell c (uri*l(c)) and left edge of cell c+1 (uri*r(c)),
     // both stored at interface c+1/2's index
 #pragma unroll
-    for (int n = 0; n < 9; n++) { wl[n] = E[(long long)(9 + n) * N + c]; wr[n] = E[(long long)n * N + c]; }
+    for (int n = 0; n < 9; n++) {
+      wl[n] = ld_(E + (long long)(9 + n) * N, c * (unsigned)sizeof(R));
+      wr[n] = ld_(E + (long long)n * N, c * (unsigned)sizeof(R));
+    }
   } else {
+    const unsigned c8 = c * 8u;
 #pragma unroll
     for (int n = 0; n < 9; n++) {
-      const double* Pn = W + (long long)n * N + c;
-      const R a = R(Pn[-2 * s]), b = R(Pn[-s]), cc = R(Pn[0]), d = R(Pn[s]), e = R(Pn[2 * s]), f = R(Pn[3 * s]);
+      const double* Pn = W + (long long)n * N;
+      const R a = R(ld_(Pn - 2 * s, c8)), b = R(ld_(Pn - s, c8)), cc = R(ld_(Pn, c8)), d = R(ld_(Pn + s, c8)),
+              e = R(ld_(Pn + 2 * s, c8)), f = R(ld_(Pn + 3 * s, c8));
       if (IREC == 6) {
         const R sl[5] = {a, b, cc, d, e};
         const R sr[5] = {b, cc, d, e, f};
@@ -539,7 +529,7 @@ constexpr int PS_NV = 8;                                     // reconstructed va
 RH_DEV constexpr int ps_plane(int q) { return q < 5 ? q : q + 1; }
 
 template <int D, class R, int ICHA, bool MK>
-RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
+RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, unsigned blk) {
   const int bt = blockDim.x, tid = threadIdx.x;
   const long long N = G.N;
   const double* __restrict__ W = A.W;
@@ -557,7 +547,7 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
     R w[9];
 #pragma unroll
     for (int n = 0; n < 9; n++) {
-      const R u = n == 5 ? R(0) : R(W[(long long)n * N + c]);
+      const R u = n == 5 ? R(0) : R(ld_(W + (long long)n * N, c * 8u));
       w[n] = absr(u) == R(__builtin_inf()) ? R(__builtin_nan("")) : u;
     }
     const MetOf<MK, R> M(A.metF, G.P2, q2(i, k, G));
@@ -611,21 +601,21 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
     k = D == 2 ? G.nm0 + (int)tt : p;
   }
   const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
-  const long long c = cidx(i, j, k, G);
+  const unsigned c = cidx(i, j, k, G), c8 = c * 8u;
   // the lane's own cell from memory, its neighbours from the lanes beside it
   // (the tile's first and last cells read theirs)
   const int nx = pl < TP - 1 ? st : 0, pv = pl > 0 ? -st : 0;
   R um[PS_NV], u0[PS_NV], up[PS_NV], ue[PS_NV];
 #pragma unroll
-  for (int q = 0; q < PS_NV; q++) u0[q] = R(W[(long long)ps_plane(q) * N + c]);
+  for (int q = 0; q < PS_NV; q++) u0[q] = R(ld_(W + (long long)ps_plane(q) * N, c8));
   const bool edge = pl == 0 || pl == TP - 1;
   if (edge) {
-    const long long ce = c + (pl == 0 ? -s : s);
+    const unsigned e8 = c8 + (pl == 0 ? 0u - (unsigned)s : (unsigned)s) * 8u;
 #pragma unroll
-    for (int q = 0; q < PS_NV; q++) ue[q] = R(W[(long long)ps_plane(q) * N + ce]);
+    for (int q = 0; q < PS_NV; q++) ue[q] = R(ld_(W + (long long)ps_plane(q) * N, e8));
   }
   // (the cell at phi + 3 has no second neighbour and needs no indicator)
-  const R pm2 = R(W[4 * N + c - 2 * s]), pp2 = R(W[4 * N + c + (p < phi + 3 ? 2 : 1) * s]);
+  const R pm2 = R(ld_(W + 4 * N - 2 * s, c8)), pp2 = R(ld_(W + 4 * N, c8 + (unsigned)((p < phi + 3 ? 2 : 1) * s) * 8u));
   const long long npc = ((D == 1) ? G.ni : (D == 2) ? G.nj : G.nk) + 2;
   const double* __restrict__ pc = A.pc + p;
 #pragma unroll
@@ -703,43 +693,45 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, long long blk) {
 // in the mixed form); the averages are formed in double.
 // ------------------------------------------------------------------------
 template <class FT>
-RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, long long blk) {
+RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, unsigned blk) {
   const FT* __restrict__ CTsrc = (const FT*)A.CTsrc;
   FT* __restrict__ F1 = (FT*)A.F1;
   FT* __restrict__ F2 = (FT*)A.F2;
   FT* __restrict__ F3 = (FT*)A.F3;
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   if (!box_index(t, G.nm1, G.ni - G.nm1, jlo(G, G.nm1), jhi(G, G.nj - G.nm1), G.nm1, G.nk - G.nm1, i, j, k)) return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
   const long long si = 1, sj = jstride(G), sk = kstride(G);
-  const FT* fyx = CTsrc + 0 * N;  // ww(2,7)
-  const FT* fzx = CTsrc + 1 * N;  // ww(3,7)
-  const FT* fxy = CTsrc + 2 * N;  // ww(1,8)
-  const FT* fzy = CTsrc + 3 * N;  // ww(3,8)
-  const FT* fxz = CTsrc + 4 * N;  // ww(1,9)
-  const FT* fyz = CTsrc + 5 * N;  // ww(2,9)
+  const unsigned co = c * (unsigned)sizeof(FT);
+  auto fyx = [&](long long d) { return ld_(CTsrc + 0 * N + d, co); };  // ww(2,7)
+  auto fzx = [&](long long d) { return ld_(CTsrc + 1 * N + d, co); };  // ww(3,7)
+  auto fxy = [&](long long d) { return ld_(CTsrc + 2 * N + d, co); };  // ww(1,8)
+  auto fzy = [&](long long d) { return ld_(CTsrc + 3 * N + d, co); };  // ww(3,8)
+  auto fxz = [&](long long d) { return ld_(CTsrc + 4 * N + d, co); };  // ww(1,9)
+  auto fyz = [&](long long d) { return ld_(CTsrc + 5 * N + d, co); };  // ww(2,9)
   const double c8 = 1.0 / 8.0;
   // 2.0 * x leads each sum, so every term is added in double
   double v[6];
-  v[0] = c8 * (2.0 * fyx[c] + fyx[c + si] + fyx[c - si] - fxy[c] - fxy[c + sj] - fxy[c - si] - fxy[c - si + sj]);
-  v[1] = c8 * (2.0 * fzx[c] + fzx[c + si] + fzx[c - si] - fxz[c] - fxz[c + sk] - fxz[c - si] - fxz[c - si + sk]);
-  v[2] = c8 * (2.0 * fxy[c] + fxy[c + sj] + fxy[c - sj] - fyx[c] - fyx[c + si] - fyx[c - sj] - fyx[c + si - sj]);
-  v[3] = c8 * (2.0 * fzy[c] + fzy[c + sj] + fzy[c - sj] - fyz[c] - fyz[c + sk] - fyz[c - sj] - fyz[c - sj + sk]);
-  v[4] = c8 * (2.0 * fxz[c] + fxz[c + sk] + fxz[c - sk] - fzx[c] - fzx[c + si] - fzx[c - sk] - fzx[c + si - sk]);
-  v[5] = c8 * (2.0 * fyz[c] + fyz[c + sk] + fyz[c - sk] - fzy[c] - fzy[c + sj] - fzy[c - sk] - fzy[c + sj - sk]);
-  F2[6 * N + c] = FT(v[0]);
-  F3[6 * N + c] = FT(v[1]);
-  F1[7 * N + c] = FT(v[2]);
-  F3[7 * N + c] = FT(v[3]);
-  F1[8 * N + c] = FT(v[4]);
-  F2[8 * N + c] = FT(v[5]);
+  v[0] = c8 * (2.0 * fyx(0) + fyx(si) + fyx(-si) - fxy(0) - fxy(sj) - fxy(-si) - fxy(-si + sj));
+  v[1] = c8 * (2.0 * fzx(0) + fzx(si) + fzx(-si) - fxz(0) - fxz(sk) - fxz(-si) - fxz(-si + sk));
+  v[2] = c8 * (2.0 * fxy(0) + fxy(sj) + fxy(-sj) - fyx(0) - fyx(si) - fyx(-sj) - fyx(si - sj));
+  v[3] = c8 * (2.0 * fzy(0) + fzy(sj) + fzy(-sj) - fyz(0) - fyz(sk) - fyz(-sj) - fyz(-sj + sk));
+  v[4] = c8 * (2.0 * fxz(0) + fxz(sk) + fxz(-sk) - fzx(0) - fzx(si) - fzx(-sk) - fzx(si - sk));
+  v[5] = c8 * (2.0 * fyz(0) + fyz(sk) + fyz(-sk) - fzy(0) - fzy(sj) - fzy(-sk) - fzy(sj - sk));
+  st_(F2 + 6 * N, co, FT(v[0]));
+  st_(F3 + 6 * N, co, FT(v[1]));
+  st_(F1 + 7 * N, co, FT(v[2]));
+  st_(F3 + 7 * N, co, FT(v[3]));
+  st_(F1 + 8 * N, co, FT(v[4]));
+  st_(F2 + 8 * N, co, FT(v[5]));
   // the mixed form keeps the CT update of B in FP64: the update reads these
   // (the float copies above are what a later sweep keeps where its wave
   // speeds are unordered, as ww keeps what ct wrote)
   if (sizeof(FT) == 4 && A.CTd) {
 #pragma unroll
-    for (int q = 0; q < 6; q++) A.CTd[(long long)q * N + c] = v[q];
+    for (int q = 0; q < 6; q++) st_(A.CTd + (long long)q * N, c * 8u, v[q]);
   }
 }
 
@@ -1173,16 +1165,17 @@ RH_DEV long long chr_plane(int l, int a, int b) {
 }
 
 template <int STAGE, bool SYM, class FT, bool MK>
-RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
+RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
   const FT* __restrict__ F1 = (const FT*)A.F1;
   const FT* __restrict__ F2 = (const FT*)A.F2;
   const FT* __restrict__ F3 = (const FT*)A.F3;
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   if (!box_index(t, G.nm1 + 1, G.ni - G.nm1, jlo(G, G.nm1 + 1), jhi(G, G.nj - G.nm1), G.nm1 + 1, G.nk - G.nm1, i, j,
                  k))
     return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G), c8 = c * 8u;
   const long long sj = jstride(G), sk = kstride(G);
   const double gam = A.gam;
   // dt and dt/dx (main.f90:760-780), recomputed per thread from the CFL minimum
@@ -1199,7 +1192,7 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
 
   double w[9];
 #pragma unroll
-  for (int n = 0; n < 9; n++) w[n] = A.W[(long long)n * N + c];
+  for (int n = 0; n < 9; n++) w[n] = ld_(A.W + (long long)n * N, c8);
 
   // geometric source: sf(2..5) = sqrt(-g) T^m_n Gamma^n_{(1,2,3,0) m}
   double sf[4];
@@ -1207,17 +1200,17 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
     Prel s;
     prelude(w, gam, M, s);
     double ta = 0.0, tb = 0.0, tc = 0.0, td = 0.0;
-    const long long q = q2(i, k, G);
+    const unsigned q = q2(i, k, G) * 8u;
 #pragma unroll
     for (int n = 0; n < 4; n++)
 #pragma unroll
       for (int m = 0; m < 4; m++) {
         const double dl = (m == n) ? 1.0 : 0.0;
         const double tv = (s.roh + s.bbsq) * s.ucon[m] * s.ucov[n] + (s.pr + 0.5 * s.bbsq) * dl - s.bb[m] * s.bbcov[n];
-        ta = ta + tv * A.chr[chr_plane<SYM>(n, 1, m) * G.P2 + q];
-        tb = tb + tv * A.chr[chr_plane<SYM>(n, 2, m) * G.P2 + q];
-        tc = tc + tv * A.chr[chr_plane<SYM>(n, 3, m) * G.P2 + q];
-        td = td + tv * A.chr[chr_plane<SYM>(n, 0, m) * G.P2 + q];
+        ta = ta + tv * ld_(A.chr + chr_plane<SYM>(n, 1, m) * G.P2, q);
+        tb = tb + tv * ld_(A.chr + chr_plane<SYM>(n, 2, m) * G.P2, q);
+        tc = tc + tv * ld_(A.chr + chr_plane<SYM>(n, 3, m) * G.P2, q);
+        td = td + tv * ld_(A.chr + chr_plane<SYM>(n, 0, m) * G.P2, q);
       }
     const double dg = M.detg();
     sf[0] = dg * ta; sf[1] = dg * tb; sf[2] = dg * tc; sf[3] = dg * td;
@@ -1229,22 +1222,23 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
   const bool ctd = sizeof(FT) == 4 && A.CTd;
 #pragma unroll
   for (int m = 0; m < 9; m++) {
-    const long long o = (long long)m * N + c;
+    const long long o = (long long)m * N;
     auto fl = [&](const FT* Fd, int d, long long off) -> double {
-      if (m >= 6 && ctd && ctp[m - 6][d] >= 0) return A.CTd[(long long)ctp[m - 6][d] * N + c - off];
-      return double(Fd[o - off]);
+      if (m >= 6 && ctd && ctp[m - 6][d] >= 0) return ld_(A.CTd + (long long)ctp[m - 6][d] * N - off, c8);
+      return double(ld_(Fd + o - off, c * (unsigned)sizeof(FT)));
     };
+    const double ua = ld_(A.Ua + o, c8), ub = STAGE == 1 ? 0.0 : ld_(A.Ub + o, c8);
     const double d1 = fl(F1, 0, 0) - fl(F1, 0, 1), d2 = fl(F2, 1, 0) - fl(F2, 1, sj),
                  d3 = fl(F3, 2, 0) - fl(F3, 2, sk);
     double v;
     if (STAGE == 1) {
-      v = A.Ua[o] - a1 * d1 - a2 * d2 - a3 * d3;
+      v = ua - a1 * d1 - a2 * d2 - a3 * d3;
     } else if (STAGE == 2) {
-      v = (A.Ua[o] + A.Ub[o]) * 0.5 + (-a1 * d1 - a2 * d2 - a3 * d3) * 0.5;
+      v = (ua + ub) * 0.5 + (-a1 * d1 - a2 * d2 - a3 * d3) * 0.5;
     } else if (STAGE == 3) {
-      v = (3.0 * A.Ua[o] + A.Ub[o]) * 0.25 + (-a1 * d1 - a2 * d2 - a3 * d3) * 0.25;
+      v = (3.0 * ua + ub) * 0.25 + (-a1 * d1 - a2 * d2 - a3 * d3) * 0.25;
     } else {
-      v = (A.Ua[o] + 2.0 * A.Ub[o]) * (double)(1.0f / 3.0f) + (-a1 * d1 - a2 * d2 - a3 * d3) * (double)(2.0f / 3.0f);
+      v = (ua + 2.0 * ub) * (double)(1.0f / 3.0f) + (-a1 * d1 - a2 * d2 - a3 * d3) * (double)(2.0f / 3.0f);
     }
     if (m >= 1 && m <= 4) {
       const double sdt = sf[m - 1] * dt;
@@ -1253,7 +1247,7 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
       else if (STAGE == 3) v = v + sdt * 0.25;
       else v = v + sdt * (double)(2.0f / 3.0f);
     }
-    A.Ukeep[o] = v;
+    st_(A.Ukeep + o, c8, v);
   }
 }
 
@@ -1261,19 +1255,20 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, long long blk) {
 // interior cell from the stage's RK result; cells whose initial W is
 // inherited are flagged for k_recov_carry.
 template <int IW, bool MK>
-RH_DEV void b_recov(const Geo& G, const StageArgs& A, long long blk) {
+RH_DEV void b_recov(const Geo& G, const StageArgs& A, unsigned blk) {
   int i, j, k;
-  const long long t = blk * blockDim.x + threadIdx.x;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   if (!box_index(t, G.nm1 + 1, G.ni - G.nm1, jlo(G, G.nm1 + 1), jhi(G, G.nj - G.nm1), G.nm1 + 1, G.nk - G.nm1, i, j,
                  k))
     return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
   const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
   double w[9], u[9];
 #pragma unroll
   for (int n = 0; n < 9; n++) {
-    w[n] = A.W[(long long)n * N + c];
-    u[n] = A.Ukeep[(long long)n * N + c];
+    w[n] = ld_(A.W + (long long)n * N, c * 8u);
+    u[n] = ld_((const double*)A.Ukeep + (long long)n * N, c * 8u);
   }
   RecovOut ro;
   bool carry;
@@ -1282,8 +1277,8 @@ RH_DEV void b_recov(const Geo& G, const StageArgs& A, long long blk) {
                 wgout);
   const bool dep = carry && !ro.indep;
 #pragma unroll
-  for (int n = 0; n < 9; n++) A.Wpre[(long long)n * N + c] = ro.w[n];
-  A.wgout[c] = wgout;
+  for (int n = 0; n < 9; n++) st_(A.Wpre + (long long)n * N, c * 8u, ro.w[n]);
+  st_(A.wgout, c * 8u, wgout);
   // a flagged cell's outcome is counted when the fix-up computes it
   count_wave(A.cpart, blk, C_FALLBACK, ro.fallback && !dep);
   count_wave(A.cpart, blk, C_FAIL, ro.fail && !dep);
@@ -1439,10 +1434,11 @@ RH_DEV bool ghost_index(long long t, const Geo& G, int& i, int& j, int& k) {
 // ghost slots of the recovered primitives.  bnd_value reads only interior
 // cells of that array (and the stage-start values of other ghosts), so the
 // writes cannot race with the reads.
-RH_DEV void b_bnd(const Geo& G, const PostArgs& A, long long blk) {
+RH_DEV void b_bnd(const Geo& G, const PostArgs& A, unsigned blk) {
   int i, j, k;
   if (!ghost_index(blk * blockDim.x + threadIdx.x, G, i, j, k)) return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
   const BndCtx B{&G, A.Wpre, A.Wold, A.Wo, A.bc};
 #pragma unroll 1
   for (int n = 0; n < 9; n++) A.Wghost[(long long)n * N + c] = bnd_value(B, n, i, j, k);
@@ -1460,16 +1456,17 @@ RH_DEV MetOf<MK, double> reload_met(const void* metC, const Geo& G, int i, int k
 }
 
 template <bool MK>
-RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
-  const long long t = blk * blockDim.x + threadIdx.x;
+RH_DEV void b_post(const Geo& G, const PostArgs& A, unsigned blk) {
+  const unsigned t = blk * blockDim.x + threadIdx.x;
   int i, j, k;
   if (!box_index(t, 1, G.ni, jlo(G, 1), jhi(G, G.nj), 1, G.nk, i, j, k)) return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
   const double gam = A.gam;
   const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
   double w[9];
 #pragma unroll
-  for (int n = 0; n < 9; n++) w[n] = A.Wpre[(long long)n * N + c];
+  for (int n = 0; n < 9; n++) w[n] = ld_(A.Wpre + (long long)n * N, c * 8u);
   // infchk, outer radial ghosts (bnd.f90:1740-1819); model 7..20
   if (A.model >= 7 && A.model <= 20 && i > G.ni - G.nm1) {
     const double gfl = calgfl(w[1], w[2], w[3], M);
@@ -1564,7 +1561,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
   count_wave(A.cpart, blk, C_PMMSCALE, scaled, rows);
   count_wave(A.cpart, blk, C_PMMFLOOR, hit, rows);
 #pragma unroll
-  for (int n = 0; n < 9; n++) A.Wout[(long long)n * N + c] = w[n];
+  for (int n = 0; n < 9; n++) st_(A.Wout + (long long)n * N, c * 8u, w[n]);
   // caluu1 (caluu.f90:2-126): conserved variables of the final primitives
   {
     const auto M = reload_met<MK>(A.metC, G, i, k);
@@ -1573,7 +1570,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, long long blk) {
     double u[9];
     tmunu_row(s2, 0, M.detg(), pow(s2.de, gam), u);
 #pragma unroll
-    for (int n = 0; n < 9; n++) A.Uout[(long long)n * N + c] = u[n];
+    for (int n = 0; n < 9; n++) st_(A.Uout + (long long)n * N, c * 8u, u[n]);
   }
 }
 
@@ -1597,29 +1594,32 @@ RH_DEV double wave_min(double v) {
   }
   return v;
 }
-RH_DEV long long wave_max_ll(long long v) {
+template <class T>
+RH_DEV T wave_max(T v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    const long long o = __shfl_xor(v, off, 64);
+    const T o = __shfl_xor(v, off, 64);
     v = o > v ? o : v;
   }
   return v;
 }
 
 template <int ICHA, bool MK>
-RH_DEV void b_cfl(const Geo& G, const CflArgs& A, long long blk) {
-  __shared__ long long s_last[4][4];
+RH_DEV void b_cfl(const Geo& G, const CflArgs& A, unsigned blk) {
+  __shared__ int s_last[4][4];
   __shared__ double s_min[4][4];
-  const long long t = blk * blockDim.x + threadIdx.x;
+  // positions of the elements in the reference's order: below 3 * 2^29
+  const int t = (int)(blk * blockDim.x + threadIdx.x);
   int i, j, k;
   double e[4] = {__builtin_inf(), __builtin_inf(), __builtin_inf(), 0.0};  // dtx1a, dtx2a, dtx3a
-  bool valid = box_index(t, 2, G.ni - 1, jlo(G, 2), jhi(G, G.nj - 1), 2, G.nk - 1, i, j, k);
+  bool valid = box_index((unsigned)t, 2, G.ni - 1, jlo(G, 2), jhi(G, G.nj - 1), 2, G.nk - 1, i, j, k);
   if (valid) {
-    const long long N = G.N, c = cidx(i, j, k, G);
+    const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
     const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
     double w[9];
 #pragma unroll
-    for (int n = 0; n < 9; n++) w[n] = A.W[(long long)n * N + c];
+    for (int n = 0; n < 9; n++) w[n] = ld_(A.W + (long long)n * N, c * 8u);
     Prel s;
     prelude(w, A.gam, M, s);
     double vp[4], vm[4];
@@ -1639,10 +1639,10 @@ RH_DEV void b_cfl(const Geo& G, const CflArgs& A, long long blk) {
     }
   }
   // per accumulator: this thread's last NaN position and minimum after it
-  long long last[4];
+  int last[4];
   double mn[4];
   {
-    long long l0 = -1;
+    int l0 = -1;
     double m0 = __builtin_inf();
     if (valid)
 #pragma unroll
@@ -1659,16 +1659,16 @@ RH_DEV void b_cfl(const Geo& G, const CflArgs& A, long long blk) {
     }
   }
   const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
-  long long L[4];
+  int L[4];
 #pragma unroll
   for (int a = 0; a < 4; a++) {
-    const long long v = wave_max_ll(last[a]);
+    const int v = wave_max(last[a]);
     if (lane == 0) s_last[wid][a] = v;
   }
   __syncthreads();
 #pragma unroll
   for (int a = 0; a < 4; a++) {
-    long long v = s_last[0][a];
+    int v = s_last[0][a];
     for (int w = 1; w < (int)(blockDim.x / 64); w++) v = s_last[w][a] > v ? s_last[w][a] : v;
     L[a] = v;
   }
@@ -1717,7 +1717,7 @@ RH_DEV void b_cfl_finish(const CflArgs& A) {
       if (A.blast[4 * b + a] >= 0) bg[a] = b > bg[a] ? b : bg[a];
 #pragma unroll
   for (int a = 0; a < 4; a++) {
-    const long long v = wave_max_ll(bg[a]);
+    const long long v = wave_max(bg[a]);
     if (lane == 0) s_l[wid][a] = v;
   }
   __syncthreads();
@@ -1782,7 +1782,7 @@ RH_DEV long long carry_pred(const Geo& G, long long c, int& i, int& k) {
   const int j = G.jfix ? G.jfix : (int)((c / G.ni) % G.nj) + 1;
   int pi = i - 1, pj = j, pk = k;
   if (pi < G.nm1 + 1) { pi = G.ni - G.nm1; pj = j - 1; if (pj < G.nm1 + 1) { pj = G.nj - G.nm1; pk = k - 1; } }
-  return pk >= G.nm1 + 1 ? cidx(pi, pj, pk, G) : -1;
+  return pk >= G.nm1 + 1 ? (long long)cidx(pi, pj, pk, G) : -1LL;
 }
 
 template <int IW, bool MK>
@@ -1970,19 +1970,20 @@ hipError_t launch_metric_tables(int ni, int nk, int metric, double akm, const do
 template <bool MK>
 __global__ void __launch_bounds__(256) k_caluu1(Geo G, const double* __restrict__ W, const void* __restrict__ metC,
                                                 double gam, double* __restrict__ U) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
   int i, j, k;
   if (!box_index(t, 1, G.ni, jlo(G, 1), jhi(G, G.nj), 1, G.nk, i, j, k)) return;
-  const long long N = G.N, c = cidx(i, j, k, G);
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
   const MetOf<MK, double> M(metC, G.P2, q2(i, k, G));
   double w[9], u[9];
 #pragma unroll
-  for (int n = 0; n < 9; n++) w[n] = W[(long long)n * N + c];
+  for (int n = 0; n < 9; n++) w[n] = ld_(W + (long long)n * N, c * 8u);
   Prel s;
   prelude(w, gam, M, s);
   tmunu_row(s, 0, M.detg(), pow(s.de, gam), u);
 #pragma unroll
-  for (int n = 0; n < 9; n++) U[(long long)n * N + c] = u[n];
+  for (int n = 0; n < 9; n++) st_(U + (long long)n * N, c * 8u, u[n]);
 }
 
 // ------------------------------------------------------------------------
@@ -2043,8 +2044,8 @@ RH_DEV int batch_find(const BatchItem* __restrict__ it, int n, long long b) {
   return lo;
 }
 
-RH_DEV void b_copy(const CopyArgs& A, long long blk) {
-  const long long t = blk * blockDim.x + threadIdx.x;
+RH_DEV void b_copy(const CopyArgs& A, unsigned blk) {
+  const long long t = (long long)blk * blockDim.x + threadIdx.x;
   if (t < A.n) A.dst[t] = A.src[t];
 }
 
@@ -2085,7 +2086,7 @@ __global__ void __launch_bounds__(64) k_advance_time(AdvArgs A) { b_advance_time
 #define RH_BATCH_PROLOGUE                                  \
   const int q = batch_find(it, n, (long long)blockIdx.x);  \
   const Geo G = it[q].G;                                   \
-  const long long blk = (long long)blockIdx.x - it[q].off;
+  const unsigned blk = blockIdx.x - (unsigned)it[q].off;
 template <int D, class R>
 __global__ void __launch_bounds__(256) kb_ppm_edges(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
