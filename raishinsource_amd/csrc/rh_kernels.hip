@@ -1325,49 +1325,42 @@ RH_DEV void b_recov(const Geo& G, const StageArgs& A, unsigned blk) {
 // atmosphere1a (correction.f90:226), pminmax2b (correction.f90:744) and
 // caluu1 (caluu.f90:2).
 // ------------------------------------------------------------------------
-struct BndCtx {
-  const Geo* G;
+RH_DEV bool is_ghost(int p, int n, int nm1) { return p <= nm1 || p > n - nm1; }
+
+// p folded into the interior by whole periods (nm1 periods reach past every ghost)
+RH_DEV int fold(int p, int n, int nm1) {
+  const unsigned Wd = (unsigned)(n - 2 * nm1);
+  return nm1 + 1 + (int)((unsigned)(p - (nm1 + 1) + nm1 * (int)Wd) % Wd);
+}
+
+// One variable's planes and boundary codes (bc[axis*2+side]) in the ghost fill.
+struct BndVar {
   const double* Wpre;   // post-recov interior values
   const double* Wold;   // values before this stage (ghosts not rewritten keep these)
   const double* Wo;     // primitives at the start of the step (fixed-value type 2)
-  const int* bc;        // [axis*2+side][m] boundary codes
+  const int *bc, *bc2;  // its codes bc[axis*2+side], and those of u^1
+  long long v2;         // from these planes to those of u^1
 };
 
-RH_DEV bool is_ghost(int p, int n, int nm1) { return p <= nm1 || p > n - nm1; }
-
 // value after the periodic pass (bndpefb4)
-RH_DEV double bnd_s0(const BndCtx& B, int m, int i, int j, int k) {
-  const Geo& G = *B.G;
+RH_DEV double bnd_s0(const Geo& G, const BndVar& B, int i, int j, int k) {
   const int nm1 = G.nm1;
   const bool gi = is_ghost(i, G.ni, nm1), gj = is_ghost(j, G.nj, nm1), gk = is_ghost(k, G.nk, nm1);
   const int ng = (int)gi + (int)gj + (int)gk;
-  if (ng == 0) return B.Wpre[(long long)m * G.N + cidx(i, j, k, G)];
+  bool inner = ng == 0;
   if (ng == 1) {
-    if (gi && (B.bc[0 * 9 + m] == 1 || B.bc[1 * 9 + m] == 1)) {
-      const int Wd = G.ni - 2 * nm1;
-      const int ii = nm1 + 1 + (((i - (nm1 + 1)) % Wd) + Wd) % Wd;
-      return B.Wpre[(long long)m * G.N + cidx(ii, j, k, G)];
-    }
-    if (gj && (B.bc[2 * 9 + m] == 1 || B.bc[3 * 9 + m] == 1)) {
-      const int Wd = G.nj - 2 * nm1;
-      const int jj = nm1 + 1 + (((j - (nm1 + 1)) % Wd) + Wd) % Wd;
-      return B.Wpre[(long long)m * G.N + cidx(i, jj, k, G)];
-    }
-    if (gk && (B.bc[4 * 9 + m] == 1 || B.bc[5 * 9 + m] == 1)) {
-      const int Wd = G.nk - 2 * nm1;
-      const int kk = nm1 + 1 + (((k - (nm1 + 1)) % Wd) + Wd) % Wd;
-      return B.Wpre[(long long)m * G.N + cidx(i, j, kk, G)];
-    }
+    if (gi && (B.bc[0] == 1 || B.bc[1] == 1)) { i = fold(i, G.ni, nm1); inner = true; }
+    else if (gj && (B.bc[2] == 1 || B.bc[3] == 1)) { j = fold(j, G.nj, nm1); inner = true; }
+    else if (gk && (B.bc[4] == 1 || B.bc[5] == 1)) { k = fold(k, G.nk, nm1); inner = true; }
   }
-  return B.Wold[(long long)m * G.N + cidx(i, j, k, G)];
+  return (inner ? B.Wpre : B.Wold)[cidx(i, j, k, G)];
 }
 
-// Value of variable m at ghost (i,j,k) after the three physical passes.  Each
-// pass maps the cell to its source in the previous pass (copy, mirror, with a
-// sign for antisymmetric codes) or ends in a constant: walking x3 -> x2 -> x1
-// and then reading the periodic-pass value composes the passes exactly.
-RH_DEV double bnd_value(const BndCtx& B, int m, int i, int j, int k) {
-  const Geo& G = *B.G;
+// Value at ghost (i,j,k) after the three physical passes.  Each pass maps the
+// cell to its source in the previous pass (copy, mirror, with a sign for
+// antisymmetric codes) or ends in a constant: walking x3 -> x2 -> x1 and then
+// reading the periodic-pass value composes the passes exactly.
+RH_DEV double bnd_value(const Geo& G, const BndVar& B, int i, int j, int k) {
   const int nm1 = G.nm1;
   double sgn = 1.0;
   int c[4] = {0, i, j, k};
@@ -1377,75 +1370,58 @@ RH_DEV double bnd_value(const BndCtx& B, int m, int i, int j, int k) {
     const int p = c[ax];
     if (!is_ghost(p, n[ax], nm1)) continue;
     const bool outer = p > n[ax] - nm1;
-    const int type = B.bc[((ax - 1) * 2 + (outer ? 1 : 0)) * 9 + m];
-    switch (type) {
-      case 2: return sgn * B.Wo[(long long)m * G.N + cidx(c[1], c[2], c[3], G)];
-      case 5: c[ax] = outer ? n[ax] - nm1 : nm1 + 1; break;
-      case 12: sgn = -sgn; c[ax] = outer ? 2 * n[ax] - 2 * nm1 + 1 - p : 2 * nm1 - p + 1; break;
-      case 13: return sgn * 0.0;
-      case 14: c[ax] = outer ? 2 * n[ax] - 2 * nm1 + 1 - p : 2 * nm1 - p + 1; break;
-      case 18: {
-        // bnd.f90:598-610 (x1 outer only): no inflow through the outer boundary
-        const double v2 = bnd_s0(B, 1, n[ax] - nm1, c[2], c[3]);
-        if (v2 < 0.0) return sgn * 0.0;
-        c[ax] = n[ax] - nm1;
-        break;
-      }
-      default: break;  // 1: periodic, filled by the periodic pass
-    }
+    const int type = outer ? B.bc[(ax - 1) * 2 + 1] : B.bc[(ax - 1) * 2];
+    if (type == 5) {
+      c[ax] = outer ? n[ax] - nm1 : nm1 + 1;
+    } else if (type == 12 || type == 14) {
+      if (type == 12) sgn = -sgn;
+      c[ax] = outer ? 2 * n[ax] - 2 * nm1 + 1 - p : 2 * nm1 - p + 1;
+    } else if (type == 13) {
+      return sgn * 0.0;
+    } else if (type == 2) {
+      return sgn * B.Wo[cidx(c[1], c[2], c[3], G)];
+    } else if (type == 18) {
+      // bnd.f90:598-610 (x1 outer only, u^1 to u^3): no inflow through the outer boundary
+      BndVar V = B;
+      V.Wpre = B.Wpre + B.v2;
+      V.Wold = B.Wold + B.v2;
+      V.bc = B.bc2;
+      if (bnd_s0(G, V, n[ax] - nm1, c[2], c[3]) < 0.0) return sgn * 0.0;
+      c[ax] = n[ax] - nm1;
+    }  // 1: periodic, filled by the periodic pass
   }
-  return sgn * bnd_s0(B, m, c[1], c[2], c[3]);
+  return sgn * bnd_s0(G, B, c[1], c[2], c[3]);
 }
 
 // 1-based (i,j,k) of the t-th ghost cell: the two theta slabs (all i, j),
 // then the two phi slabs (interior k), then the two r slabs (interior j, k).
-RH_DEV bool ghost_index(long long t, const Geo& G, int& i, int& j, int& k) {
-  const long long ni = G.ni, nj = G.nj, nk = G.nk, g = G.nm1;
-  if (t < 0) return false;
-  if (G.jfix) {
-    // collapsed: the stored row's theta and r ghosts (no phi ghosts are stored)
-    const long long nkS1 = 2 * g * ni, niS1 = 2 * g * (nk - 2 * g);
-    j = G.jfix;
-    if (t < nkS1) {
-      i = (int)(t % ni) + 1;
-      const long long kk = t / ni;
-      k = (int)(kk < g ? kk : nk - 2 * g + kk) + 1;
-      return true;
-    }
-    t -= nkS1;
-    if (t < niS1) {
-      const long long ii = t % (2 * g);
-      i = (int)(ii < g ? ii : ni - 2 * g + ii) + 1;
-      k = (int)(g + t / (2 * g)) + 1;
-      return true;
-    }
-    return false;
-  }
-  const long long nkS = 2 * g * ni * nj, njS = 2 * g * ni * (nk - 2 * g), niS = 2 * g * (nj - 2 * g) * (nk - 2 * g);
+// A collapsed model stores no phi ghosts: its row's theta and r ghosts.
+RH_DEV bool ghost_index(unsigned t, const Geo& G, int& i, int& j, int& k) {
+  const unsigned ni = G.ni, nj = G.jfix ? 1u : (unsigned)G.nj, nk = G.nk, g = G.nm1;
+  const unsigned jin = G.jfix ? 1u : nj - 2 * g, j0 = G.jfix ? (unsigned)G.jfix - 1u : 0u;
+  const unsigned nkS = 2 * g * ni * nj, njS = G.jfix ? 0u : 2 * g * ni * (nk - 2 * g), niS = 2 * g * jin * (nk - 2 * g);
+  auto slab = [&](unsigned a, unsigned n) { return (int)(a < g ? a : n - 2 * g + a) + 1; };
   if (t < nkS) {
-    i = (int)(t % ni) + 1;
-    const long long r = t / ni;
-    j = (int)(r % nj) + 1;
-    const long long kk = r / nj;
-    k = (int)(kk < g ? kk : nk - 2 * g + kk) + 1;
+    const unsigned r = t / ni, kk = r / nj;
+    i = (int)(t - r * ni) + 1;
+    j = (int)(j0 + r - kk * nj) + 1;
+    k = slab(kk, nk);
     return true;
   }
   t -= nkS;
   if (t < njS) {
-    i = (int)(t % ni) + 1;
-    const long long r = t / ni;
-    const long long jj = r % (2 * g);
-    j = (int)(jj < g ? jj : nj - 2 * g + jj) + 1;
-    k = (int)(g + r / (2 * g)) + 1;
+    const unsigned r = t / ni, kk = r / (2 * g);
+    i = (int)(t - r * ni) + 1;
+    j = slab(r - kk * 2 * g, nj);
+    k = (int)(g + kk) + 1;
     return true;
   }
   t -= njS;
   if (t < niS) {
-    const long long ii = t % (2 * g);
-    i = (int)(ii < g ? ii : ni - 2 * g + ii) + 1;
-    const long long r = t / (2 * g);
-    j = (int)(g + r % (nj - 2 * g)) + 1;
-    k = (int)(g + r / (nj - 2 * g)) + 1;
+    const unsigned r = t / (2 * g), kk = r / jin;
+    i = slab(t - r * 2 * g, ni);
+    j = (int)((G.jfix ? j0 : g) + r - kk * jin) + 1;
+    k = (int)(g + kk) + 1;
     return true;
   }
   return false;
@@ -1454,15 +1430,36 @@ RH_DEV bool ghost_index(long long t, const Geo& G, int& i, int& j, int& k) {
 // Ghost fill of the stage: bnd4 composed per ghost cell, written into the
 // ghost slots of the recovered primitives.  bnd_value reads only interior
 // cells of that array (and the stage-start values of other ghosts), so the
-// writes cannot race with the reads.
-RH_DEV void b_bnd(const Geo& G, const PostArgs& A, unsigned blk) {
+// writes cannot race with the reads.  A thread takes NV variables of a ghost
+// cell, the same ones in its workgroup (A.nbc workgroups per NV variables),
+// so their codes are scalars and their reads in flight together: one where
+// the launch is then still small (every read's latency counts: one 128x128
+// row 4.4 us, with three 6.4 us), three beyond (they share the thread's index
+// arithmetic: 256x128x128 0.046 ms, with one 0.048; eight 1024-zone tubes
+// 0.054, with one 0.064).  A thread that took the nine in turn waited nine
+// times: 13.2 us, 0.054 and 0.062 ms.
+template <int NV>
+RH_DEV void bnd_cells(const Geo& G, const PostArgs& A, unsigned blk) {
+  const int g = (int)(blk / (unsigned)A.nbc);
   int i, j, k;
-  if (!ghost_index(blk * blockDim.x + threadIdx.x, G, i, j, k)) return;
-  const long long N = G.N;
+  if (!ghost_index((blk - (unsigned)g * (unsigned)A.nbc) * blockDim.x + threadIdx.x, G, i, j, k)) return;
   const unsigned c = cidx(i, j, k, G);
-  const BndCtx B{&G, A.Wpre, A.Wold, A.Wo, A.bc};
-#pragma unroll 1
-  for (int n = 0; n < 9; n++) A.Wghost[(long long)n * N + c] = bnd_value(B, n, i, j, k);
+  double v[NV];
+#pragma unroll
+  for (int q = 0; q < NV; q++) {
+    const int m = NV * g + q;
+    const long long o = (long long)m * G.N;
+    int bc[6], bc2[6];
+#pragma unroll
+    for (int e = 0; e < 6; e++) { bc[e] = A.bc[e * 9 + m]; bc2[e] = A.bc[e * 9 + 1]; }
+    v[q] = bnd_value(G, BndVar{A.Wpre + o, A.Wold + o, A.Wo + o, bc, bc2, (1 - m) * G.N}, i, j, k);
+  }
+#pragma unroll
+  for (int q = 0; q < NV; q++) A.Wghost[(long long)(NV * g + q) * G.N + c] = v[q];
+}
+RH_DEV void b_bnd(const Geo& G, const PostArgs& A, unsigned blk) {
+  if (A.nbv == 1) bnd_cells<1>(G, A, blk);
+  else bnd_cells<3>(G, A, blk);
 }
 
 // infchk + atmosphere1a + pminmax2b + caluu1 on every cell, after k_bnd.
@@ -2511,18 +2508,22 @@ hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st) {
+hipError_t launch_post(const Geo& G, const PostArgs& A0, hipStream_t st) {
   const long long g = G.nm1;
   const long long ng = G.N - (long long)(G.ni - 2 * g) * (G.jfix ? 1 : G.nj - 2 * g) * (G.nk - 2 * g);
   const int bt = slot_threads(G, TS_POST);
+  PostArgs A = A0;
+  A.nbc = ng > 0 ? (int)nblk(ng, bt) : 0;
+  // one variable a thread while that is at most two waves per SIMD (1024 of them)
+  A.nbv = 9 * ng <= 2 * 64 * 1024 ? 1 : 3;
   if (g_rec) {
     AnyArgs a{};
     a.p = A;
-    record(LK_BND, 0, bt, ng > 0 ? nblk(ng, bt) : 0, G, a);
+    record(LK_BND, 0, bt, (9LL / A.nbv) * A.nbc, G, a);
     record(LK_POST, G.mk, bt, nblk(G.N, bt), G, a);
     return hipSuccess;
   }
-  if (ng > 0) hipLaunchKernelGGL(k_bnd, dim3(nblk(ng, bt)), dim3(bt), 0, st, G, A);
+  if (ng > 0) hipLaunchKernelGGL(k_bnd, dim3((unsigned)(9 / A.nbv * A.nbc)), dim3(bt), 0, st, G, A);
   with_mk(G.mk, [&](auto K) {
     hipLaunchKernelGGL(k_post<K.value>, dim3(nblk(G.N, bt)), dim3(bt), 0, st, G, A);
   });

@@ -44,6 +44,7 @@ struct PostArgs {
   unsigned long long *cnt, *cpart;
   double gam, dmin, pmin, pmax;
   int model;
+  int nbv, nbc;                    // ghost fill: variables per thread, workgroups of those (set by launch_post)
 };
 
 struct CflArgs {
