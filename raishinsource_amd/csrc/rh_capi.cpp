@@ -378,8 +378,7 @@ void raishin_model_debug_stage(raishin_model* m, int stage, double* ww, double* 
   tap.wpre = wpre;
   auto go = [&]() -> bool {
     if (stage == 1) {
-      if (!run_cfl(m, m->W)) return false;
-      HIPCHK(launch_advance_time(m->G, m->dtbits, m->p.cfl, m->tdt, m->st));
+      if (!run_cfl(m, m->W, true)) return false;
       if (m->need_wo) HIPCHK(launch_copy(m->G, m->Wo, m->W, 9 * m->G.N, m->st));
       return run_stage(m, 1, m->Ucur, nullptr, m->Uh, &tap);
     }

@@ -1598,9 +1598,12 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, unsigned blk) {
 // and MIN(a,b) = a<b?a:b: a NaN element sets the running value to NaN and
 // the next element replaces it.  So the result is the minimum over the
 // elements after the last NaN (NaN if a NaN is the last element; 1.0 and all
-// elements if there is none).  Each block reduces its contiguous range to
-// (position of its last NaN, minimum after it) with wavefront shuffles; one
-// block then combines the block results in order.
+// elements if there is none).  Each workgroup reduces its contiguous range of
+// A.per cells, 256 at a time, to (position of its last NaN, minimum after it)
+// with wavefront shuffles; one workgroup then combines their results in order
+// and, in a step, advances the time (main.f90:760-781).  (The last workgroup
+// to finish doing that in the same launch measured slower: its device-scope
+// fence writes the L2 back in every workgroup, 256x128x128 0.135 -> 0.21 ms.)
 // Accumulators: 0 dtcfl (three elements per cell: dtx1a, dtx2a, dtx3a),
 // 1..3 dtx1..dtx3 (one element per cell).
 // ------------------------------------------------------------------------
@@ -1612,170 +1615,158 @@ RH_DEV double wave_min(double v) {
   }
   return v;
 }
-template <class T>
-RH_DEV T wave_max(T v) {
+RH_DEV int wave_max(int v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
-    const T o = __shfl_xor(v, off, 64);
+    const int o = __shfl_xor(v, off, 64);
     v = o > v ? o : v;
   }
   return v;
 }
 
+// The four accumulators' values over a 256-thread workgroup (maximum of v,
+// or minimum of m), every thread the same.
+RH_DEV void group_max4(int v[4]) {
+  __shared__ int part[4][4];
+  const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    const int w = wave_max(v[a]);
+    if (lane == 0) part[wid][a] = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    v[a] = part[0][a];
+    for (int w = 1; w < 4; w++) v[a] = part[w][a] > v[a] ? part[w][a] : v[a];
+  }
+}
+RH_DEV void group_min4(double m[4]) {
+  __shared__ double part[4][4];
+  const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    const double w = wave_min(m[a]);
+    if (lane == 0) part[wid][a] = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; a++) {
+    m[a] = part[0][a];
+    for (int w = 1; w < 4; w++) m[a] = (part[w][a] < m[a]) ? part[w][a] : m[a];
+  }
+}
+
+// Signal times of the cell at box position t (dtx1a, dtx2a, dtx3a); infinite
+// past the box.
+template <int ICHA, bool MK>
+RH_DEV bool cfl_cell(const Geo& G, const CflArgs& A, unsigned t, double e[3]) {
+  int i, j, k;
+  e[0] = e[1] = e[2] = __builtin_inf();
+  if (!box_index(t, 2, G.ni - 1, jlo(G, 2), jhi(G, G.nj - 1), 2, G.nk - 1, i, j, k)) return false;
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
+  const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
+  double w[9];
+#pragma unroll
+  for (int n = 0; n < 9; n++) w[n] = ld_(A.W + (long long)n * N, c * 8u);
+  Prel s;
+  prelude(w, A.gam, M, s);
+  double vp[4], vm[4];
+  centre_speeds<ICHA>(s, A.gam, M, vp, vm);
+  const int nmax = G.nm1 * 2 + (G.nm1 - 1);
+  const int nd[4] = {0, G.ni, G.nj, G.nk};
+  const double dxv[4] = {0.0, A.dx1b[i - 1], A.dx2b[j - 1], A.dx3b[k - 1]};
+#pragma unroll
+  for (int q = 1; q <= 3; q++) {
+    double vf = fmaxf_(fmaxf_(0.0, fabs(vp[q])), fabs(vm[q]));
+    if (nd[q] > nmax && vf > 0.0) {
+      if (vf > 1.0) vf = 1.0;
+      e[q - 1] = fabs(dxv[q] / (vf + 1.0e-12));
+    } else {
+      e[q - 1] = 1.0e10;
+    }
+  }
+  return true;
+}
+
 template <int ICHA, bool MK>
 RH_DEV void b_cfl(const Geo& G, const CflArgs& A, unsigned blk) {
-  __shared__ int s_last[4][4];
-  __shared__ double s_min[4][4];
-  // positions of the elements in the reference's order: below 3 * 2^29
-  const int t = (int)(blk * blockDim.x + threadIdx.x);
-  int i, j, k;
-  double e[4] = {__builtin_inf(), __builtin_inf(), __builtin_inf(), 0.0};  // dtx1a, dtx2a, dtx3a
-  bool valid = box_index((unsigned)t, 2, G.ni - 1, jlo(G, 2), jhi(G, G.nj - 1), 2, G.nk - 1, i, j, k);
-  if (valid) {
-    const long long N = G.N;
-  const unsigned c = cidx(i, j, k, G);
-    const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
-    double w[9];
-#pragma unroll
-    for (int n = 0; n < 9; n++) w[n] = ld_(A.W + (long long)n * N, c * 8u);
-    Prel s;
-    prelude(w, A.gam, M, s);
-    double vp[4], vm[4];
-    centre_speeds<ICHA>(s, A.gam, M, vp, vm);
-    const int nmax = G.nm1 * 2 + (G.nm1 - 1);
-    const int nd[4] = {0, G.ni, G.nj, G.nk};
-    const double dxv[4] = {0.0, A.dx1b[i - 1], A.dx2b[j - 1], A.dx3b[k - 1]};
-#pragma unroll
-    for (int q = 1; q <= 3; q++) {
-      double vf = fmaxf_(fmaxf_(0.0, fabs(vp[q])), fabs(vm[q]));
-      if (nd[q] > nmax && vf > 0.0) {
-        if (vf > 1.0) vf = 1.0;
-        e[q - 1] = fabs(dxv[q] / (vf + 1.0e-12));
-      } else {
-        e[q - 1] = 1.0e10;
-      }
-    }
-  }
-  // per accumulator: this thread's last NaN position and minimum after it
-  int last[4];
+  // the workgroup's last NaN per accumulator (positions below 3 * 2^29) and
+  // the minimum after it; without a NaN among the cells, a plain minimum
+  int L[4] = {-1, -1, -1, -1};
   double mn[4];
-  {
-    int l0 = -1;
-    double m0 = __builtin_inf();
-    if (valid)
+#pragma unroll
+  for (int a = 0; a < 4; a++) mn[a] = __builtin_inf();
+  const unsigned t0 = blk * (unsigned)A.per;
+  for (unsigned b = 0; b < (unsigned)A.per; b += 256) {
+    const int t = (int)(t0 + b + threadIdx.x);
+    double e[3];
+    const bool valid = cfl_cell<ICHA, MK>(G, A, (unsigned)t, e);
+    if (__syncthreads_or(valid && (isnan(e[0]) || isnan(e[1]) || isnan(e[2])))) {
+      // minima so far count only where this chunk has no NaN of the accumulator
+      int last[4] = {-1, -1, -1, -1};
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        if (valid && isnan(e[q])) { last[0] = 3 * t + q; last[q + 1] = t; }
+      group_max4(last);
+#pragma unroll
+      for (int a = 0; a < 4; a++)
+        if (last[a] >= 0) { L[a] = last[a]; mn[a] = __builtin_inf(); }
 #pragma unroll
       for (int q = 0; q < 3; q++) {
-        if (isnan(e[q])) { l0 = 3 * t + q; m0 = __builtin_inf(); }
-        else m0 = (e[q] < m0) ? e[q] : m0;
+        if (!valid || isnan(e[q])) continue;
+        if (3 * t + q > last[0]) mn[0] = (e[q] < mn[0]) ? e[q] : mn[0];
+        if (t > last[q + 1]) mn[q + 1] = (e[q] < mn[q + 1]) ? e[q] : mn[q + 1];
       }
-    last[0] = l0; mn[0] = m0;
+    } else {
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-      const bool nan = valid && isnan(e[q]);
-      last[q + 1] = nan ? t : -1;
-      mn[q + 1] = (valid && !nan) ? e[q] : __builtin_inf();
-    }
-  }
-  const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
-  int L[4];
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const int v = wave_max(last[a]);
-    if (lane == 0) s_last[wid][a] = v;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    int v = s_last[0][a];
-    for (int w = 1; w < (int)(blockDim.x / 64); w++) v = s_last[w][a] > v ? s_last[w][a] : v;
-    L[a] = v;
-  }
-  // contribute the minimum over own elements after the block's last NaN
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    double m = __builtin_inf();
-    if (valid) {
-      if (a == 0) {
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-          if (3 * t + q > L[0] && !isnan(e[q])) m = (e[q] < m) ? e[q] : m;
-      } else if (t > L[a] && !isnan(e[a - 1])) {
-        m = e[a - 1];
+      for (int q = 0; q < 3; q++) {
+        mn[0] = (e[q] < mn[0]) ? e[q] : mn[0];
+        mn[q + 1] = (e[q] < mn[q + 1]) ? e[q] : mn[q + 1];
       }
     }
-    const double v = wave_min(m);
-    if (lane == 0) s_min[wid][a] = v;
   }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    const int a = threadIdx.x;
-    double v = s_min[0][a];
-    for (int w = 1; w < (int)(blockDim.x / 64); w++) v = (s_min[w][a] < v) ? s_min[w][a] : v;
-    A.blast[4 * blk + a] = L[a];
-    A.bmin[4 * blk + a] = v;
-  }
-}
-
-// Combine the per-block results in block order (one workgroup): the last NaN
-// lies in the last block that has one; that block's minimum after it and the
-// full minima of every later block make the result.
-RH_DEV void b_cfl_finish(const CflArgs& A) {
-  // the four accumulators together: two passes over the per-block results
-  // (last NaN, then the minimum after it); max and min do not depend on the
-  // order, so the result is the sequential fold's
-  const int nblocks = A.nblocks;
-  __shared__ long long s_l[16][4];
-  __shared__ double s_m[16][4];
-  __shared__ long long s_B[4];
-  const int lane = threadIdx.x % 64, wid = threadIdx.x / 64, nw = blockDim.x / 64;
-  long long bg[4] = {-1, -1, -1, -1};
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-      if (A.blast[4 * b + a] >= 0) bg[a] = b > bg[a] ? b : bg[a];
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const long long v = wave_max(bg[a]);
-    if (lane == 0) s_l[wid][a] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    long long B = s_l[0][threadIdx.x];
-    for (int w = 1; w < nw; w++) B = s_l[w][threadIdx.x] > B ? s_l[w][threadIdx.x] : B;
-    s_B[threadIdx.x] = B;
-  }
-  __syncthreads();
-  long long B[4];
-  double m[4];
-#pragma unroll
-  for (int a = 0; a < 4; a++) { B[a] = s_B[a]; m[a] = __builtin_inf(); }
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-      if (b >= B[a]) { const double v = A.bmin[4 * b + a]; m[a] = (v < m[a]) ? v : m[a]; }
-#pragma unroll
-  for (int a = 0; a < 4; a++) {
-    const double v = wave_min(m[a]);
-    if (lane == 0) s_m[wid][a] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    const int a = threadIdx.x;
-    double M = s_m[0][a];
-    for (int w = 1; w < nw; w++) M = (s_m[w][a] < M) ? s_m[w][a] : M;
-    double r;
-    if (B[a] < 0) r = fminf_(1.0, M);                              // no NaN: MIN over 1.0 and all
-    else r = (M == __builtin_inf()) ? __builtin_nan("") : M;  // a trailing NaN stays
-    A.dtbits[a] = (unsigned long long)__double_as_longlong(r);
-  }
-}
-
-// time <- time + cfl*dtcfl ; last dt kept (main.f90:760-781)
-RH_DEV void b_advance_time(const AdvArgs& A) {
+  group_min4(mn);
   if (threadIdx.x == 0) {
-    const double dt = A.cfl * __longlong_as_double((long long)A.dtbits[0]);
-    A.tdt[0] = A.tdt[0] + dt;
-    A.tdt[1] = dt;
+#pragma unroll
+    for (int a = 0; a < 4; a++) { A.blast[4 * blk + a] = L[a]; A.bmin[4 * blk + a] = mn[a]; }
+  }
+}
+
+// One workgroup of 256 combines the results of A.nblocks workgroups.
+RH_DEV void b_cfl_finish(const CflArgs& A) {
+  double mn[4];
+  // the last NaN lies in the last workgroup that has one; that workgroup's
+  // minimum after it and the full minima of every later one make the result
+  int B[4] = {-1, -1, -1, -1};
+  for (int q = threadIdx.x; q < A.nblocks; q += 256)
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+      if (A.blast[4 * q + a] >= 0) B[a] = q;
+  group_max4(B);
+#pragma unroll
+  for (int a = 0; a < 4; a++) mn[a] = __builtin_inf();
+  for (int q = threadIdx.x; q < A.nblocks; q += 256)
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+      if (q >= B[a]) { const double v = A.bmin[4 * q + a]; mn[a] = (v < mn[a]) ? v : mn[a]; }
+  group_min4(mn);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      double r;
+      if (B[a] < 0) r = fminf_(1.0, mn[a]);                               // no NaN: MIN over 1.0 and all
+      else r = (mn[a] == __builtin_inf()) ? __builtin_nan("") : mn[a];  // a trailing NaN stays
+      A.dtbits[a] = (unsigned long long)__double_as_longlong(r);
+      if (a == 0 && A.tdt) {  // time <- time + cfl*dtcfl; last dt kept
+        const double dt = A.cfl * r;
+        A.tdt[0] = A.tdt[0] + dt;
+        A.tdt[1] = dt;
+      }
+    }
   }
 }
 
@@ -2097,8 +2088,7 @@ template <bool MK>
 __global__ void __launch_bounds__(256) k_post(Geo G, PostArgs A) { b_post<MK>(G, A, xcd_block()); }
 template <int ICHA, bool MK>
 __global__ void __launch_bounds__(256) k_cfl(Geo G, CflArgs A) { b_cfl<ICHA, MK>(G, A, blockIdx.x); }
-__global__ void __launch_bounds__(1024) k_cfl_finish(CflArgs A) { b_cfl_finish(A); }
-__global__ void __launch_bounds__(64) k_advance_time(AdvArgs A) { b_advance_time(A); }
+__global__ void __launch_bounds__(256) k_cfl_finish(CflArgs A) { b_cfl_finish(A); }
 
 // batched twins: BODY(G, A, blk) for the model that owns workgroup blockIdx.x
 #define RH_BATCH_PROLOGUE                                  \
@@ -2181,15 +2171,11 @@ __global__ void __launch_bounds__(1024) kb_recov_carry(const BatchItem* __restri
   const FixArgs A = it[blockIdx.x].A.fx;
   b_recov_carry<IW, MK>(G, A, 0, 1);
 }
-__global__ void __launch_bounds__(1024) kb_cfl_finish(const BatchItem* __restrict__ it, int n) {
+
+__global__ void __launch_bounds__(256) kb_cfl_finish(const BatchItem* __restrict__ it, int n) {
   if ((int)blockIdx.x >= n) return;
   const CflArgs A = it[blockIdx.x].A.cf;
   b_cfl_finish(A);
-}
-__global__ void __launch_bounds__(64) kb_advance_time(const BatchItem* __restrict__ it, int n) {
-  if ((int)blockIdx.x >= n) return;
-  const AdvArgs A = it[blockIdx.x].A.a;
-  b_advance_time(A);
 }
 
 // ------------------------------------------------------------------------
@@ -2214,13 +2200,12 @@ static void record(int kind, int variant, int threads, long long nb, const Geo& 
 
 int block_threads(int kind) {
   switch (kind) {
-    case LK_CARRY: case LK_CFL_FINISH: return 1024;
-    case LK_ADVANCE: return 64;
+    case LK_CARRY: return 1024;
     default: return 256;
   }
 }
 
-bool one_group_per_model(int kind) { return kind == LK_CARRY || kind == LK_CFL_FINISH || kind == LK_ADVANCE; }
+bool one_group_per_model(int kind) { return kind == LK_CARRY || kind == LK_CFL_FINISH; }
 
 hipError_t launch_edges(const Geo& G, int dir, int irec, const double* W, const double* dxs, const double* xs,
                         const double* tab, double gam, void* E, bool mixed, hipStream_t st) {
@@ -2535,34 +2520,34 @@ hipError_t launch_sum_counters(unsigned long long* cpart, long long rows, unsign
   return hipGetLastError();
 }
 
+static long long cfl_cells(const Geo& G) {
+  return box(2, G.ni - 1) * jbox(G, 2, G.nj - 1) * box(2, G.nk - 1);
+}
+
 long long cfl_blocks(const Geo& G) {
-  const long long n = box(2, G.ni - 1) * jbox(G, 2, G.nj - 1) * box(2, G.nk - 1);
+  const long long n = cfl_cells(G);
   return n > 0 ? (long long)nblk(n, 256) : 1;
 }
 
 hipError_t launch_cfl(const Geo& G, const CflArgs& A0, hipStream_t st) {
   CflArgs A = A0;
-  const unsigned nb = (unsigned)cfl_blocks(G);
+  // 256 cells per workgroup, or more so that there are CFL_GROUPS at most,
+  // whose results one workgroup reads
+  const long long chunks = cfl_blocks(G), each = (chunks + CFL_GROUPS - 1) / CFL_GROUPS;
+  const unsigned nb = (unsigned)((chunks + each - 1) / each);
   A.nblocks = (int)nb;
+  A.per = (int)(256 * each);
   if (g_rec) {
     AnyArgs a{};
     a.cf = A;
     record(LK_CFL, G.icha + 4 * G.mk, 256, nb, G, a);
-    record(LK_CFL_FINISH, 0, 1024, 1, G, a);
+    record(LK_CFL_FINISH, 0, 256, 1, G, a);
     return hipSuccess;
   }
   with_icha(G.icha, G.mk, [&](auto C, auto K) {
     hipLaunchKernelGGL((k_cfl<C.value, K.value>), dim3(nb), dim3(256), 0, st, G, A);
   });
-  hipLaunchKernelGGL(k_cfl_finish, dim3(1), dim3(1024), 0, st, A);
-  return hipGetLastError();
-}
-
-hipError_t launch_advance_time(const Geo& G, const unsigned long long* dtbits, double cfl, double* tdt,
-                               hipStream_t st) {
-  AdvArgs A{dtbits, cfl, tdt};
-  if (g_rec) { AnyArgs a{}; a.a = A; record(LK_ADVANCE, 0, 64, 1, G, a); return hipSuccess; }
-  hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(64), 0, st, A);
+  hipLaunchKernelGGL(k_cfl_finish, dim3(1), dim3(256), 0, st, A);
   return hipGetLastError();
 }
 
@@ -2628,13 +2613,12 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       });
       break;
     case LK_COPY: hipLaunchKernelGGL(kb_copy, g, b, 0, st, it, n); break;
+    case LK_CFL_FINISH: hipLaunchKernelGGL(kb_cfl_finish, dim3(n), dim3(256), 0, st, it, n); break;
     case LK_CARRY:
       with_recov(variant, [&](auto I, auto K) {
         hipLaunchKernelGGL((kb_recov_carry<I.value, K.value>), dim3(n), dim3(1024), 0, st, it, n);
       });
       break;
-    case LK_CFL_FINISH: hipLaunchKernelGGL(kb_cfl_finish, dim3(n), dim3(1024), 0, st, it, n); break;
-    case LK_ADVANCE: hipLaunchKernelGGL(kb_advance_time, dim3(n), dim3(64), 0, st, it, n); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

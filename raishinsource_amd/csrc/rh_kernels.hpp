@@ -54,8 +54,9 @@ struct CflArgs {
   unsigned long long *dtbits;      // [0] dtcfl [1..3] dt1..dt3 (bit patterns of the doubles)
   long long *blast;                // per block and accumulator: position of the last NaN
   double *bmin;                    // per block and accumulator: minimum after it
-  double gam;
-  int nblocks;                     // workgroups of the k_cfl launch (set by launch_cfl)
+  double *tdt;                     // time and last dt to advance by cfl*dtcfl, or null
+  double gam, cfl;
+  int nblocks, per;                // workgroups of the launch, cells of each (set by launch_cfl)
 };
 
 struct FixArgs {
@@ -102,12 +103,6 @@ struct CtArgs {
   double *CTd;        // mixed form: the six averages also in FP64 (StageArgs::CTd)
 };
 
-struct AdvArgs {
-  const unsigned long long *dtbits;
-  double cfl;
-  double *tdt;
-};
-
 struct CopyArgs {
   const double *src;
   double *dst;
@@ -125,7 +120,7 @@ inline int slot_threads(const Geo& G, int slot) { return G.bs[slot] ? (int)G.bs[
 // Launch kinds of one step, in the order run_step makes them.
 enum LaunchKind {
   LK_EDGES, LK_SWEEP, LK_FLUXCT, LK_RK, LK_RECOV, LK_CARRY, LK_BND, LK_POST, LK_CFL, LK_CFL_FINISH,
-  LK_ADVANCE, LK_COPY, LK_PSWEEP, LK_N
+  LK_COPY, LK_PSWEEP, LK_N
 };
 
 union AnyArgs {
@@ -137,7 +132,6 @@ union AnyArgs {
   FixArgs fx;
   PostArgs p;
   CflArgs cf;
-  AdvArgs a;
   CopyArgs cp;
 };
 
@@ -206,11 +200,10 @@ hipError_t launch_recov(const Geo& G, const StageArgs& A, hipStream_t st);
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st);
 hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st);
 hipError_t launch_cfl(const Geo& G, const CflArgs& A, hipStream_t st);
-long long cfl_blocks(const Geo& G);
+long long cfl_blocks(const Geo& G);  // 256-cell chunks of the CFL reduction
+constexpr int CFL_GROUPS = 1024;     // its workgroups at most
 // Fold the per-wavefront event rows into cnt (and clear them).
 hipError_t launch_sum_counters(unsigned long long* cpart, long long rows, unsigned long long* cnt, hipStream_t st);
-hipError_t launch_advance_time(const Geo& G, const unsigned long long* dtbits, double cfl, double* tdt,
-                               hipStream_t st);
 // dst <- src (n doubles), stream-ordered
 // The metric and Christoffel (i,k) tables of an axisymmetric metric from the
 // grid, on the device (k_metric_tables); tr: per k the host's sin/cos at

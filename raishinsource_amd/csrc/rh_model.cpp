@@ -580,16 +580,17 @@ bool copy_fluxes_out(raishin_model* m, double* ww, double* ct) {
   return !ct || copy_planes_out(m, m->CT, 6, 1, 0, ct, m->mixed);
 }
 
-bool run_cfl(raishin_model* m, const double* W) {
+bool run_cfl(raishin_model* m, const double* W, bool advance) {
   CflArgs C{};
   C.W = W; C.metC = m->metric_centre(); C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
   C.dtbits = m->dtbits; C.blast = m->cfl_last; C.bmin = m->cfl_min; C.gam = m->p.gam;
+  C.cfl = m->p.cfl; C.tdt = advance ? m->tdt : nullptr;
   { TimedLaunch t(m, K_CFL); HIPCHK(launch_cfl(m->G, C, m->st)); }
   return true;
 }
 
 bool cdtcfl4_on(raishin_model* m, const double* W, double* dtcfl, double* dt1, double* dt2, double* dt3) {
-  if (!run_cfl(m, W)) return false;
+  if (!run_cfl(m, W, false)) return false;
   unsigned long long b[4];
   HIPCHK(hipMemcpyAsync(b, m->dtbits, 32, hipMemcpyDeviceToHost, m->st));
   HIPCHK(hipStreamSynchronize(m->st));
@@ -604,8 +605,7 @@ bool cdtcfl4_on(raishin_model* m, const double* W, double* dtcfl, double* dt1, d
 
 bool run_step(raishin_model* m) {
   const long long N = m->G.N;
-  if (!run_cfl(m, m->W)) return false;
-  HIPCHK(launch_advance_time(m->G, m->dtbits, m->p.cfl, m->tdt, m->st));
+  if (!run_cfl(m, m->W, true)) return false;
   if (m->need_wo) HIPCHK(launch_copy(m->G, m->Wo, m->W, 9 * N, m->st));
   if (!run_stage(m, 1, m->Ucur, nullptr, m->Uh)) return false;
   if (m->p.irkt == 2) {

@@ -138,7 +138,8 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
                   const double* F, const HostDt* hd);
 // Ghost fill, floors and conserved variables: m->Wpre -> Wout, Uout.
 bool stage_post(raishin_model* m, const double* Wold, const double* Wo, double* Wout, double* Uout);
-bool run_cfl(raishin_model* m, const double* W);
+// The CFL minimum of primitives W; advance: then time += cfl * dtcfl.
+bool run_cfl(raishin_model* m, const double* W, bool advance);
 bool run_stage(raishin_model* m, int rkstage, const double* Ua, const double* Ub, double* Uout,
                const struct StageTap* tap = nullptr);
 bool run_step(raishin_model* m);
