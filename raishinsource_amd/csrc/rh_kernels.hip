@@ -43,11 +43,13 @@ RH_DEV bool box_index(unsigned t, int ilo, int ihi, int jlo, int jhi, int klo, i
 
 // Workgroup b is dispatched to XCD b % 8.  Renumbering the workgroups so that
 // each XCD takes one contiguous eighth of the launch keeps neighbouring rows
-// of a stencil in the same L2.  A bijection on [0, gridDim.x).
-RH_DEV unsigned xcd_block() {
-  const unsigned nb = gridDim.x, b = blockIdx.x, x = b % 8u, idx = b / 8u, q = nb / 8u, r = nb % 8u;
+// of a stencil in the same L2.  A bijection on [0, nb), for a launch or a part
+// of one that starts at a multiple of 8.
+RH_DEV unsigned xcd_renumber(unsigned nb, unsigned b) {
+  const unsigned x = b % 8u, idx = b / 8u, q = nb / 8u, r = nb % 8u;
   return x < r ? x * (q + 1) + idx : r * (q + 1) + (x - r) * q + idx;
 }
+RH_DEV unsigned xcd_block() { return xcd_renumber(gridDim.x, blockIdx.x); }
 
 // As box_index with the j and k axes swapped in the ordering (i fastest, then
 // k, then j): consecutive workgroups step along k, the k sweep's stencil axis.
@@ -692,8 +694,14 @@ RH_DEV void b_psweep(const Geo& G, const PSweepArgs& A, unsigned blk) {
 // the flux array in place, like ct.f90:98-109.  FT: the stored type (float
 // in the mixed form); the averages are formed in double.
 // ------------------------------------------------------------------------
+RH_DEV void b_cfl_finish(const CflArgs& A);
+
 template <class FT>
 RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, unsigned blk) {
+  if (A.fin >= 0 && blk == (unsigned)A.fin) {  // the workgroup that combines the CFL reduction
+    b_cfl_finish(A.cfl);
+    return;
+  }
   const FT* __restrict__ CTsrc = (const FT*)A.CTsrc;
   FT* __restrict__ F1 = (FT*)A.F1;
   FT* __restrict__ F2 = (FT*)A.F2;
@@ -1599,7 +1607,7 @@ RH_DEV void b_post(const Geo& G, const PostArgs& A, unsigned blk) {
 // the next element replaces it.  So the result is the minimum over the
 // elements after the last NaN (NaN if a NaN is the last element; 1.0 and all
 // elements if there is none).  Each workgroup reduces its contiguous range of
-// A.per cells, 256 at a time, to (position of its last NaN, minimum after it)
+// A.per cells, a thread each at a time, to (position of its last NaN, minimum after it)
 // with wavefront shuffles; one workgroup then combines their results in order
 // and, in a step, advances the time (main.f90:760-781).  (The last workgroup
 // to finish doing that in the same launch measured slower: its device-scope
@@ -1624,8 +1632,8 @@ RH_DEV int wave_max(int v) {
   return v;
 }
 
-// The four accumulators' values over a 256-thread workgroup (maximum of v,
-// or minimum of m), every thread the same.
+// The four accumulators' values over a workgroup of at most 256 (maximum of
+// v, or minimum of m), every thread the same.
 RH_DEV void group_max4(int v[4]) {
   __shared__ int part[4][4];
   const int lane = threadIdx.x % 64, wid = threadIdx.x / 64;
@@ -1639,7 +1647,7 @@ RH_DEV void group_max4(int v[4]) {
 #pragma unroll
   for (int a = 0; a < 4; a++) {
     v[a] = part[0][a];
-    for (int w = 1; w < 4; w++) v[a] = part[w][a] > v[a] ? part[w][a] : v[a];
+    for (int w = 1; w < (int)(blockDim.x / 64); w++) v[a] = part[w][a] > v[a] ? part[w][a] : v[a];
   }
 }
 RH_DEV void group_min4(double m[4]) {
@@ -1655,7 +1663,7 @@ RH_DEV void group_min4(double m[4]) {
 #pragma unroll
   for (int a = 0; a < 4; a++) {
     m[a] = part[0][a];
-    for (int w = 1; w < 4; w++) m[a] = (part[w][a] < m[a]) ? part[w][a] : m[a];
+    for (int w = 1; w < (int)(blockDim.x / 64); w++) m[a] = (part[w][a] < m[a]) ? part[w][a] : m[a];
   }
 }
 
@@ -1701,7 +1709,7 @@ RH_DEV void b_cfl(const Geo& G, const CflArgs& A, unsigned blk) {
 #pragma unroll
   for (int a = 0; a < 4; a++) mn[a] = __builtin_inf();
   const unsigned t0 = blk * (unsigned)A.per;
-  for (unsigned b = 0; b < (unsigned)A.per; b += 256) {
+  for (unsigned b = 0; b < (unsigned)A.per; b += blockDim.x) {
     const int t = (int)(t0 + b + threadIdx.x);
     double e[3];
     const bool valid = cfl_cell<ICHA, MK>(G, A, (unsigned)t, e);
@@ -1736,20 +1744,20 @@ RH_DEV void b_cfl(const Geo& G, const CflArgs& A, unsigned blk) {
   }
 }
 
-// One workgroup of 256 combines the results of A.nblocks workgroups.
+// One workgroup combines the results of A.nblocks workgroups.
 RH_DEV void b_cfl_finish(const CflArgs& A) {
   double mn[4];
   // the last NaN lies in the last workgroup that has one; that workgroup's
   // minimum after it and the full minima of every later one make the result
   int B[4] = {-1, -1, -1, -1};
-  for (int q = threadIdx.x; q < A.nblocks; q += 256)
+  for (int q = threadIdx.x; q < A.nblocks; q += blockDim.x)
 #pragma unroll
     for (int a = 0; a < 4; a++)
       if (A.blast[4 * q + a] >= 0) B[a] = q;
   group_max4(B);
 #pragma unroll
   for (int a = 0; a < 4; a++) mn[a] = __builtin_inf();
-  for (int q = threadIdx.x; q < A.nblocks; q += 256)
+  for (int q = threadIdx.x; q < A.nblocks; q += blockDim.x)
 #pragma unroll
     for (int a = 0; a < 4; a++)
       if (q >= B[a]) { const double v = A.bmin[4 * q + a]; mn[a] = (v < mn[a]) ? v : mn[a]; }
@@ -2073,6 +2081,31 @@ k_sweep(Geo G, SweepArgs A) { b_sweep<D, IREC, R, ICHA, MK>(G, A, xcd_block()); 
 template <int D, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
 k_psweep(Geo G, PSweepArgs A) { b_psweep<D, R, ICHA, MK>(G, A, xcd_block()); }
+// The three sweeps of a stage, and in a step's first stage the CFL reduction
+// of the same primitives, in one launch: none reads what another writes.
+// COLL: a collapsed model's j sweep.
+// Each part starts at a multiple of 8 workgroups (a batch member's does too)
+// and is renumbered per XCD by itself.  Against a launch each (and three of
+// the CFL reduction's): 64x64 and 128x128 torus 116 -> 78 and 125 -> 84 us a
+// step, 64^3 443 -> 371, 96x64x64 593 -> 521, 256x128x128 5880 -> 5800 us;
+// without the renumbering 6010 us.
+template <class R, int ICHA, bool MK, bool COLL>
+RH_DEV void b_psweep3(const Geo& G, const PSweep3Args& A, unsigned blk) {
+  auto part = [&](int d, unsigned& b) {
+    b = blk - (d ? A.end[d - 1] : 0u);
+    if (b >= A.n[d]) return false;  // the filling up to a multiple of 8
+    b = xcd_renumber(A.n[d], b);
+    return true;
+  };
+  unsigned b;
+  if (blk < A.end[0]) { if (part(0, b)) b_psweep<1, R, ICHA, MK>(G, A.s[0], b); }
+  else if (blk < A.end[1]) { if (part(1, b)) b_psweep<COLL ? 0 : 2, R, ICHA, MK>(G, A.s[1], b); }
+  else if (blk < A.end[2]) { if (part(2, b)) b_psweep<3, R, ICHA, MK>(G, A.s[2], b); }
+  else if (blk - A.end[2] < (unsigned)A.cfl.nblocks) b_cfl<ICHA, MK>(G, A.cfl, blk - A.end[2]);
+}
+template <class R, int ICHA, bool MK, bool COLL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
+k_psweep3(Geo G, PSweep3Args A) { b_psweep3<R, ICHA, MK, COLL>(G, A, blockIdx.x); }
 template <class FT>
 __global__ void __launch_bounds__(256) k_fluxct(Geo G, CtArgs A) { b_fluxct<FT>(G, A, xcd_block()); }
 template <int STAGE, bool SYM, class FT, bool MK>
@@ -2120,6 +2153,13 @@ kb_psweep(const BatchItem* __restrict__ it, int n) {
   RH_BATCH_PROLOGUE
   const PSweepArgs A = it[q].A.ps;
   b_psweep<D, R, ICHA, MK>(G, A, blk);
+}
+template <class R, int ICHA, bool MK, bool COLL>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
+kb_psweep3(const BatchItem* __restrict__ it, int n) {
+  RH_BATCH_PROLOGUE
+  const PSweep3Args A = it[q].A.ps3;
+  b_psweep3<R, ICHA, MK, COLL>(G, A, blk);
 }
 template <class FT>
 __global__ void __launch_bounds__(256) kb_fluxct(const BatchItem* __restrict__ it, int n) {
@@ -2405,28 +2445,48 @@ int psweep_segment(const Geo& G, int dir) {
 
 size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads * (mixed ? sizeof(float) : sizeof(double)); }
 
-hipError_t launch_psweep(const Geo& G, int dir, const double* W, const void* metF, const double* dxs,
-                         const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,
-                         hipStream_t st) {
-  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
+static long long cfl_cells(const Geo& G) {
+  return box(2, G.ni - 1) * jbox(G, 2, G.nj - 1) * box(2, G.nk - 1);
+}
+
+long long cfl_blocks(const Geo& G) {
+  const long long n = cfl_cells(G);
+  return n > 0 ? (long long)nblk(n, 256) : 1;
+}
+
+long long cfl_slots(const Geo& G) { return std::min<long long>(CFL_GROUPS, std::max(1LL, (cfl_cells(G) + 63) / 64)); }
+
+// Workgroups of bt threads of the CFL reduction (set in A with their cells):
+// bt cells each, or more so that there are CFL_GROUPS at most, whose results
+// one workgroup reads.
+static unsigned cfl_groups(const Geo& G, int bt, CflArgs& A) {
+  const long long chunks = std::max(1LL, (cfl_cells(G) + bt - 1) / bt), each = (chunks + CFL_GROUPS - 1) / CFL_GROUPS;
+  A.nblocks = (int)((chunks + each - 1) / each);
+  A.per = (int)(bt * each);
+  return (unsigned)A.nblocks;
+}
+
+// Arguments and workgroups (of bt threads) of one fused sweep.
+static long long psweep_args(const Geo& G, int dir, int bt, PSweepArgs& A) {
   long long along, lines, across;
   psweep_extent(G, dir, along, lines, across);
-  const bool self = dir == 2 && G.jfix;  // one stored phi row: its own neighbour
-  PSweepArgs A{W, metF, dxs, xs, pc, gam, F, CTsrc, 0, 0, 0, 0};
-  long long n = 0;  // workgroups
-  if (self) {
-    n = (lines * across + bt - 1) / bt;
-  } else if (along > 0 && lines > 0 && across > 0) {
-    A.tp = psweep_tp(G, dir, bt);
-    const int ti = bt / A.tp;
-    // log2 of the lanes that vary fastest (D = 1 with the whole workgroup on one row: all)
-    const int fast = dir == 1 ? A.tp : ti;
-    A.sh = dir == 1 && ti == 1 ? 30 : __builtin_ctz((unsigned)fast);
-    A.nig = (int)((lines + ti - 1) / ti);
-    A.ndc = (int)((along + A.tp - 4) / (A.tp - 3));
-    n = (long long)A.nig * A.ndc * across;
-  }
-  const unsigned nb = (unsigned)n;
+  if (dir == 2 && G.jfix) return (lines * across + bt - 1) / bt;  // one stored phi row: its own neighbour
+  if (along <= 0 || lines <= 0 || across <= 0) return 0;
+  A.tp = psweep_tp(G, dir, bt);
+  const int ti = bt / A.tp;
+  // log2 of the lanes that vary fastest (D = 1 with the whole workgroup on one row: all)
+  const int fast = dir == 1 ? A.tp : ti;
+  A.sh = dir == 1 && ti == 1 ? 30 : __builtin_ctz((unsigned)fast);
+  A.nig = (int)((lines + ti - 1) / ti);
+  A.ndc = (int)((along + A.tp - 4) / (A.tp - 3));
+  return (long long)A.nig * A.ndc * across;
+}
+
+hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A0, bool mixed, hipStream_t st) {
+  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
+  const bool self = dir == 2 && G.jfix;
+  PSweepArgs A = A0;
+  const unsigned nb = (unsigned)psweep_args(G, dir, bt, A);
   const int variant = psweep_variant(self ? 0 : dir, mixed, G);
   if (g_rec) {
     AnyArgs a{};
@@ -2434,23 +2494,70 @@ hipError_t launch_psweep(const Geo& G, int dir, const double* W, const void* met
     record(LK_PSWEEP, variant, bt, nb, G, a);
     return hipSuccess;
   }
-  if (n == 0) return hipSuccess;
+  if (nb == 0) return hipSuccess;
   const size_t lds = self ? 0 : psweep_lds_bytes(bt, mixed);
   with_psweep(variant, [&](auto D, auto T, auto C, auto K) {
-    hipLaunchKernelGGL((k_psweep<D.value, typename decltype(T)::type, C.value, K.value>), dim3(nb), dim3(bt), lds, st, G, A);
+    hipLaunchKernelGGL((k_psweep<D.value, typename decltype(T)::type, C.value, K.value>), dim3(nb), dim3(bt), lds, st,
+                       G, A);
+  });
+  return hipGetLastError();
+}
+
+// variant: (collapsed) + 4*mixed + 64*icha + 256*compact
+template <class F>
+static void with_psweep3(int variant, F&& f) {
+  with_icha((variant >> 6) & 3, (variant & 256) != 0, [&](auto C, auto K) {
+    with_mk((variant & 1) != 0, [&](auto L) {
+      if (variant & 4) f(TypeTag<float>{}, C, K, L);
+      else f(TypeTag<double>{}, C, K, L);
+    });
+  });
+}
+
+hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st) {
+  const int bt = slot_threads(G, TS_SWEEP1);
+  PSweep3Args A{};
+  unsigned nb = 0;
+  for (int d = 0; d < 3; d++) {
+    A.s[d] = s[d];
+    A.n[d] = (unsigned)psweep_args(G, d + 1, bt, A.s[d]);
+    nb += (A.n[d] + 7u) & ~7u;
+    A.end[d] = nb;
+  }
+  if (cfl) {
+    A.cfl = *cfl;
+    nb += (cfl_groups(G, bt, A.cfl) + 7u) & ~7u;
+  }
+  const int variant = psweep_variant(G.jfix ? 1 : 0, mixed, G);
+  if (g_rec) {
+    AnyArgs a{};
+    a.ps3 = A;
+    record(LK_PSWEEP3, variant, bt, nb, G, a);
+    return hipSuccess;
+  }
+  if (nb == 0) return hipSuccess;
+  with_psweep3(variant, [&](auto T, auto C, auto K, auto L) {
+    hipLaunchKernelGGL((k_psweep3<typename decltype(T)::type, C.value, K.value, L.value>), dim3(nb), dim3(bt),
+                       psweep_lds_bytes(bt, mixed), st, G, A);
   });
   return hipGetLastError();
 }
 
 hipError_t launch_fluxct(const Geo& G, const void* CTsrc, void* F1, void* F2, void* F3, bool f32, double* CTd,
-                         hipStream_t st) {
+                         const CflArgs* cfl, hipStream_t st) {
   const long long n = box(G.nm1, G.ni - G.nm1) * jbox(G, G.nm1, G.nj - G.nm1) * box(G.nm1, G.nk - G.nm1);
-  CtArgs A{CTsrc, F1, F2, F3, f32 ? CTd : nullptr};
+  CtArgs A{CTsrc, F1, F2, F3, f32 ? CTd : nullptr, -1, CflArgs{}};
   const int bt = slot_threads(G, TS_FLUXCT);
-  if (g_rec) { AnyArgs a{}; a.c = A; record(LK_FLUXCT, (int)f32, bt, nblk(n, bt), G, a); return hipSuccess; }
-  if (n == 0) return hipSuccess;
-  if (f32) hipLaunchKernelGGL(k_fluxct<float>, dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
-  else hipLaunchKernelGGL(k_fluxct<double>, dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
+  unsigned nb = nblk(n, bt);
+  if (cfl) {  // one more workgroup combines the CFL reduction of launch_psweep3
+    A.cfl = *cfl;
+    (void)cfl_groups(G, slot_threads(G, TS_SWEEP1), A.cfl);
+    A.fin = (int)nb++;
+  }
+  if (g_rec) { AnyArgs a{}; a.c = A; record(LK_FLUXCT, (int)f32, bt, nb, G, a); return hipSuccess; }
+  if (nb == 0) return hipSuccess;
+  if (f32) hipLaunchKernelGGL(k_fluxct<float>, dim3(nb), dim3(bt), 0, st, G, A);
+  else hipLaunchKernelGGL(k_fluxct<double>, dim3(nb), dim3(bt), 0, st, G, A);
   return hipGetLastError();
 }
 
@@ -2520,23 +2627,9 @@ hipError_t launch_sum_counters(unsigned long long* cpart, long long rows, unsign
   return hipGetLastError();
 }
 
-static long long cfl_cells(const Geo& G) {
-  return box(2, G.ni - 1) * jbox(G, 2, G.nj - 1) * box(2, G.nk - 1);
-}
-
-long long cfl_blocks(const Geo& G) {
-  const long long n = cfl_cells(G);
-  return n > 0 ? (long long)nblk(n, 256) : 1;
-}
-
 hipError_t launch_cfl(const Geo& G, const CflArgs& A0, hipStream_t st) {
   CflArgs A = A0;
-  // 256 cells per workgroup, or more so that there are CFL_GROUPS at most,
-  // whose results one workgroup reads
-  const long long chunks = cfl_blocks(G), each = (chunks + CFL_GROUPS - 1) / CFL_GROUPS;
-  const unsigned nb = (unsigned)((chunks + each - 1) / each);
-  A.nblocks = (int)nb;
-  A.per = (int)(256 * each);
+  const unsigned nb = cfl_groups(G, 256, A);
   if (g_rec) {
     AnyArgs a{};
     a.cf = A;
@@ -2591,6 +2684,12 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       });
       break;
     }
+    case LK_PSWEEP3:
+      with_psweep3(variant, [&](auto T, auto C, auto K, auto L) {
+        hipLaunchKernelGGL((kb_psweep3<typename decltype(T)::type, C.value, K.value, L.value>), g, b,
+                           psweep_lds_bytes(threads, (variant & 4) != 0), st, it, n);
+      });
+      break;
     case LK_FLUXCT:
       if (variant == 1) hipLaunchKernelGGL(kb_fluxct<float>, g, b, 0, st, it, n);
       else hipLaunchKernelGGL(kb_fluxct<double>, g, b, 0, st, it, n);

@@ -97,10 +97,20 @@ struct PSweepArgs {
   int tp, sh, nig, ndc;
 };
 
+// The three sweeps of a stage in one launch, then the CFL reduction: n
+// workgroups of each sweep, the next part from end (a multiple of 8).
+struct PSweep3Args {
+  PSweepArgs s[3];
+  unsigned n[3], end[3];
+  CflArgs cfl;
+};
+
 struct CtArgs {
-  const void *CTsrc;  // double, or float when mixed (as the sweeps wrote them)
+  const void* CTsrc;  // double, or float when mixed (as the sweeps wrote them)
   void *F1, *F2, *F3;
   double *CTd;        // mixed form: the six averages also in FP64 (StageArgs::CTd)
+  int fin;            // the workgroup that combines the CFL reduction cfl, or -1
+  CflArgs cfl;
 };
 
 struct CopyArgs {
@@ -120,13 +130,14 @@ inline int slot_threads(const Geo& G, int slot) { return G.bs[slot] ? (int)G.bs[
 // Launch kinds of one step, in the order run_step makes them.
 enum LaunchKind {
   LK_EDGES, LK_SWEEP, LK_FLUXCT, LK_RK, LK_RECOV, LK_CARRY, LK_BND, LK_POST, LK_CFL, LK_CFL_FINISH,
-  LK_COPY, LK_PSWEEP, LK_N
+  LK_COPY, LK_PSWEEP, LK_PSWEEP3, LK_N
 };
 
 union AnyArgs {
   EdgeArgs e;
   SweepArgs s;
   PSweepArgs ps;
+  PSweep3Args ps3;
   CtArgs c;
   StageArgs st;
   FixArgs fx;
@@ -184,14 +195,16 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const 
 // i per wave; a workgroup's waves are stacked along the axis), a power of two
 // from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
-hipError_t launch_psweep(const Geo& G, int dir, const double* W, const void* metF, const double* dxs,
-                         const double* xs, const double* pc, double gam, void* F, void* CTsrc, bool mixed,
-                         hipStream_t st);
+hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A, bool mixed, hipStream_t st);
+// The three in one launch (s[d]: the sweep along d + 1), with the CFL
+// reduction of the same primitives when cfl is given; its workgroups' results
+// are then combined by the launch_fluxct that is given the same cfl.
+hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st);
 int psweep_segment(const Geo& G, int dir);
 size_t psweep_lds_bytes(int threads, bool mixed);
 // f32: CTsrc and F hold floats (the averages are formed in double either way)
 hipError_t launch_fluxct(const Geo& G, const void* CTsrc, void* F1, void* F2, void* F3, bool f32, double* CTd,
-                         hipStream_t st);
+                         const CflArgs* cfl, hipStream_t st);
 // n values of type double (to_float) or float (else) from src into dst, the other type
 hipError_t launch_retype(const void* src, void* dst, long long n, bool to_float, hipStream_t st);
 // RK update + sources into A.Ukeep (every interior cell), then recov1a into A.Wpre.
@@ -201,6 +214,7 @@ hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st);
 hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st);
 hipError_t launch_cfl(const Geo& G, const CflArgs& A, hipStream_t st);
 long long cfl_blocks(const Geo& G);  // 256-cell chunks of the CFL reduction
+long long cfl_slots(const Geo& G);   // its workgroups at most, of any size from 64 threads
 constexpr int CFL_GROUPS = 1024;     // its workgroups at most
 // Fold the per-wavefront event rows into cnt (and clear them).
 hipError_t launch_sum_counters(unsigned long long* cpart, long long rows, unsigned long long* cnt, hipStream_t st);

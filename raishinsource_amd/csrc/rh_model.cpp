@@ -253,8 +253,8 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
       !dalloc(&m->Uh, 9 * N) || !dalloc(&m->Us, 9 * N) || !dalloc(&m->Unext, 9 * N) || !dalloc(&m->F, 27 * N) ||
       !dalloc(&m->CT, 6 * N) || !dalloc(&m->wgout, N) || !dalloc(&m->chr, 64 * G.P2) || !dalloc(&m->bc, 54) || !dalloc(&m->dtbits, 4) || !dalloc(&m->cnt, NCOUNT) ||
       !dalloc(&m->carry, 2 + m->carry_cap) || !dalloc(&m->tdt, 2) || !dalloc(&m->cflag, N) ||
-      !dalloc(&m->pend, m->carry_cap) || !dalloc(&m->cfl_last, 4 * cfl_blocks(G)) ||
-      !dalloc(&m->cfl_min, 4 * cfl_blocks(G)))
+      !dalloc(&m->pend, m->carry_cap) || !dalloc(&m->cfl_last, 4 * cfl_slots(G)) ||
+      !dalloc(&m->cfl_min, 4 * cfl_slots(G)))
     return false;
   if (m->need_wo && !dalloc(&m->Wo, 9 * N)) return false;
   if ((p->irec == 5 || p->irec == 1) && !dalloc(&m->E, 18 * N)) return false;  // face values
@@ -486,14 +486,39 @@ static void* flux_plane(const raishin_model* m, double* F, long long p) {
   return m->mixed ? (void*)((float*)F + p * m->G.N) : (void*)(F + p * m->G.N);
 }
 
-bool stage_sweeps(raishin_model* m, const double* W, double* F) {
+static CflArgs cfl_args(raishin_model* m, const double* W, bool advance) {
+  CflArgs C{};
+  C.W = W; C.metC = m->metric_centre(); C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
+  C.dtbits = m->dtbits; C.blast = m->cfl_last; C.bmin = m->cfl_min; C.gam = m->p.gam;
+  C.cfl = m->p.cfl; C.tdt = advance ? m->tdt : nullptr;
+  return C;
+}
+
+// The three PPM sweeps go in one launch (with the step's CFL reduction),
+// except where the kernels are timed one by one.
+static bool sweeps_merged(const raishin_model* m) {
+  constexpr unsigned timed = 1u << K_SWEEP1 | 1u << K_SWEEP2 | 1u << K_SWEEP3 | 1u << K_FLUXCT | 1u << K_CFL;
+  return m->p.irec == 5 && !m->G.ppm_split && !(m->timing & timed);
+}
+
+bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* cfl) {
   const Geo& G = m->G;
   const int irec = m->p.irec;
+  auto ps = [&](int d) {
+    PSweepArgs A{};
+    A.W = W; A.metF = m->metric_face(d); A.dxs = m->dxs[d - 1]; A.xs = m->xs[d - 1]; A.pc = m->ppmc[d - 1];
+    A.gam = m->p.gam; A.F = flux_plane(m, F, (d - 1) * 9); A.CTsrc = m->CT;
+    return A;
+  };
+  if (sweeps_merged(m)) {
+    const PSweepArgs s[3] = {ps(1), ps(2), ps(3)};
+    HIPCHK(launch_psweep3(G, s, m->mixed, cfl, m->st));
+    return true;
+  }
   for (int d = 1; d <= 3; d++) {
     if (irec == 5 && !G.ppm_split) {
       TimedLaunch t(m, K_SWEEP1 + d - 1);
-      HIPCHK(launch_psweep(G, d, W, m->metric_face(d), m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam,
-                           flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed, m->st));
+      HIPCHK(launch_psweep(G, d, ps(d), m->mixed, m->st));
       continue;
     }
     if (irec == 5 || irec == 1) {
@@ -512,14 +537,16 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F) {
 // second half, which the float planes leave unused.
 static double* ct_fp64(const raishin_model* m, double* F) { return m->mixed ? F + 14 * m->G.N : nullptr; }
 
-bool stage_ct(raishin_model* m, double* F) {
+bool stage_ct(raishin_model* m, double* F, const CflArgs* cfl) {
   TimedLaunch t(m, K_FLUXCT);
   HIPCHK(launch_fluxct(m->G, m->CT, flux_plane(m, F, 0), flux_plane(m, F, 9), flux_plane(m, F, 18), m->mixed,
-                       ct_fp64(m, F), m->st));
+                       ct_fp64(m, F), cfl, m->st));
   return true;
 }
 
-bool stage_fluxes(raishin_model* m, const double* W, double* F) { return stage_sweeps(m, W, F) && stage_ct(m, F); }
+bool stage_fluxes(raishin_model* m, const double* W, double* F, const CflArgs* cfl) {
+  return stage_sweeps(m, W, F, cfl) && stage_ct(m, F, cfl);
+}
 
 bool stage_update(raishin_model* m, int rkstage, const double* W, const double* Ua, const double* Ub, double* Uout,
                   const double* F, const HostDt* hd) {
@@ -560,8 +587,8 @@ bool stage_post(raishin_model* m, const double* Wold, const double* Wo, double* 
 // One RK stage of the model path: sweeps -> flux-CT -> update (RK + recov) ->
 // fix-up -> ghosts/floors/conserved.
 bool run_stage(raishin_model* m, int rkstage, const double* Ua, const double* Ub, double* Uout,
-               const StageTap* tap) {
-  if (!stage_fluxes(m, m->W, m->F)) return false;
+               const StageTap* tap, const CflArgs* cfl) {
+  if (!stage_fluxes(m, m->W, m->F, cfl)) return false;
   if (tap && tap->ww) {
     // ww(d,n,i,j,k) as after ct()
     for (int d = 0; d < 3; d++)
@@ -581,11 +608,8 @@ bool copy_fluxes_out(raishin_model* m, double* ww, double* ct) {
 }
 
 bool run_cfl(raishin_model* m, const double* W, bool advance) {
-  CflArgs C{};
-  C.W = W; C.metC = m->metric_centre(); C.dx1b = m->dxb[0]; C.dx2b = m->dxb[1]; C.dx3b = m->dxb[2];
-  C.dtbits = m->dtbits; C.blast = m->cfl_last; C.bmin = m->cfl_min; C.gam = m->p.gam;
-  C.cfl = m->p.cfl; C.tdt = advance ? m->tdt : nullptr;
-  { TimedLaunch t(m, K_CFL); HIPCHK(launch_cfl(m->G, C, m->st)); }
+  TimedLaunch t(m, K_CFL);
+  HIPCHK(launch_cfl(m->G, cfl_args(m, W, advance), m->st));
   return true;
 }
 
@@ -605,9 +629,12 @@ bool cdtcfl4_on(raishin_model* m, const double* W, double* dtcfl, double* dt1, d
 
 bool run_step(raishin_model* m) {
   const long long N = m->G.N;
-  if (!run_cfl(m, m->W, true)) return false;
+  // merged sweeps: the CFL reduction goes with the first stage's
+  const bool merged = sweeps_merged(m);
+  const CflArgs C = cfl_args(m, m->W, true);
+  if (!merged && !run_cfl(m, m->W, true)) return false;
   if (m->need_wo) HIPCHK(launch_copy(m->G, m->Wo, m->W, 9 * N, m->st));
-  if (!run_stage(m, 1, m->Ucur, nullptr, m->Uh)) return false;
+  if (!run_stage(m, 1, m->Ucur, nullptr, m->Uh, nullptr, merged ? &C : nullptr)) return false;
   if (m->p.irkt == 2) {
     if (!run_stage(m, 2, m->Ucur, m->Uh, m->Unext)) return false;
   } else {

@@ -127,9 +127,10 @@ void theta_trig_table(const raishin_pram& p, const double* x3, const double* x3a
 
 // Pieces of one RK stage on explicit buffers (SoA planes on the device).
 // Fluxes: the three direction sweeps and flux-CT from primitives W into F (27 planes).
-bool stage_fluxes(raishin_model* m, const double* W, double* F);
-bool stage_sweeps(raishin_model* m, const double* W, double* F);  // the three sweeps (hll)
-bool stage_ct(raishin_model* m, double* F);                        // flux-CT in place (ct)
+// cfl: the step's CFL reduction goes with them (merged sweeps only).
+bool stage_fluxes(raishin_model* m, const double* W, double* F, const rh::CflArgs* cfl = nullptr);
+bool stage_sweeps(raishin_model* m, const double* W, double* F, const rh::CflArgs* cfl = nullptr);  // the three sweeps (hll)
+bool stage_ct(raishin_model* m, double* F, const rh::CflArgs* cfl = nullptr);                        // flux-CT in place (ct)
 // RK update + sources + recovery into m->Wpre (interior), then the in-order fix-up.
 // ak: device dt/dx*b arrays and dt from the caller, or all null to use the
 // model's own CFL result.
@@ -141,7 +142,7 @@ bool stage_post(raishin_model* m, const double* Wold, const double* Wo, double* 
 // The CFL minimum of primitives W; advance: then time += cfl * dtcfl.
 bool run_cfl(raishin_model* m, const double* W, bool advance);
 bool run_stage(raishin_model* m, int rkstage, const double* Ua, const double* Ub, double* Uout,
-               const struct StageTap* tap = nullptr);
+               const struct StageTap* tap = nullptr, const rh::CflArgs* cfl = nullptr);
 bool run_step(raishin_model* m);
 // cdtcfl4 of primitives W: dtcfl, dt1..dt3 to the host (synchronises).
 bool cdtcfl4_on(raishin_model* m, const double* W, double* dtcfl, double* dt1, double* dt2, double* dt3);

@@ -81,7 +81,7 @@ def footprint(p):
     cap = (ni - 2 * nm1) * (nj - 2 * nm1) * (nk - 2 * nm1)
     need_wo = any(2 in getattr(p, a) for a in ("iboux1in", "iboux1ot", "iboux2in", "iboux2ot", "iboux3in",
                                                "iboux3ot"))
-    ncfl = max((max(ni - 2, 0) * max(nj - 2, 0) * max(nk - 2, 0) + 255) // 256, 1)
+    ncfl = min(1024, max((max(ni - 2, 0) * max(nj - 2, 0) * max(nk - 2, 0) + 63) // 64, 1))
     planes = 7 * 9 + 27 + 6 + 1 + 9 + (9 if need_wo else 0) + (18 if p.irec in (1, 5) else 0)
     b = 8 * n * planes
     b += n + 8 * (2 + cap) + cap                     # cflag, carry count + list + counter, pend

@@ -129,3 +129,20 @@ def test_workgroup_tiles_equal_split(threads, ni, nj, nk, seg, mixed):
     same(a, b, threads)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("name,mixed,threads", [("t2d", False, 256), ("t2d", True, 64), ("t3dppm", False, 128)])
+def test_one_launch_equals_separate(name, mixed, threads):
+    """The three sweeps, the CFL reduction and its combination in the
+    launches of a stage against a launch each (a model whose kernels are
+    timed), with the same time and step."""
+    a, b = make(configs.ALL[name], mixed), make(configs.ALL[name], mixed)
+    for mm in (a, b):
+        mm.set_block_sizes([threads] * 8)
+    b.set_timing(True)
+    for s in range(3):
+        assert a.step(1) == b.step(1), s
+    assert b.get_timing()["sweep_k"][1] > 0 and b.get_timing()["cfl"][1] == 3
+    same(a, b, name)
+    a.close()
+    b.close()
