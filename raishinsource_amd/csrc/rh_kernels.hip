@@ -1172,18 +1172,21 @@ RH_DEV long long chr_plane(int l, int a, int b) {
   return (long long)(l + 4 * a + 16 * b);
 }
 
-template <int STAGE, bool SYM, class FT, bool MK>
-RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
+// The cell's index and (i,k) to c, i, k; its stage-start primitives to w; its
+// updated conserved variables to put(m, value).
+template <int STAGE, bool SYM, class FT, bool MK, int NGF, class Put>
+RH_DEV bool rk_cell(const Geo& G, const StageArgs& A, unsigned blk, unsigned& c, int& i, int& k, double w[9], Put&& put) {
   const FT* __restrict__ F1 = (const FT*)A.F1;
   const FT* __restrict__ F2 = (const FT*)A.F2;
   const FT* __restrict__ F3 = (const FT*)A.F3;
-  int i, j, k;
+  int j;
   const unsigned t = blk * blockDim.x + threadIdx.x;
   if (!box_index(t, G.nm1 + 1, G.ni - G.nm1, jlo(G, G.nm1 + 1), jhi(G, G.nj - G.nm1), G.nm1 + 1, G.nk - G.nm1, i, j,
                  k))
-    return;
+    return false;
   const long long N = G.N;
-  const unsigned c = cidx(i, j, k, G), c8 = c * 8u;
+  c = cidx(i, j, k, G);
+  const unsigned c8 = c * 8u;
   const long long sj = jstride(G), sk = kstride(G);
   const double gam = A.gam;
   // dt and dt/dx (main.f90:760-780), recomputed per thread from the CFL minimum
@@ -1198,7 +1201,6 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
   }
   const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
 
-  double w[9];
 #pragma unroll
   for (int n = 0; n < 9; n++) w[n] = ld_(A.W + (long long)n * N, c8);
 
@@ -1237,10 +1239,10 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
   // Several variables at a time, their reads in flight together (left to
   // itself the compiler waits for one variable's eight before the next one's):
   // three in FP64 (256x128x128 0.449 -> 0.431 ms, with all nine 0.479; one
-  // 128x128 row 11.7 -> 7.8 us), all nine where the fluxes are floats (0.401
-  // -> 0.377 ms, with three 0.414; 0.43 ms is 2.0 GB at 4.7 TB/s, near what a
-  // copy reaches).
-  constexpr int NG = sizeof(FT) == 4 ? 9 : 3;
+  // 128x128 row 11.7 -> 7.8 us); where the fluxes are floats NGF, nine in the
+  // update alone (0.401 -> 0.377 ms, with three 0.414) and one in the fused
+  // kernel, whose registers more of them would spill (0.432, three 0.613).
+  constexpr int NG = sizeof(FT) == 4 ? NGF : 3;
 #pragma unroll
   for (int g = 0; g < 9; g += NG) {
     double f[NG][6], ua[NG], ub[NG];
@@ -1275,30 +1277,29 @@ RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
         else if (STAGE == 3) v = v + sdt * 0.25;
         else v = v + sdt * (double)(2.0f / 3.0f);
       }
-      st_(A.Ukeep + (long long)m * N, c8, v);
+      put(m, v);
     }
   }
+  return true;
+}
+
+template <int STAGE, bool SYM, class FT, bool MK>
+RH_DEV void b_rk(const Geo& G, const StageArgs& A, unsigned blk) {
+  unsigned c;
+  int i, k;
+  double w[9];
+  rk_cell<STAGE, SYM, FT, MK, 9>(G, A, blk, c, i, k, w,
+                              [&](int m, double v) { st_(A.Ukeep + (long long)m * G.N, c * 8u, v); });
 }
 
 // recov1a (recov.f90:578-1228) or recov2 (recov.f90:1919-2454) on every
 // interior cell from the stage's RK result; cells whose initial W is
 // inherited are flagged for k_recov_carry.
 template <int IW, bool MK>
-RH_DEV void b_recov(const Geo& G, const StageArgs& A, unsigned blk) {
-  int i, j, k;
-  const unsigned t = blk * blockDim.x + threadIdx.x;
-  if (!box_index(t, G.nm1 + 1, G.ni - G.nm1, jlo(G, G.nm1 + 1), jhi(G, G.nj - G.nm1), G.nm1 + 1, G.nk - G.nm1, i, j,
-                 k))
-    return;
+RH_DEV void recov_put(const Geo& G, const StageArgs& A, unsigned blk, unsigned c, int i, int k, const double u[9],
+                      const double w[9], bool keep) {
   const long long N = G.N;
-  const unsigned c = cidx(i, j, k, G);
   const MetOf<MK, double> M(A.metC, G.P2, q2(i, k, G));
-  double w[9], u[9];
-#pragma unroll
-  for (int n = 0; n < 9; n++) {
-    w[n] = ld_(A.W + (long long)n * N, c * 8u);
-    u[n] = ld_((const double*)A.Ukeep + (long long)n * N, c * 8u);
-  }
   RecovOut ro;
   bool carry;
   double wgout;
@@ -1323,7 +1324,43 @@ RH_DEV void b_recov(const Geo& G, const StageArgs& A, unsigned blk) {
     A.cflag[c] = 1;
     const unsigned long long slot = atomicAdd(&A.carry[0], 1ULL);
     if (slot < (unsigned long long)A.carry_cap) A.carry[1 + slot] = (unsigned long long)c;
+    if (keep)
+#pragma unroll
+      for (int n = 0; n < 9; n++) st_(A.Ukeep + (long long)n * N, c * 8u, u[n]);
   }
+}
+
+template <int IW, bool MK>
+RH_DEV void b_recov(const Geo& G, const StageArgs& A, unsigned blk) {
+  int i, j, k;
+  const unsigned t = blk * blockDim.x + threadIdx.x;
+  if (!box_index(t, G.nm1 + 1, G.ni - G.nm1, jlo(G, G.nm1 + 1), jhi(G, G.nj - G.nm1), G.nm1 + 1, G.nk - G.nm1, i, j,
+                 k))
+    return;
+  const long long N = G.N;
+  const unsigned c = cidx(i, j, k, G);
+  double w[9], u[9];
+#pragma unroll
+  for (int n = 0; n < 9; n++) {
+    w[n] = ld_(A.W + (long long)n * N, c * 8u);
+    u[n] = ld_((const double*)A.Ukeep + (long long)n * N, c * 8u);
+  }
+  recov_put<IW, MK>(G, A, blk, c, i, k, u, w, false);
+}
+
+// The update and the recovery of a cell in one kernel: the stage's conserved
+// variables stay in registers (they are read again only where k_recov_carry
+// has the cell, which finds them in Ukeep), and W is read once: 27 planes
+// less.  164 VGPRs put it at 3 waves per SIMD, enough for the update's reads
+// since they go out in groups: 256x128x128 0.433 + 0.166 -> 0.466 ms, 64^3
+// 33 -> 24 us, one 128x128 row 14.2 -> 11.3 us.
+template <int STAGE, class FT, int IW>
+RH_DEV void b_rkrecov(const Geo& G, const StageArgs& A, unsigned blk) {
+  unsigned c;
+  int i, k;
+  double w[9], u[9];
+  if (!rk_cell<STAGE, true, FT, true, 1>(G, A, blk, c, i, k, w, [&](int m, double v) { u[m] = v; })) return;
+  recov_put<IW, true>(G, A, blk, c, i, k, u, w, true);
 }
 
 // ------------------------------------------------------------------------
@@ -2110,6 +2147,8 @@ template <class FT>
 __global__ void __launch_bounds__(256) k_fluxct(Geo G, CtArgs A) { b_fluxct<FT>(G, A, xcd_block()); }
 template <int STAGE, bool SYM, class FT, bool MK>
 __global__ void __launch_bounds__(256) k_rk(Geo G, StageArgs A) { b_rk<STAGE, SYM, FT, MK>(G, A, xcd_block()); }
+template <int STAGE, class FT, int IW>
+__global__ void __launch_bounds__(256) k_rkrecov(Geo G, StageArgs A) { b_rkrecov<STAGE, FT, IW>(G, A, xcd_block()); }
 template <int IW, bool MK>
 __global__ void __launch_bounds__(256) k_recov(Geo G, StageArgs A) { b_recov<IW, MK>(G, A, xcd_block()); }
 template <int IW, bool MK>
@@ -2172,6 +2211,12 @@ __global__ void __launch_bounds__(256) kb_rk(const BatchItem* __restrict__ it, i
   RH_BATCH_PROLOGUE
   const StageArgs A = it[q].A.st;
   b_rk<STAGE, SYM, FT, MK>(G, A, blk);
+}
+template <int STAGE, class FT, int IW>
+__global__ void __launch_bounds__(256) kb_rkrecov(const BatchItem* __restrict__ it, int n) {
+  RH_BATCH_PROLOGUE
+  const StageArgs A = it[q].A.st;
+  b_rkrecov<STAGE, FT, IW>(G, A, blk);
 }
 template <int IW, bool MK>
 __global__ void __launch_bounds__(256) kb_recov(const BatchItem* __restrict__ it, int n) {
@@ -2561,17 +2606,15 @@ hipError_t launch_fluxct(const Geo& G, const void* CTsrc, void* F1, void* F2, vo
   return hipGetLastError();
 }
 
+static int rk_variant(const Geo& G, int stage, const StageArgs& A) {
+  return stage + 8 * (int)A.chr_sym + 16 * (int)A.f32flux + 32 * G.mk;
+}
+
 hipError_t launch_update(const Geo& G, int stage, const StageArgs& A, hipStream_t st) {
   const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
   const int bt = slot_threads(G, TS_RK);
   const unsigned nb = nblk(n, bt);
-  const int variant = stage + 8 * (int)A.chr_sym + 16 * (int)A.f32flux + 32 * G.mk;
-  if (g_rec) {
-    AnyArgs a{};
-    a.st = A;
-    record(LK_RK, variant, bt, nb, G, a);
-    return hipSuccess;
-  }
+  const int variant = rk_variant(G, stage, A);
   if (n == 0) return hipSuccess;
   with_rk(variant, [&](auto S, auto Y, auto T, auto K) {
     hipLaunchKernelGGL((k_rk<S.value, Y.value, typename decltype(T)::type, K.value>), dim3(nb), dim3(bt), 0, st, G, A);
@@ -2582,12 +2625,49 @@ hipError_t launch_update(const Geo& G, int stage, const StageArgs& A, hipStream_
 hipError_t launch_recov(const Geo& G, const StageArgs& A, hipStream_t st) {
   const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
   const int bt = slot_threads(G, TS_RECOV);
-  if (g_rec) { AnyArgs a{}; a.st = A; record(LK_RECOV, G.iwvec + 4 * G.mk, bt, nblk(n, bt), G, a); return hipSuccess; }
   if (n == 0) return hipSuccess;
   with_recov(G.iwvec + 4 * G.mk, [&](auto I, auto K) {
     hipLaunchKernelGGL((k_recov<I.value, K.value>), dim3(nblk(n, bt)), dim3(bt), 0, st, G, A);
   });
   return hipGetLastError();
+}
+
+// The fused update and recovery for a variant as launch_update's, plus
+// 64*(iwvec == 2); false where it is not built (general metric tables or
+// Christoffel symbols that are not symmetric).
+template <class F>
+static bool with_rkrecov(int variant, F&& f) {
+  if ((variant & 40) != 40) return false;
+  auto t = [&](auto S) {
+    auto w = [&](auto T) {
+      if (variant & 64) f(S, T, IC<2>{});
+      else f(S, T, IC<1>{});
+    };
+    if (variant & 16) w(TypeTag<float>{});
+    else w(TypeTag<double>{});
+  };
+  switch (variant & 7) {
+    case 1: t(IC<1>{}); break;
+    case 2: t(IC<2>{}); break;
+    case 3: t(IC<3>{}); break;
+    default: t(IC<4>{}); break;
+  }
+  return true;
+}
+
+hipError_t launch_update_recov(const Geo& G, int stage, const StageArgs& A, hipStream_t st) {
+  const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
+  const int bt = slot_threads(G, TS_RK);
+  const unsigned nb = nblk(n, bt);
+  const int variant = rk_variant(G, stage, A) + 64 * (G.iwvec == 2);
+  if (g_rec) { AnyArgs a{}; a.st = A; record(LK_RKRECOV, variant, bt, nb, G, a); return hipSuccess; }
+  if (n == 0) return hipSuccess;
+  if (with_rkrecov(variant, [&](auto S, auto T, auto I) {
+        hipLaunchKernelGGL((k_rkrecov<S.value, typename decltype(T)::type, I.value>), dim3(nb), dim3(bt), 0, st, G, A);
+      }))
+    return hipGetLastError();
+  const hipError_t e = launch_update(G, stage, A, st);
+  return e == hipSuccess ? launch_recov(G, A, st) : e;
 }
 
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st) {
@@ -2694,13 +2774,17 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
       if (variant == 1) hipLaunchKernelGGL(kb_fluxct<float>, g, b, 0, st, it, n);
       else hipLaunchKernelGGL(kb_fluxct<double>, g, b, 0, st, it, n);
       break;
-    case LK_RK:
-      with_rk(variant, [&](auto S, auto Y, auto T, auto K) {
+    case LK_RKRECOV:
+      if (with_rkrecov(variant, [&](auto S, auto T, auto I) {
+            hipLaunchKernelGGL((kb_rkrecov<S.value, typename decltype(T)::type, I.value>), g, b, 0, st, it, n);
+          }))
+        break;
+      with_rk(variant & 63, [&](auto S, auto Y, auto T, auto K) {
         hipLaunchKernelGGL((kb_rk<S.value, Y.value, typename decltype(T)::type, K.value>), g, b, 0, st, it, n);
       });
-      break;
-    case LK_RECOV:
-      with_recov(variant, [&](auto I, auto K) { hipLaunchKernelGGL((kb_recov<I.value, K.value>), g, b, 0, st, it, n); });
+      with_recov(((variant & 64) ? 2 : 1) + ((variant & 32) ? 4 : 0), [&](auto I, auto K) {
+        hipLaunchKernelGGL((kb_recov<I.value, K.value>), g, b, 0, st, it, n);
+      });
       break;
     case LK_BND: hipLaunchKernelGGL(kb_bnd, g, b, 0, st, it, n); break;
     case LK_POST:

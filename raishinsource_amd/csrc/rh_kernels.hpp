@@ -129,7 +129,7 @@ inline int slot_threads(const Geo& G, int slot) { return G.bs[slot] ? (int)G.bs[
 
 // Launch kinds of one step, in the order run_step makes them.
 enum LaunchKind {
-  LK_EDGES, LK_SWEEP, LK_FLUXCT, LK_RK, LK_RECOV, LK_CARRY, LK_BND, LK_POST, LK_CFL, LK_CFL_FINISH,
+  LK_EDGES, LK_SWEEP, LK_FLUXCT, LK_RKRECOV, LK_CARRY, LK_BND, LK_POST, LK_CFL, LK_CFL_FINISH,
   LK_COPY, LK_PSWEEP, LK_PSWEEP3, LK_N
 };
 
@@ -210,6 +210,9 @@ hipError_t launch_retype(const void* src, void* dst, long long n, bool to_float,
 // RK update + sources into A.Ukeep (every interior cell), then recov1a into A.Wpre.
 hipError_t launch_update(const Geo& G, int stage, const StageArgs& A, hipStream_t st);
 hipError_t launch_recov(const Geo& G, const StageArgs& A, hipStream_t st);
+// Both, fused where it is built: A.Ukeep then holds only the cells left to
+// launch_recov_carry.
+hipError_t launch_update_recov(const Geo& G, int stage, const StageArgs& A, hipStream_t st);
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st);
 hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st);
 hipError_t launch_cfl(const Geo& G, const CflArgs& A, hipStream_t st);
