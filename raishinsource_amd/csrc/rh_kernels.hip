@@ -748,13 +748,14 @@ RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, unsigned blk) {
 // u[9] = stage conserved (after RK + sources); wold = previous primitives
 // (initial guess and fallback).  Writes w[9].  The initial W of a cell whose
 // quadratic has no non-negative root is inherited from the previous cell in
-// the reference's loop order; that cell is flagged in *carry.
+// the reference's loop order; that cell is flagged in *carry.  s5: whether
+// w[5] (a pow) is wanted; 0 otherwise.
 // ------------------------------------------------------------------------
 struct RecovOut { double w[9]; int fallback, fail, negrho, negp, vsqgt1, det0, guard, indep; };
 
 template <class MT>
 RH_DEV void recov_cell(const double u[9], const double wold[9], const MT& M, double gam, double dmin,
-                       double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool& carry,
+                       double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool s5, bool& carry,
                        RecovOut& o, double& wg_out) {
   const double safty = 1.0e-4, saftybig = 1.0e5, dv = 1.0e-2;
   const double gam1 = gam / (gam - 1.0);
@@ -962,11 +963,11 @@ RH_DEV void recov_cell(const double u[9], const double wold[9], const MT& M, dou
   }
   if (irecov == 0) {
     o.w[0] = ro; o.w[1] = util[1]; o.w[2] = util[2]; o.w[3] = util[3]; o.w[4] = pp;
-    o.w[5] = ro * pp / pow(ro, gam - 1.0);
+    o.w[5] = s5 ? ro * pp / pow(ro, gam - 1.0) : 0.0;
   } else {
     o.fail = 1;
     o.w[0] = ro1; o.w[1] = wold[1]; o.w[2] = wold[2]; o.w[3] = wold[3]; o.w[4] = pp1;
-    o.w[5] = ro1 * pp1 / pow(ro1, gam);
+    o.w[5] = s5 ? ro1 * pp1 / pow(ro1, gam) : 0.0;
   }
   o.w[6] = u[6] * (1.0 / detg1);
   o.w[7] = u[7] * (1.0 / detg1);
@@ -983,7 +984,7 @@ RH_DEV void recov_cell(const double u[9], const double wold[9], const MT& M, dou
 // ------------------------------------------------------------------------
 template <class MT>
 RH_DEV void recov2_cell(const double u[9], const double wold[9], const MT& M, double gam, double dmin,
-                        double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool& carry,
+                        double pmin, int iter, double x1pow15, double x1pow25, double wg_in, bool s5, bool& carry,
                         RecovOut& o, double& wg_out) {
   const double safty = 1.0e-5, dv = 1.0e-4;
   const double gam1 = gam / (gam - 1.0);
@@ -1136,11 +1137,11 @@ RH_DEV void recov2_cell(const double u[9], const double wold[9], const MT& M, do
       util[m] = (gf * (1.0 / (wg + bsq))) * (qt + qdotb * bcon[m] * (1.0 / wg));
     }
     o.w[0] = ro; o.w[1] = util[1]; o.w[2] = util[2]; o.w[3] = util[3]; o.w[4] = pp;
-    o.w[5] = pp / pow(ro, gam - 1.0);
+    o.w[5] = s5 ? pp / pow(ro, gam - 1.0) : 0.0;
   } else {
     o.fail = 1;
     o.w[0] = ro1; o.w[1] = wold[1]; o.w[2] = wold[2]; o.w[3] = wold[3]; o.w[4] = pp1;
-    o.w[5] = pp1 / pow(ro1, gam - 1.0);
+    o.w[5] = s5 ? pp1 / pow(ro1, gam - 1.0) : 0.0;
   }
   o.w[6] = u[6] * (1.0 / detg1);
   o.w[7] = u[7] * (1.0 / detg1);
@@ -1151,10 +1152,10 @@ RH_DEV void recov2_cell(const double u[9], const double wold[9], const MT& M, do
 // one cell of the recovery iwvec selects
 template <int IW, class MT>
 RH_DEV void recov_any(const double u[9], const double wold[9], const MT& M, double gam, double dmin, double pmin,
-                      int iter, double x1pow15, double x1pow25, double wg_in, bool& carry, RecovOut& o,
+                      int iter, double x1pow15, double x1pow25, double wg_in, bool s5, bool& carry, RecovOut& o,
                       double& wg_out) {
-  if constexpr (IW == 2) recov2_cell(u, wold, M, gam, dmin, pmin, iter, x1pow15, x1pow25, wg_in, carry, o, wg_out);
-  else recov_cell(u, wold, M, gam, dmin, pmin, iter, x1pow15, x1pow25, wg_in, carry, o, wg_out);
+  if constexpr (IW == 2) recov2_cell(u, wold, M, gam, dmin, pmin, iter, x1pow15, x1pow25, wg_in, s5, carry, o, wg_out);
+  else recov_cell(u, wold, M, gam, dmin, pmin, iter, x1pow15, x1pow25, wg_in, s5, carry, o, wg_out);
 }
 
 // ------------------------------------------------------------------------
@@ -1303,8 +1304,8 @@ RH_DEV void recov_put(const Geo& G, const StageArgs& A, unsigned blk, unsigned c
   RecovOut ro;
   bool carry;
   double wgout;
-  recov_any<IW>(u, w, M, A.gam, A.dmin, A.pmin, A.iter, A.r15[i - 1], A.r25[i - 1], __builtin_nan(""), carry, ro,
-                wgout);
+  recov_any<IW>(u, w, M, A.gam, A.dmin, A.pmin, A.iter, A.r15[i - 1], A.r25[i - 1], __builtin_nan(""), A.s5,
+                carry, ro, wgout);
   const bool dep = carry && !ro.indep;
 #pragma unroll
   for (int n = 0; n < 9; n++) st_(A.Wpre + (long long)n * N, c * 8u, ro.w[n]);
@@ -1848,7 +1849,8 @@ RH_DEV void carry_cell(const Geo& G, const FixArgs& A, long long c, int i, int k
   RecovOut ro;
   bool carry;
   double wgout;
-  recov_any<IW>(u, w, M, A.gam, A.dmin, A.pmin, A.iter, A.r15[i - 1], A.r25[i - 1], wg_prev, carry, ro, wgout);
+  recov_any<IW>(u, w, M, A.gam, A.dmin, A.pmin, A.iter, A.r15[i - 1], A.r25[i - 1], wg_prev, A.s5, carry, ro,
+                wgout);
   for (int m = 0; m < 9; m++) A.Wpre[(long long)m * N + c] = ro.w[m];
   A.wgout[c] = wgout;
   if (ro.fallback) atomicAdd(&A.cnt[C_FALLBACK], 1ULL);
@@ -1969,7 +1971,7 @@ __global__ void __launch_bounds__(256) k_metric_tables(int ni, int nk, int metri
 // Compact tables (MetK) of the four locations from the general ones, in
 // double and, for the three faces, in float (the derived values formed in
 // float from float-rounded entries, as the mixed form forms them), one
-// thread per (i,k).  *ok is cleared where the metric does not have the
+// thread per location (blockIdx.y) and (i,k).  *ok is cleared where the metric does not have the
 // structure the compact form assumes (the caller sets it to 1 first).
 template <class R>
 RH_DEV void put_compact(const double* met, long long P2, long long q, R* out, bool centre) {
@@ -1988,25 +1990,24 @@ RH_DEV void put_compact(const double* met, long long P2, long long q, R* out, bo
 __global__ void __launch_bounds__(256) k_compact_metric(CompactArgs A, long long P2, int* ok) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= P2) return;
+  const int a = blockIdx.y;
+  const double* met = A.met[a];
+  auto bits = [&](int e) { return __double_as_longlong(met[(long long)e * P2 + q]); };
   bool fine = true;
-  for (int a = 0; a < 4; a++) {
-    const double* met = A.met[a];
-    auto bits = [&](int e) { return __double_as_longlong(met[(long long)e * P2 + q]); };
-    for (int h = 0; h < 2; h++)
-      for (int m = 0; m < 4; m++)
-        for (int n = m + 1; n < 4; n++) {
-          fine = fine && bits(16 * h + m + 4 * n) == bits(16 * h + n + 4 * m);
-          if (n == 3 || (h == 1 && m == 0 && n == 2)) fine = fine && bits(16 * h + m + 4 * n) == 0;
-        }
-    put_compact<double>(met, P2, q, A.mk[a], a == 0);
-    if (a > 0) put_compact<float>(met, P2, q, A.mkf[a - 1], false);
-  }
+  for (int h = 0; h < 2; h++)
+    for (int m = 0; m < 4; m++)
+      for (int n = m + 1; n < 4; n++) {
+        fine = fine && bits(16 * h + m + 4 * n) == bits(16 * h + n + 4 * m);
+        if (n == 3 || (h == 1 && m == 0 && n == 2)) fine = fine && bits(16 * h + m + 4 * n) == 0;
+      }
+  put_compact<double>(met, P2, q, A.mk[a], a == 0);
+  if (a > 0) put_compact<float>(met, P2, q, A.mkf[a - 1], false);
   if (!fine) atomicAnd(ok, 0);
 }
 
 hipError_t launch_compact_metric(const CompactArgs& A, long long P2, int* ok, hipStream_t st) {
   if (P2 <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_compact_metric, dim3((unsigned)((P2 + 255) / 256)), dim3(256), 0, st, A, P2, ok);
+  hipLaunchKernelGGL(k_compact_metric, dim3((unsigned)((P2 + 255) / 256), 4), dim3(256), 0, st, A, P2, ok);
   return hipGetLastError();
 }
 

@@ -32,6 +32,7 @@ struct StageArgs {
   // (planes ww(2,7) ww(3,7) ww(1,8) ww(3,8) ww(1,9) ww(2,9)), which the
   // update reads instead of their float copies in F1..F3; null in FP64
   const double *CTd;
+  bool s5;                         // the recovered entropy variable is wanted
 };
 
 struct PostArgs {
@@ -69,6 +70,7 @@ struct FixArgs {
   long long carry_cap;
   double gam, dmin, pmin;
   int iter;
+  bool s5;                         // as StageArgs
 };
 
 struct EdgeArgs {

@@ -549,7 +549,7 @@ bool stage_fluxes(raishin_model* m, const double* W, double* F, const CflArgs* c
 }
 
 bool stage_update(raishin_model* m, int rkstage, const double* W, const double* Ua, const double* Ub, double* Uout,
-                  const double* F, const HostDt* hd, bool keep_u) {
+                  const double* F, const HostDt* hd, bool inner) {
   const Geo& G = m->G;
   StageArgs A{};
   A.W = W; A.Ua = Ua; A.Ub = Ub;
@@ -564,7 +564,10 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
   A.gam = m->p.gam; A.cfl = m->p.cfl; A.dmin = m->p.dmin; A.pmin = m->p.pmin; A.iter = m->p.iter;
   A.chr_sym = m->chr_sym;
   if (hd) { A.ak1 = hd->ak1; A.ak2 = hd->ak2; A.ak3 = hd->ak3; A.dt_host = hd->dt; }
-  if (keep_u) {
+  // the atmosphere of models 7..15 sets the entropy variable to zero whatever
+  // the recovery gave (a pow of some 230 instructions)
+  A.s5 = !inner || m->p.model < 7 || m->p.model > 15;
+  if (!inner) {
     { TimedLaunch t(m, K_UPDATE); HIPCHK(launch_update(G, rkstage, A, m->st)); }
     { TimedLaunch t(m, K_RECOV); HIPCHK(launch_recov(G, A, m->st)); }
   } else {
@@ -575,7 +578,7 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
   X.W = W; X.Ustage = Uout; X.metC = m->metric_centre(); X.r15 = m->r15; X.r25 = m->r25; X.Wpre = m->Wpre;
   X.wgout = m->wgout; X.carry = m->carry; X.cnt = m->cnt; X.cflag = m->cflag; X.pend = m->pend;
   X.carry_cap = m->carry_cap; X.gam = m->p.gam;
-  X.dmin = m->p.dmin; X.pmin = m->p.pmin; X.iter = m->p.iter;
+  X.dmin = m->p.dmin; X.pmin = m->p.pmin; X.iter = m->p.iter; X.s5 = A.s5;
   { TimedLaunch t(m, K_CARRY); HIPCHK(launch_recov_carry(G, X, m->st)); }
   return true;
 }
@@ -599,7 +602,7 @@ bool run_stage(raishin_model* m, int rkstage, const double* Ua, const double* Ub
     for (int d = 0; d < 3; d++)
       if (!copy_planes_out(m, flux_plane(m, m->F, (long long)d * 9), 9, 3, d, tap->ww, m->mixed)) return false;
   }
-  if (!stage_update(m, rkstage, m->W, Ua, Ub, Uout, m->F, nullptr, false)) return false;
+  if (!stage_update(m, rkstage, m->W, Ua, Ub, Uout, m->F, nullptr, !(tap && tap->wpre))) return false;
   if (tap && tap->wpre && !copy_planes_out(m, m->Wpre, 9, 1, 0, tap->wpre)) return false;
   if (!stage_post(m, m->W, m->need_wo ? m->Wo : m->W, m->Wb, Uout)) return false;
   std::swap(m->W, m->Wb);

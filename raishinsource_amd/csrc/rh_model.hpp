@@ -132,12 +132,13 @@ bool stage_fluxes(raishin_model* m, const double* W, double* F, const rh::CflArg
 bool stage_sweeps(raishin_model* m, const double* W, double* F, const rh::CflArgs* cfl = nullptr);  // the three sweeps (hll)
 bool stage_ct(raishin_model* m, double* F, const rh::CflArgs* cfl = nullptr);                        // flux-CT in place (ct)
 // RK update + sources + recovery into m->Wpre (interior), then the in-order
-// fix-up.  keep_u: the RK result to Uout whole (else it need not be there).
+// fix-up.  inner: nobody reads the RK result in Uout or the recovered
+// primitives but the stage itself.
 // ak: device dt/dx*b arrays and dt from the caller, or all null to use the
 // model's own CFL result.
 struct HostDt { const double *ak1 = nullptr, *ak2 = nullptr, *ak3 = nullptr; double dt = 0.0; };
 bool stage_update(raishin_model* m, int rkstage, const double* W, const double* Ua, const double* Ub, double* Uout,
-                  const double* F, const HostDt* hd, bool keep_u);
+                  const double* F, const HostDt* hd, bool inner);
 // Ghost fill, floors and conserved variables: m->Wpre -> Wout, Uout.
 bool stage_post(raishin_model* m, const double* Wold, const double* Wo, double* Wout, double* Uout);
 // The CFL minimum of primitives W; advance: then time += cfl * dtcfl.

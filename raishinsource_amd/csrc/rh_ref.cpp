@@ -484,7 +484,7 @@ void raishin_recov(double* uu, double* uri, const double* gcov, const double* gc
   hd.ak2 = g.ak + g.p.imax;
   hd.ak3 = g.ak + g.p.imax + g.p.jmax;
   hd.dt = g.pd.dt;
-  if (!stage_update(g.m, g.pd.rk, W, Ua, Ub, Uout, F, &hd, true)) return;
+  if (!stage_update(g.m, g.pd.rk, W, Ua, Ub, Uout, F, &hd, false)) return;
   g.pd.phase = 5;
 }
 
