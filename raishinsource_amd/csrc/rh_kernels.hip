@@ -751,6 +751,40 @@ RH_DEV void b_fluxct(const Geo& G, const CtArgs& A, unsigned blk) {
 // the reference's loop order; that cell is flagged in *carry.  s5: whether
 // w[5] (a pow) is wanted; 0 otherwise.
 // ------------------------------------------------------------------------
+// The reference's "goto 95": W times 1.5 or 0.9 until it is admissible.  It may
+// never be; the trips are bounded, and true says the bound was hit.  Such a
+// cell's W wanders between the two conditions without repeating, so it needs
+// all its trips, one dependent chain: they are free of branches, eight between
+// two looks at the result (with a branch per condition and trip 320 cycles,
+// 13.3 ms for one cell of a strongly magnetised tube, the length of the whole
+// launch; now 9.5).  The first trip, which ends it for most cells, is by itself.
+RH_DEV bool admissible_w(double& wg, double gf, double drogf, double gam2, double bsq, double qtsq, double qdotn,
+                         double qdotbsq) {
+  const double b2 = 2.0 * bsq, qb = qtsq - bsq * bsq, bq = 0.5 * bsq + qdotn, q2b = 0.5 * qdotbsq;
+  int n = 0;
+  auto trip = [&](bool go) {
+    const double pp = gam2 * (wg * gf - drogf);
+    const double wsq = wg * wg, w3 = wsq * wg;
+    const double t3a = w3 * (wg + b2) - qdotbsq * (2.0 * wg + bsq);
+    const double t3b = wsq * qb;
+    const double t3c = w3 + wsq * (bq - pp) - q2b;
+    const bool up = t3a <= t3b;
+    go = go && n < 100000 && (up || t3c > 0.0);
+    const double next = fabs((up ? 1.5 : (double)0.9f) * wg);
+    wg = go ? next : wg;
+    n += go;
+    return go;
+  };
+  if (trip(true)) {
+    bool go = true;
+    while (go) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) go = trip(go);
+    }
+  }
+  return n >= 100000;
+}
+
 struct RecovOut { double w[9]; int fallback, fail, negrho, negp, vsqgt1, det0, guard, indep; };
 
 template <class MT>
@@ -814,18 +848,8 @@ RH_DEV void recov_cell(const double u[9], const double wold[9], const MT& M, dou
   else if (wgm >= 0.0) wg = wgm;
   else carry = true;
   double pp = 0.0, ro = 0.0;
-  // recov.f90:823-850 ("goto 95"); bounded here, bound hits are counted
-  int guard = 0;
-  for (; guard < 100000; guard++) {
-    pp = gam2 * (wg * gf - dro * sqrt(gf));
-    const double t3a = (wg * wg * wg) * (wg + 2.0 * bsq) - qdotbsq * (2.0 * wg + bsq);
-    const double t3b = (wg * wg) * (qtsq - bsq * bsq);
-    const double t3c = (wg * wg * wg) + (wg * wg) * (0.5 * bsq + qdotn - pp) - 0.5 * qdotbsq;
-    if (t3a <= t3b) { wg = fabs(1.5 * wg); continue; }
-    if (t3c > 0.0) { wg = fabs((double)0.9f * wg); continue; }
-    break;
-  }
-  if (guard >= 100000) o.guard = 1;
+  // recov.f90:823-850 ("goto 95")
+  if (admissible_w(wg, gf, dro * sqrt(gf), gam2, bsq, qtsq, qdotn, qdotbsq)) o.guard = 1;
   double wsq = wg * wg;
   const double xsq = (bsq + wg) * (bsq + wg);
   vsq = fabs((wsq * qtsq + qdotbsq * (bsq + 2.0 * wg)) * (1.0 / (wsq * xsq)));
@@ -1042,18 +1066,8 @@ RH_DEV void recov2_cell(const double u[9], const double wold[9], const MT& M, do
   else if (wgm >= 0.0) wg = wgm;
   else carry = true;
   double pp = 0.0, ro = 0.0;
-  // recov.f90:2150-2172 ("goto 95"); bounded here, bound hits are counted
-  int guard = 0;
-  for (; guard < 100000; guard++) {
-    pp = gam2 * (wg * gf - dro * sqrt(gf));
-    const double t3a = (wg * wg * wg) * (wg + 2.0 * bsq) - qdotbsq * (2.0 * wg + bsq);
-    const double t3b = (wg * wg) * (qtsq - bsq * bsq);
-    const double t3c = (wg * wg * wg) + (wg * wg) * (0.5 * bsq + qdotn - pp) - 0.5 * qdotbsq;
-    if (t3a <= t3b) { wg = fabs(1.5 * wg); continue; }
-    if (t3c > 0.0) { wg = fabs((double)0.9f * wg); continue; }
-    break;
-  }
-  if (guard >= 100000) o.guard = 1;
+  // recov.f90:2150-2172 ("goto 95")
+  if (admissible_w(wg, gf, dro * sqrt(gf), gam2, bsq, qtsq, qdotn, qdotbsq)) o.guard = 1;
   double wgd = wg - dro;
   double xxn = wgd;
   // Newton-Raphson on W' (recov.f90:2180-2300); a trip is a function of xxn
