@@ -335,41 +335,14 @@ RH_DEV void b_ppm_edges(const Geo& G, const EdgeArgs& A, unsigned blk) {
   }
 }
 
-// MC-limited linear reconstruction of every cell along D (mclim,
-// rec.f90:208-367, irec=1): slopes to both neighbours over the centre
-// distances (+1e-12), the MC limiter, edges at the cell's faces; stored like
-// the PPM edges.  A.pc holds the face positions x*a of the direction.
-template <int D, class R>
-RH_DEV void b_mc_edges(const Geo& G, const EdgeArgs& A, unsigned blk) {
-  const double* __restrict__ W = A.W;
-  const double* __restrict__ xs = A.xs;
-  const double* __restrict__ xa = A.pc;
-  R* __restrict__ E = (R*)A.E;
-  int i, j, k;
-  const unsigned t = blk * blockDim.x + threadIdx.x;
-  const int hi = G.ni - G.nm0 + (D == 1), hj = jhi(G, G.nj - G.nm0 + (D == 2)), hk = G.nk - G.nm0 + (D == 3);
-  const int lj = jlo(G, G.nm0);
-  const bool in = (D == 3) ? box_index_ikj(t, G.nm0, hi, lj, hj, G.nm0, hk, i, j, k)
-                           : box_index(t, G.nm0, hi, lj, hj, G.nm0, hk, i, j, k);
-  if (!in) return;
-  const long long N = G.N;
-  const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
-  const unsigned c = cidx(i, j, k, G);
-  const int p = (D == 1) ? i : (D == 2) ? j : k;
-  const R small = R(1.0e-12);
-  const R xp = R(xs[p]), xc = R(xs[p - 1]), xm = R(xs[p - 2]), xap = R(xa[p - 1]), xam = R(xa[p - 2]);
-  const R ip = R(1) / (xp - xc + small), im = R(1) / (xc - xm + small);
-#pragma unroll 3
-  for (int n = 0; n < 9; n++) {
-    const double* Pn = W + (long long)n * N + c;
-    const R u = R(Pn[0]), up = R(Pn[s]), um = R(Pn[-s]);
-    const R sp = (up - u) * ip;
-    const R sm = (u - um) * im;
-    const R tmp = (sp < R(0)) ? R(-1) : R(1);
-    const R dk = tmp * fmaxf_(R(0), fminf_(fminf_(R(2) * absr(sp), tmp * R(2) * sm), tmp * R(0.5) * (sp + sm)));
-    E[(long long)n * N + c - s] = u - dk * (xc - xam);   // left edge, at the interface c-1/2
-    E[(long long)(9 + n) * N + c] = u + dk * (xap - xc); // right edge
-  }
+// MC-limited slope of a cell (mclim, rec.f90:208-367, irec=1) from its
+// neighbours; im, ip: 1 / (distance to them + 1e-12).
+template <class R>
+RH_DEV R mc_slope(R um, R u, R up, R im, R ip) {
+  const R sp = (up - u) * ip;
+  const R sm = (u - um) * im;
+  const R tmp = (sp < R(0)) ? R(-1) : R(1);
+  return tmp * fmaxf_(R(0), fminf_(fminf_(R(2) * absr(sp), tmp * R(2) * sm), tmp * R(0.5) * (sp + sm)));
 }
 
 // Face physics and HLLE of interface c+1/2 along D from its two face states
@@ -445,7 +418,10 @@ RH_DEV void sweep_face(const Geo& G, R* __restrict__ F, R* __restrict__ CTsrc, u
 // also go to their plane of CTsrc (the copies ct.f90:54-67 takes before
 // averaging); inside the CT box fluxct then writes F itself.
 //
-// PPM's face values come from k_ppm_edges (E); MP5 and WENO5 reconstruct here.
+// PPM's face values come from k_ppm_edges (E); MC, MP5 and WENO5 reconstruct
+// here.  (MC from its four cells: with the face values of every cell through
+// HBM from a kernel of their own, as PPM's, 151x50x83 took 0.195 ms for a
+// stage's edges and sweeps, now 0.127.)
 template <int D, int IREC, class R, int ICHA, bool MK>
 RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, unsigned blk) {
   const double* __restrict__ W = A.W;
@@ -456,11 +432,11 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, unsigned blk) {
   int i, j, k;
   const unsigned t = blk * blockDim.x + threadIdx.x;
   const int lj = jlo(G, G.nm0), hj = jhi(G, G.nj - G.nm0);
-  // k sweeps that read a stencil along k (MP5, WENO5) walk k before j so
+  // k sweeps that read a stencil along k (MC, MP5, WENO5) walk k before j so
   // neighbouring workgroups share the stencil planes in L2; with the face
-  // values precomputed (PPM, MC) the i,j,k walk keeps each (i,k) metric
-  // entry in L2 across the j rows instead.
-  constexpr bool kfirst = D == 3 && (IREC == 6 || IREC == 7);
+  // values precomputed (PPM) the i,j,k walk keeps each (i,k) metric entry in
+  // L2 across the j rows instead.
+  constexpr bool kfirst = D == 3 && IREC != 5;
   const bool in = kfirst ? box_index_ikj(t, G.nm0, G.ni - G.nm0, lj, hj, G.nm0, G.nk - G.nm0, i, j, k)
                          : box_index(t, G.nm0, G.ni - G.nm0, lj, hj, G.nm0, G.nk - G.nm0, i, j, k);
   if (!in) return;
@@ -468,13 +444,26 @@ RH_DEV void b_sweep(const Geo& G, const SweepArgs& A, unsigned blk) {
   const long long s = (D == 1) ? 1LL : (D == 2) ? jstride(G) : kstride(G);
   const unsigned c = cidx(i, j, k, G);
   R wl[9], wr[9];
-  if (IREC == 5 || IREC == 1) {
+  if (IREC == 5) {
     // right edge of cell c (uri*l(c)) and left edge of cell c+1 (uri*r(c)),
     // both stored at interface c+1/2's index
 #pragma unroll
     for (int n = 0; n < 9; n++) {
       wl[n] = ld_(E + (long long)(9 + n) * N, c * (unsigned)sizeof(R));
       wr[n] = ld_(E + (long long)n * N, c * (unsigned)sizeof(R));
+    }
+  } else if (IREC == 1) {
+    const unsigned c8 = c * 8u;
+    const int p = (D == 1) ? i : (D == 2) ? j : k;
+    const R small = R(1.0e-12);
+    const R xm = R(A.xs[p - 2]), x0 = R(A.xs[p - 1]), x1 = R(A.xs[p]), x2 = R(A.xs[p + 1]), xf = R(A.xa[p - 1]);
+    const R i0 = R(1) / (x0 - xm + small), i1 = R(1) / (x1 - x0 + small), i2 = R(1) / (x2 - x1 + small);
+#pragma unroll
+    for (int n = 0; n < 9; n++) {
+      const double* Pn = W + (long long)n * N;
+      const R a = R(ld_(Pn - s, c8)), b = R(ld_(Pn, c8)), d = R(ld_(Pn + s, c8)), e = R(ld_(Pn + 2 * s, c8));
+      wl[n] = b + mc_slope<R>(a, b, d, i0, i1) * (xf - x0);
+      wr[n] = d - mc_slope<R>(b, d, e, i1, i2) * (x1 - xf);
     }
   } else {
     const unsigned c8 = c * 8u;
@@ -2120,11 +2109,8 @@ RH_DEV void b_copy(const CopyArgs& A, unsigned blk) {
 
 template <int D, class R>
 __global__ void __launch_bounds__(256) k_ppm_edges(Geo G, EdgeArgs A) { b_ppm_edges<D, R>(G, A, xcd_block()); }
-template <int D, class R>
-__global__ void __launch_bounds__(256) k_mc_edges(Geo G, EdgeArgs A) { b_mc_edges<D, R>(G, A, xcd_block()); }
-// the sweeps over precomputed face values (PPM, MC) fit 3 waves per SIMD in
-// FP64 (168 VGPRs, against 170 and 2 waves unconstrained) and 5 in float (96);
-// MP5 and WENO5 are left to the compiler
+// the PPM and MC sweeps fit 3 waves per SIMD in FP64 (168 VGPRs) and 5 in
+// float (96); MP5 and WENO5 are left to the compiler
 template <class R, int IREC>
 constexpr int sweep_waves = (IREC == 5 || IREC == 1) ? (sizeof(R) == 4 ? 5 : 3) : 1;
 template <int D, int IREC, class R, int ICHA, bool MK>
@@ -2187,12 +2173,6 @@ __global__ void __launch_bounds__(256) kb_ppm_edges(const BatchItem* __restrict_
   RH_BATCH_PROLOGUE
   const EdgeArgs A = it[q].A.e;
   b_ppm_edges<D, R>(G, A, blk);
-}
-template <int D, class R>
-__global__ void __launch_bounds__(256) kb_mc_edges(const BatchItem* __restrict__ it, int n) {
-  RH_BATCH_PROLOGUE
-  const EdgeArgs A = it[q].A.e;
-  b_mc_edges<D, R>(G, A, blk);
 }
 template <int D, int IREC, class R, int ICHA, bool MK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, IREC>)))
@@ -2307,27 +2287,25 @@ int block_threads(int kind) {
 
 bool one_group_per_model(int kind) { return kind == LK_CARRY || kind == LK_CFL_FINISH; }
 
-hipError_t launch_edges(const Geo& G, int dir, int irec, const double* W, const double* dxs, const double* xs,
-                        const double* tab, double gam, void* E, bool mixed, hipStream_t st) {
+hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dxs, const double* xs,
+                        const double* pc, double gam, void* E, bool mixed, hipStream_t st) {
   const long long ci = box(G.nm0, G.ni - G.nm0 + (dir == 1));
-  // PPM along j and k: whole 64-lane rows (box_index_wave)
-  const long long ciw = (irec == 5 && dir != 1) ? 64 * ((ci + 63) / 64) : ci;
+  // along j and k: whole 64-lane rows (box_index_wave)
+  const long long ciw = dir != 1 ? 64 * ((ci + 63) / 64) : ci;
   const long long n = ciw * jbox(G, G.nm0, G.nj - G.nm0 + (dir == 2)) * box(G.nm0, G.nk - G.nm0 + (dir == 3));
-  EdgeArgs A{W, dxs, xs, tab, gam, E};
+  EdgeArgs A{W, dxs, xs, pc, gam, E};
   const int bt = slot_threads(G, TS_EDGES);
   const unsigned nb = nblk(n, bt);
-  const bool mc = irec == 1;
   if (g_rec) {
     AnyArgs a{};
     a.e = A;
-    record(LK_EDGES, dir + 4 * (int)mixed + 16 * (int)mc, bt, nb, G, a);
+    record(LK_EDGES, dir + 4 * (int)mixed, bt, nb, G, a);
     return hipSuccess;
   }
   if (n == 0) return hipSuccess;
-#define L(K, Dd, T) hipLaunchKernelGGL((K<Dd, T>), dim3(nb), dim3(bt), 0, st, G, A)
-#define LD(K, T) do { if (dir == 1) L(K, 1, T); else if (dir == 2) L(K, 2, T); else L(K, 3, T); } while (0)
-  if (mc) { if (mixed) LD(k_mc_edges, float); else LD(k_mc_edges, double); }
-  else { if (mixed) LD(k_ppm_edges, float); else LD(k_ppm_edges, double); }
+#define L(Dd, T) hipLaunchKernelGGL((k_ppm_edges<Dd, T>), dim3(nb), dim3(bt), 0, st, G, A)
+#define LD(T) do { if (dir == 1) L(1, T); else if (dir == 2) L(2, T); else L(3, T); } while (0)
+  if (mixed) LD(float); else LD(double);
 #undef LD
 #undef L
   return hipGetLastError();
@@ -2412,9 +2390,10 @@ static void with_sweep(int variant, F&& f) {
 }
 
 hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
-                        double gam, void* F, void* CTsrc, bool mixed, hipStream_t st) {
+                        const double* xs, const double* xa, double gam, void* F, void* CTsrc, bool mixed,
+                        hipStream_t st) {
   const long long n = box(G.nm0, G.ni - G.nm0) * jbox(G, G.nm0, G.nj - G.nm0) * box(G.nm0, G.nk - G.nm0);
-  SweepArgs A{W, metF, E, gam, F, CTsrc};
+  SweepArgs A{W, metF, E, xs, xa, gam, F, CTsrc};
   const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
   const unsigned nb = nblk(n, bt);
   if (g_rec) {
@@ -2758,11 +2737,9 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
   switch (kind) {
     case LK_EDGES: {
       const int d = variant & 3;
-      const bool mx = (variant & 4) != 0, mc = (variant & 16) != 0;
-#define L(K, Dd, T) hipLaunchKernelGGL((K<Dd, T>), g, b, 0, st, it, n)
-#define LD(K, T) do { if (d == 1) L(K, 1, T); else if (d == 2) L(K, 2, T); else L(K, 3, T); } while (0)
-      if (mc) { if (mx) LD(kb_mc_edges, float); else LD(kb_mc_edges, double); }
-      else { if (mx) LD(kb_ppm_edges, float); else LD(kb_ppm_edges, double); }
+#define L(Dd, T) hipLaunchKernelGGL((kb_ppm_edges<Dd, T>), g, b, 0, st, it, n)
+#define LD(T) do { if (d == 1) L(1, T); else if (d == 2) L(2, T); else L(3, T); } while (0)
+      if (variant & 4) LD(float); else LD(double);
 #undef LD
 #undef L
       break;

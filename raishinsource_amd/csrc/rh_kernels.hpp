@@ -74,7 +74,7 @@ struct FixArgs {
 };
 
 struct EdgeArgs {
-  const double *W, *dxs, *xs, *pc;  // pc: PPM width coefficients, or the face positions x*a for MC
+  const double *W, *dxs, *xs, *pc;  // pc: PPM width coefficients
   double gam;
   void *E;                         // float or double planes, by the launch's variant
 };
@@ -82,7 +82,8 @@ struct EdgeArgs {
 struct SweepArgs {
   const double *W;
   const void *metF;                // face metric tables: doubles, or (compact and mixed) floats
-  const void *E;
+  const void *E;                   // PPM's face values (split form)
+  const double *xs, *xa;           // MC: cell and face positions along the sweep
   double gam;
   void *F, *CTsrc;  // element type: the sweep's arithmetic type (double, or float when mixed)
 };
@@ -178,18 +179,17 @@ int block_threads(int kind);
 hipError_t launch_gather_first(const double* const* src, double* dst, int n, hipStream_t st);
 bool one_group_per_model(int kind);
 
-// Face values of every cell along dir into E (18 planes: left edges, right
-// edges): PPM (irec 5; tab = the width-only interp coefficients of the
-// direction, 7 planes of n+2, ppm_coefficients) or the MC limiter (irec 1;
-// tab = the face positions x*a).  mixed: the reconstruction and the face
-// arithmetic in float (E holds floats), else double.
-hipError_t launch_edges(const Geo& G, int dir, int irec, const double* W, const double* dxs, const double* xs,
-                        const double* tab, double gam, void* E, bool mixed, hipStream_t st);
+// PPM face values of every cell along dir into E (18 planes: left edges, right
+// edges); pc = the width-only interp coefficients of the direction, 7 planes
+// of n+2 (ppm_coefficients).  mixed: the reconstruction in float (E holds
+// floats), else double.
+hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dxs, const double* xs,
+                        const double* pc, double gam, void* E, bool mixed, hipStream_t st);
 // Fluxes at the interfaces along dir; E = the PPM edges (irec 5), unused otherwise.
 // F and CTsrc take doubles, or floats when mixed (every value the float
 // arithmetic produced, so storing it in float loses nothing).
 hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
-                        double gam, void* F, void* CTsrc, bool mixed, hipStream_t st);
+                        const double* xs, const double* xa, double gam, void* F, void* CTsrc, bool mixed, hipStream_t st);
 // PPM (irec 5) sweep along dir with the face values computed in the same
 // kernel (through LDS): reads W and the direction's PPM width coefficients
 // pc, writes what launch_edges + launch_sweep write to F and CTsrc.

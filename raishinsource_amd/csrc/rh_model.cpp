@@ -257,7 +257,7 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
       !dalloc(&m->cfl_min, 4 * cfl_slots(G)))
     return false;
   if (m->need_wo && !dalloc(&m->Wo, 9 * N)) return false;
-  if ((p->irec == 5 || p->irec == 1) && !dalloc(&m->E, 18 * N)) return false;  // face values
+  if (p->irec == 5 && !dalloc(&m->E, 18 * N)) return false;  // face values of the split form
   if (!dalloc(&m->stage_aos, 9 * N)) return false;            // set_state / get_state staging
   m->crows = ((N + 255) / 256) * 4;  // wavefronts of the largest launch (every cell, 256 per workgroup)
   if (!dalloc(&m->cpart, (size_t)m->crows * NCOUNT)) return false;
@@ -521,14 +521,13 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* c
       HIPCHK(launch_psweep(G, d, ps(d), m->mixed, m->st));
       continue;
     }
-    if (irec == 5 || irec == 1) {
+    if (irec == 5) {
       TimedLaunch t(m, K_EDGES);
-      const double* tab = irec == 5 ? m->ppmc[d - 1] : m->xa[d - 1];
-      HIPCHK(launch_edges(G, d, irec, W, m->dxs[d - 1], m->xs[d - 1], tab, m->p.gam, m->E, m->mixed, m->st));
+      HIPCHK(launch_edges(G, d, W, m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam, m->E, m->mixed, m->st));
     }
     TimedLaunch t(m, K_SWEEP1 + d - 1);
-    HIPCHK(launch_sweep(G, d, irec, W, m->metric_face(d), m->E, m->p.gam, flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed,
-                        m->st));
+    HIPCHK(launch_sweep(G, d, irec, W, m->metric_face(d), m->E, m->xs[d - 1], m->xa[d - 1], m->p.gam,
+                        flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed, m->st));
   }
   return true;
 }
