@@ -2445,13 +2445,13 @@ static void psweep_extent(const Geo& G, int dir, long long& along, long long& li
 //  rows, whichever leaves the fewest idle or overlapping lanes.
 //  D = 2, 3: a wave holds seg cells along the axis by 64 / seg consecutive i
 //  and the workgroup's waves are stacked along the axis.  seg as set by the
-//  caller, else the one with the fewest such lanes among runs of at least 4
-//  consecutive i along j and 16 along k (along j a tile's cells share their
-//  face metric; along k every (i, k) has its own, 33 values read in runs of
-//  64 / seg: 256x128x128 at seg 4, 8, 16 0.374, 0.377, 0.329 ms along j and
-//  0.396, 0.446, 0.444 ms along k); never taller than the axis needs (Riemann
-//  tubes' four transverse interfaces), never below the 4 cells that give an
-//  interface.
+//  caller, else along j the one with the fewest such lanes among 2 to 16, and
+//  along k 4, or 8 where that has fewer: along j a tile's cells share their
+//  face metric, along k every (i, k) has its own, read in runs of 64 / seg
+//  (seg 4, 8, 16: 256x128x128 0.373, 0.406, 0.370 ms, mixed 0.202, 0.242,
+//  0.250; 64^3, fewer lanes at 8, 28.0, 25.7, 26.1 us; 251x57x77 89, 90, 119
+//  us).  Never taller than the axis needs (Riemann tubes' four transverse
+//  interfaces), never below the 4 cells that give an interface.
 static int psweep_tp(const Geo& G, int dir, int bt) {
   long long along, lines, across;
   psweep_extent(G, dir, along, lines, across);
@@ -2469,7 +2469,7 @@ static int psweep_tp(const Geo& G, int dir, int bt) {
   if (!seg) {
     seg = dir == 2 ? 16 : 4;
     for (int sg : {8, 4, 2})
-      if (sg < seg && sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
+      if ((dir == 2 || sg > 2) && sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
   }
   while (seg > 1 && seg * nw / 2 >= 4 && seg * nw / 2 - 3 >= along) seg /= 2;
   while (seg * nw < 4) seg *= 2;
