@@ -2141,6 +2141,21 @@ RH_DEV void b_psweep3(const Geo& G, const PSweep3Args& A, unsigned blk) {
   else if (blk < A.end[2]) { if (part(2, b)) b_psweep<3, R, ICHA, MK>(G, A.s[2], b); }
   else if (blk - A.end[2] < (unsigned)A.cfl.nblocks) b_cfl<ICHA, MK>(G, A.cfl, blk - A.end[2]);
 }
+// The same for the other reconstructions (a model alone, compact metric tables).
+template <int IREC, class R, int ICHA>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, IREC>)))
+k_sweep3(Geo G, Sweep3Args A) {
+  const unsigned part = blockIdx.x / A.each, b = blockIdx.x - part * A.each;
+  if (part >= 3) {
+    b_cfl<ICHA, true>(G, A.cfl, blockIdx.x - 3 * A.each);
+    return;
+  }
+  if (b >= A.n) return;
+  const unsigned blk = xcd_renumber(A.n, b);
+  if (part == 0) b_sweep<1, IREC, R, ICHA, true>(G, A.s[0], blk);
+  else if (part == 1) b_sweep<2, IREC, R, ICHA, true>(G, A.s[1], blk);
+  else b_sweep<3, IREC, R, ICHA, true>(G, A.s[2], blk);
+}
 template <class R, int ICHA, bool MK, bool COLL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
 k_psweep3(Geo G, PSweep3Args A) { b_psweep3<R, ICHA, MK, COLL>(G, A, blockIdx.x); }
@@ -2389,11 +2404,8 @@ static void with_sweep(int variant, F&& f) {
   });
 }
 
-hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
-                        const double* xs, const double* xa, double gam, void* F, void* CTsrc, bool mixed,
-                        hipStream_t st) {
+hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, bool mixed, hipStream_t st) {
   const long long n = box(G.nm0, G.ni - G.nm0) * jbox(G, G.nm0, G.nj - G.nm0) * box(G.nm0, G.nk - G.nm0);
-  SweepArgs A{W, metF, E, xs, xa, gam, F, CTsrc};
   const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
   const unsigned nb = nblk(n, bt);
   if (g_rec) {
@@ -2551,6 +2563,32 @@ static void with_psweep3(int variant, F&& f) {
       else f(TypeTag<double>{}, C, K, L);
     });
   });
+}
+
+bool sweeps_one_launch(const Geo& G, int irec) { return irec == 5 ? !G.ppm_split : G.mk && !g_rec; }
+
+hipError_t launch_sweep3(const Geo& G, int irec, const SweepArgs s[3], bool mixed, const CflArgs* cfl,
+                         hipStream_t st) {
+  const long long n = box(G.nm0, G.ni - G.nm0) * jbox(G, G.nm0, G.nj - G.nm0) * box(G.nm0, G.nk - G.nm0);
+  const int bt = slot_threads(G, TS_SWEEP1);
+  Sweep3Args A{{s[0], s[1], s[2]}, nblk(n, bt), 0, CflArgs{}};
+  A.each = (A.n + 7u) & ~7u;
+  if (A.n == 0) A.each = 8;
+  unsigned nb = 3 * A.each;
+  if (cfl) {
+    A.cfl = *cfl;
+    nb += cfl_groups(G, bt, A.cfl);
+  }
+  with_icha(G.icha, true, [&](auto C, auto) {
+    auto t = [&](auto I) {
+      if (mixed) hipLaunchKernelGGL((k_sweep3<I.value, float, C.value>), dim3(nb), dim3(bt), 0, st, G, A);
+      else hipLaunchKernelGGL((k_sweep3<I.value, double, C.value>), dim3(nb), dim3(bt), 0, st, G, A);
+    };
+    if (irec == 1) t(IC<1>{});
+    else if (irec == 6) t(IC<6>{});
+    else t(IC<7>{});
+  });
+  return hipGetLastError();
 }
 
 hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st) {

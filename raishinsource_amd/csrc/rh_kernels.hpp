@@ -108,6 +108,14 @@ struct PSweep3Args {
   CflArgs cfl;
 };
 
+// The same of the other reconstructions: n workgroups of each sweep, a part
+// every `each` (a multiple of 8).
+struct Sweep3Args {
+  SweepArgs s[3];
+  unsigned n, each;
+  CflArgs cfl;
+};
+
 struct CtArgs {
   const void* CTsrc;  // double, or float when mixed (as the sweeps wrote them)
   void *F1, *F2, *F3;
@@ -188,8 +196,7 @@ hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dx
 // Fluxes at the interfaces along dir; E = the PPM edges (irec 5), unused otherwise.
 // F and CTsrc take doubles, or floats when mixed (every value the float
 // arithmetic produced, so storing it in float loses nothing).
-hipError_t launch_sweep(const Geo& G, int dir, int irec, const double* W, const void* metF, const void* E,
-                        const double* xs, const double* xa, double gam, void* F, void* CTsrc, bool mixed, hipStream_t st);
+hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, bool mixed, hipStream_t st);
 // PPM (irec 5) sweep along dir with the face values computed in the same
 // kernel (through LDS): reads W and the direction's PPM width coefficients
 // pc, writes what launch_edges + launch_sweep write to F and CTsrc.
@@ -201,6 +208,11 @@ hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A, bool mixed,
 // The three in one launch (s[d]: the sweep along d + 1), with the CFL
 // reduction of the same primitives when cfl is given; its workgroups' results
 // are then combined by the launch_fluxct that is given the same cfl.
+// Whether a stage's sweeps go in one launch: PPM's (not the split form's)
+// always, the others' where that is built (compact metric tables, no batch).
+bool sweeps_one_launch(const Geo& G, int irec);
+hipError_t launch_sweep3(const Geo& G, int irec, const SweepArgs s[3], bool mixed, const CflArgs* cfl,
+                         hipStream_t st);
 hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st);
 int psweep_segment(const Geo& G, int dir);
 size_t psweep_lds_bytes(int threads, bool mixed);

@@ -494,11 +494,11 @@ static CflArgs cfl_args(raishin_model* m, const double* W, bool advance) {
   return C;
 }
 
-// The three PPM sweeps go in one launch (with the step's CFL reduction),
-// except where the kernels are timed one by one.
+// The three sweeps go in one launch (with the step's CFL reduction) where
+// that is built, except where the kernels are timed one by one.
 static bool sweeps_merged(const raishin_model* m) {
   constexpr unsigned timed = 1u << K_SWEEP1 | 1u << K_SWEEP2 | 1u << K_SWEEP3 | 1u << K_FLUXCT | 1u << K_CFL;
-  return m->p.irec == 5 && !m->G.ppm_split && !(m->timing & timed);
+  return sweeps_one_launch(m->G, m->p.irec) && !(m->timing & timed);
 }
 
 bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* cfl) {
@@ -510,9 +510,20 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* c
     A.gam = m->p.gam; A.F = flux_plane(m, F, (d - 1) * 9); A.CTsrc = m->CT;
     return A;
   };
+  auto sw = [&](int d) {
+    SweepArgs A{};
+    A.W = W; A.metF = m->metric_face(d); A.E = m->E; A.xs = m->xs[d - 1]; A.xa = m->xa[d - 1];
+    A.gam = m->p.gam; A.F = flux_plane(m, F, (d - 1) * 9); A.CTsrc = m->CT;
+    return A;
+  };
   if (sweeps_merged(m)) {
-    const PSweepArgs s[3] = {ps(1), ps(2), ps(3)};
-    HIPCHK(launch_psweep3(G, s, m->mixed, cfl, m->st));
+    if (irec == 5) {
+      const PSweepArgs s[3] = {ps(1), ps(2), ps(3)};
+      HIPCHK(launch_psweep3(G, s, m->mixed, cfl, m->st));
+    } else {
+      const SweepArgs s[3] = {sw(1), sw(2), sw(3)};
+      HIPCHK(launch_sweep3(G, irec, s, m->mixed, cfl, m->st));
+    }
     return true;
   }
   for (int d = 1; d <= 3; d++) {
@@ -526,8 +537,7 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* c
       HIPCHK(launch_edges(G, d, W, m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam, m->E, m->mixed, m->st));
     }
     TimedLaunch t(m, K_SWEEP1 + d - 1);
-    HIPCHK(launch_sweep(G, d, irec, W, m->metric_face(d), m->E, m->xs[d - 1], m->xa[d - 1], m->p.gam,
-                        flux_plane(m, F, (d - 1) * 9), m->CT, m->mixed, m->st));
+    HIPCHK(launch_sweep(G, d, irec, sw(d), m->mixed, m->st));
   }
   return true;
 }

@@ -146,3 +146,25 @@ def test_one_launch_equals_separate(name, mixed, threads):
     same(a, b, name)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("name,mixed,threads", [("umc", False, 64), ("uleis", True, 256), ("ump5", False, 128),
+                                                ("uweno", False, 256), ("t2dmc", False, 192)])
+def test_one_launch_of_other_sweeps(name, mixed, threads):
+    """As test_one_launch_equals_separate for MC, MP5 and WENO5, against the
+    same model in a batch too (a launch per sweep there)."""
+    a, b, c = (make(configs.ALL[name], mixed) for _ in range(3))
+    for mm in (a, b, c):
+        mm.set_block_sizes([threads] * 8)
+    b.set_timing(True)
+    batch = native.Batch([c])
+    for s in range(2):
+        assert np.array_equal(a.step(1), b.step(1), equal_nan=True), s
+    batch.step(2)
+    assert b.get_timing()["sweep_k"][1] > 0 and b.get_timing()["cfl"][1] == 2
+    same(a, b, name)
+    same(a, c, name)
+    batch.set([])
+    batch.close()
+    for mm in (a, b, c):
+        mm.close()
