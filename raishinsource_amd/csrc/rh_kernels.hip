@@ -2458,11 +2458,12 @@ static void psweep_extent(const Geo& G, int dir, long long& along, long long& li
 //  D = 2, 3: a wave holds seg cells along the axis by 64 / seg consecutive i
 //  and the workgroup's waves are stacked along the axis.  seg as set by the
 //  caller, else along j the one with the fewest such lanes among 2 to 16, and
-//  along k 4, or 8 where that has fewer: along j a tile's cells share their
-//  face metric, along k every (i, k) has its own, read in runs of 64 / seg
-//  (seg 4, 8, 16: 256x128x128 0.373, 0.406, 0.370 ms, mixed 0.202, 0.242,
-//  0.250; 64^3, fewer lanes at 8, 28.0, 25.7, 26.1 us; 251x57x77 89, 90, 119
-//  us).  Never taller than the axis needs (Riemann tubes' four transverse
+//  along k 4, or 8 where that has fewer and still two waves per SIMD (1024 of
+//  them): along j a tile's cells share their face metric, along k every (i, k)
+//  has its own, read in runs of 64 / seg (seg 4, 8, 16: 256x128x128 0.373,
+//  0.406, 0.370 ms, mixed 0.202, 0.242, 0.250; 64^3, fewer lanes at 8, 28.0,
+//  25.7, 26.1 us; 251x57x77 89, 90, 119 us; one 64x64 row, with half the
+//  workgroups at 8, 12.4, 16.7, 13.4 us).  Never taller than the axis needs (Riemann tubes' four transverse
 //  interfaces), never below the 4 cells that give an interface.
 static int psweep_tp(const Geo& G, int dir, int bt) {
   long long along, lines, across;
@@ -2479,9 +2480,14 @@ static int psweep_tp(const Geo& G, int dir, int bt) {
   const int nw = bt / 64;
   int seg = G.seg[dir - 2];
   if (!seg) {
-    seg = dir == 2 ? 16 : 4;
-    for (int sg : {8, 4, 2})
-      if ((dir == 2 || sg > 2) && sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
+    if (dir == 2) {
+      seg = 16;
+      for (int sg : {8, 4, 2})
+        if (sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
+    } else {
+      const long long l4 = lanes(4 * nw, 16), l8 = lanes(8 * nw, 8);
+      seg = l8 < l4 && l8 * across >= 2 * 64 * 1024 ? 8 : 4;
+    }
   }
   while (seg > 1 && seg * nw / 2 >= 4 && seg * nw / 2 - 3 >= along) seg /= 2;
   while (seg * nw < 4) seg *= 2;
