@@ -41,11 +41,12 @@ def algorithmic_bytes(p, kind):
              (i,k)).
     ppm_edges: per cell and direction, read the 9 primitive planes, write
              18 edge planes (all three directions per launch kind).
-    update:  read W, U (one RK input at stage 1, two after), 3x9 fluxes;
-             write the 9 RK-result planes; centre metric + Christoffel tables
+    update:  (with the recovery) read W, U (one RK input at stage 1, two
+             after), 3x9 fluxes; write the 9 recovered planes and the final W
+             of the Newton iteration; centre metric + Christoffel tables
              (97 doubles per (i,k)).
-    recov:   read the RK result and W, write 9 recovered planes and the
-             final W of the Newton iteration; centre metric table.
+    recov:   (in a kernel of its own) read the RK result and W, write 9
+             recovered planes and the final W; centre metric table.
     post:    read 9 recovered planes, write 9 primitive + 9 conserved
              planes per cell, centre metric table.
     """
@@ -60,7 +61,7 @@ def algorithmic_bytes(p, kind):
         return units, 216.0 * units, "cells"
     if kind == "update":
         units = (ni - 2 * nm1) * (nj - 2 * nm1) * (nk - 2 * nm1)
-        per = 72 + (72 if p.irkt == 2 else (72 + 2 * 144) / 3.0) + 216 + 72
+        per = 72 + (72 if p.irkt == 2 else (72 + 2 * 144) / 3.0) + 216 + 72 + 8
         return units, per * units + 776.0 * P2, "interior cells"
     if kind == "recov":
         units = (ni - 2 * nm1) * (nj - 2 * nm1) * (nk - 2 * nm1)

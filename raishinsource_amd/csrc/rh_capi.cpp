@@ -509,6 +509,8 @@ int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu
   double best_ms[TS_N];
   int best[TS_N];
   for (int q = 0; q < TS_N; q++) { best_ms[q] = 1e300; best[q] = 256; }
+  double best_sweeps = 1e300;  // the three sweeps go in one launch: one size for them
+  int sweeps = 256;
   const unsigned timing = m->timing;
   for (int cand : TUNE_CANDIDATES) {
     int bs[TS_N];
@@ -528,7 +530,10 @@ int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu
       const double avg = cnt[k] ? ms[k] / (double)cnt[k] : 1e300;
       if (avg < best_ms[q]) { best_ms[q] = avg; best[q] = cand; }
     }
+    const double sum = ms[K_SWEEP1] + ms[K_SWEEP2] + ms[K_SWEEP3];
+    if (cnt[K_SWEEP1] && sum < best_sweeps) { best_sweeps = sum; sweeps = cand; }
   }
+  best[TS_SWEEP1] = best[TS_SWEEP2] = best[TS_SWEEP3] = sweeps;
   if (raishin_model_set_block_sizes(m, best, TS_N) != 0) return -1;
   // PPM sweep tiles: the fused sweeps with each tile height along j and k,
   // the fastest per direction (the split form, slower at every measured

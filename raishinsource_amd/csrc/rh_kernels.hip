@@ -2494,10 +2494,11 @@ static int psweep_tp(const Geo& G, int dir, int bt) {
   return seg * nw;
 }
 
-// Cells along j or k that a wave of the sweep's tile holds.
+// Cells along j or k that a wave of the sweep's tile holds, as a size that can
+// be asked for: where the rule comes to one cell it comes there from two too.
 int psweep_segment(const Geo& G, int dir) {
   const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
-  return psweep_tp(G, dir, bt) / (bt / 64);
+  return std::max(2, psweep_tp(G, dir, bt) / (bt / 64));
 }
 
 size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads * (mixed ? sizeof(float) : sizeof(double)); }

@@ -168,3 +168,22 @@ def test_one_launch_of_other_sweeps(name, mixed, threads):
     batch.close()
     for mm in (a, b, c):
         mm.close()
+
+
+@pytest.mark.parametrize("threads", [64, 128, 192, 256])
+@pytest.mark.parametrize("name", ["t2d", "t3dppm", "uppm"])
+def test_tiles_read_back_can_be_set(name, threads):
+    """The tiles a model reports are ones another model of its shape takes,
+    and then has in use (a plan kept from an autotuned model)."""
+    p = configs.ALL[name].resolved()
+    g = native.setup_grid(p)
+    m = native.setup_metric(p, g)
+    a, b = native.Model(p, g, m), native.Model(p, g, m)
+    a.set_block_sizes([threads] * len(native.TUNE_SLOTS))
+    for seg in (0, 2, 64):
+        a.set_sweep_tiles(0, seg, seg)
+        plan = {**a.block_sizes(), **a.sweep_tiles()}
+        b.set_block_sizes(plan)
+        assert {**b.block_sizes(), **b.sweep_tiles()} == plan, seg
+    a.close()
+    b.close()
