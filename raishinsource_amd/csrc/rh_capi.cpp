@@ -450,12 +450,6 @@ int raishin_model_set_sweep_tiles(raishin_model* m, int split, int seg_j, int se
               "from 2 to 64");
     return -1;
   }
-  if (split && m->p.irec == 5 && !m->E) {
-    // the split form's face values: only a model that is asked for it holds them
-    const size_t n = 18 * (size_t)m->G.ni * m->G.nj * m->G.nk;
-    if (!dalloc(&m->E, n)) return -1;
-    m->dev_bytes += n * sizeof(double);
-  }
   m->G.ppm_split = (unsigned short)split;
   m->G.seg[0] = (unsigned short)seg_j;
   m->G.seg[1] = (unsigned short)seg_k;

@@ -257,6 +257,7 @@ static bool build_model_(raishin_model* m, const raishin_pram* p, const double* 
       !dalloc(&m->cfl_min, 4 * cfl_slots(G)))
     return false;
   if (m->need_wo && !dalloc(&m->Wo, 9 * N)) return false;
+  if (p->irec == 5 && !dalloc(&m->E, 18 * N)) return false;  // face values of the split form
   if (!dalloc(&m->stage_aos, 9 * N)) return false;            // set_state / get_state staging
   m->crows = ((N + 255) / 256) * 4;  // wavefronts of the largest launch (every cell, 256 per workgroup)
   if (!dalloc(&m->cpart, (size_t)m->crows * NCOUNT)) return false;

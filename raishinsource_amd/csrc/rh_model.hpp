@@ -41,7 +41,7 @@ struct raishin_model {
   double *Ucur = nullptr, *Uh = nullptr, *Us = nullptr, *Unext = nullptr;
   // F: ww(3,9,...) (27 planes); CT: the six transverse B flux copies ct.f90 averages
   double *F = nullptr, *CT = nullptr, *wgout = nullptr, *stage_aos = nullptr;
-  double* E = nullptr;  // PPM face values of one direction (18 planes; allocated when the split form is chosen)
+  double* E = nullptr;  // PPM face values of one direction (18 planes, the split form)
   double* ppmc[3] = {nullptr, nullptr, nullptr};  // PPM width coefficients per direction (irec = 5)
   // geometry
   double *met[4] = {nullptr, nullptr, nullptr, nullptr};  // centre, i-face, j-face, k-face

@@ -82,7 +82,7 @@ def footprint(p):
     need_wo = any(2 in getattr(p, a) for a in ("iboux1in", "iboux1ot", "iboux2in", "iboux2ot", "iboux3in",
                                                "iboux3ot"))
     ncfl = min(1024, max((max(ni - 2, 0) * max(nj - 2, 0) * max(nk - 2, 0) + 63) // 64, 1))
-    planes = 7 * 9 + 27 + 6 + 1 + 9 + (9 if need_wo else 0)
+    planes = 7 * 9 + 27 + 6 + 1 + 9 + (9 if need_wo else 0) + (18 if p.irec == 5 else 0)
     b = 8 * n * planes
     b += n + 8 * (2 + cap) + cap                     # cflag, carry count + list + counter, pend
     b += 8 * 64 * p2 + 2 * 8 * ni + 4 * 54 + 8 * 4 + 8 * 11 + 8 * 2
