@@ -155,6 +155,9 @@ void raishin_model_set_precision(raishin_model *m, int mode);
  * 0..2 direction sweeps i,j,k; 3 flux-CT; 4 RK update + sources;
  * 5 in-order recovery fix-up; 6 ghosts/floors/caluu1; 7 CFL reduction;
  * 8 PPM face values (irec=5, all three directions); 9 recov1a.
+ * Kind 4 includes the recovery where the step does both in one kernel (a
+ * symmetric metric); kind 9 then has no launches.  A step that times a sweep
+ * or the CFL reduction launches them apart, otherwise they share launches.
  * set_timing(1) clears the totals and starts recording; get_timing returns
  * the number of kinds and fills total milliseconds and launch counts. */
 void raishin_model_set_timing(raishin_model *m, int on);
@@ -178,8 +181,9 @@ int raishin_model_get_timing(raishin_model *m, double *ms, long long *launches, 
 
 /* Workgroup sizes of the tuned launches, in the order: PPM face values,
  * sweep i, sweep j, sweep k, flux-CT, RK update, recov1a, ghosts/floors/
- * caluu1 (8 entries; 0 = 256, else 64..256 in steps of 64).  Results do not
- * depend on them.  get returns the sizes in use. */
+ * caluu1 (8 entries; 0 = 256, else 64..256 in steps of 64).  Sweeps that share
+ * a launch take sweep i's.  Results do not depend on them.  get returns the
+ * sizes in use. */
 int raishin_model_set_block_sizes(raishin_model *m, const int *bs, int n);
 int raishin_model_get_block_sizes(raishin_model *m, int *bs, int n);
 /* Tiles of the PPM (irec = 5) sweeps.  split = 0 (default): each sweep
