@@ -2326,6 +2326,10 @@ hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dx
   return hipGetLastError();
 }
 
+void record_no_edges(const Geo& G) {
+  if (g_rec) record(LK_EDGES, 0, 256, 0, G, AnyArgs{});
+}
+
 // Sweep kernels are instantiated per (direction, reconstruction, arithmetic
 // type, wave-speed formula); the variant number packs the four so that batch
 // plans group launches of the same kernel:

@@ -193,6 +193,10 @@ bool one_group_per_model(int kind);
 // floats), else double.
 hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dxs, const double* xs,
                         const double* pc, double gam, void* E, bool mixed, hipStream_t st);
+// An empty launch_edges in a recorded step: MC has no such kernel, but its
+// batches share the sequence of launches of PPM's split form (and not that of
+// MP5 and WENO5).
+void record_no_edges(const Geo& G);
 // Fluxes at the interfaces along dir; E = the PPM edges (irec 5), unused otherwise.
 // F and CTsrc take doubles, or floats when mixed (every value the float
 // arithmetic produced, so storing it in float loses nothing).

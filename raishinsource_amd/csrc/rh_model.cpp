@@ -535,6 +535,8 @@ bool stage_sweeps(raishin_model* m, const double* W, double* F, const CflArgs* c
     if (irec == 5) {
       TimedLaunch t(m, K_EDGES);
       HIPCHK(launch_edges(G, d, W, m->dxs[d - 1], m->xs[d - 1], m->ppmc[d - 1], m->p.gam, m->E, m->mixed, m->st));
+    } else if (irec == 1) {
+      record_no_edges(G);
     }
     TimedLaunch t(m, K_SWEEP1 + d - 1);
     HIPCHK(launch_sweep(G, d, irec, sw(d), m->mixed, m->st));
