@@ -187,10 +187,11 @@ int raishin_model_get_timing(raishin_model *m, double *ms, long long *launches, 
 int raishin_model_set_block_sizes(raishin_model *m, const int *bs, int n);
 int raishin_model_get_block_sizes(raishin_model *m, int *bs, int n);
 /* Tiles of the PPM (irec = 5) sweeps.  split = 0 (default): each sweep
- * computes its face values itself, through LDS; a wave of the j (k) sweep
- * holds seg_j (seg_k) consecutive cells along j (k) by 64 / seg consecutive
- * i, a power of two from 2 to 64 (0: by rule), and a workgroup's waves are
- * stacked along the axis; a size the axis has no use for is reduced.  split = 1:
+ * computes its face values itself, through LDS; a workgroup of the j (k)
+ * sweep holds a tile of seg_j (seg_k) consecutive cells along j (k) by
+ * threads / seg consecutive i, a power of two from 2 to 64 (0: by rule; of 192
+ * threads three quarters as many); a size too small for an interface is
+ * raised, one the axis has no use for reduced.  split = 1:
  * the face values of every cell go through HBM from a kernel of their own.
  * Results do not depend on them.  0, or -1 with the error set. */
 int raishin_model_set_sweep_tiles(raishin_model *m, int split, int seg_j, int seg_k);
@@ -205,10 +206,12 @@ int raishin_model_get_sweep_tiles(raishin_model *m, int *split, int *seg_j, int 
 int raishin_model_set_divb_form(raishin_model *m, int form);
 /* Autotuner: for each candidate size (64, 128, 256) runs one warm-up step
  * and `steps` timed steps from the state (uri, uu or NULL, time), keeps the
- * fastest size per launch slot (one for the three sweeps, which go in one
- * launch); for PPM models it then times the fused
- * sweeps with tiles of 8, 16 and 32 cells along j and k and keeps the
- * fastest tile per direction (the split form is never chosen: it is slower
+ * fastest size per launch slot.  Where sweeps share a launch, the time of
+ * whole steps in a graph of two decides on that against the default sizes, on
+ * one size for the sweeps and, for PPM, on a tile of 8, 16, 32 or 64 cells
+ * along j and along k (where the axis fills three quarters of it): the
+ * defaults stay unless something is faster by
+ * more than 1% (the split form is never chosen: it is slower
  * at every size measured, and members of a batch must agree on the form);
  * then it sets the state again and clears the counters, so the run
  * starts as if untuned.  Returns 0 or -1. */

@@ -480,20 +480,36 @@ int raishin_model_get_sweep_tiles(raishin_model* m, int* split, int* seg_j, int*
 }
 
 namespace {
-// Milliseconds per step of each timed kind over `steps` steps from the state
-// (after one warm-up step); false on failure.
-bool time_kinds(raishin_model* m, const double* uri, const double* uu, double time, int steps, double* ms) {
-  raishin_model_set_state(m, uri, uu, time);
-  if (!run_step(m)) return false;
-  raishin_model_set_timing(m, 1);
-  for (int s = 0; s < steps; s++)
-    if (!run_step(m)) return false;
-  long long cnt[K_NKINDS];
-  raishin_model_get_timing(m, ms, cnt, K_NKINDS);
-  raishin_model_set_timing(m, 0);
-  for (int k = 0; k < K_NKINDS; k++) ms[k] /= steps;
-  return true;
+// Milliseconds a step from the state, launched as raishin_model_step_graph
+// launches it: the least of three runs of `steps` steps (rounded up to pairs)
+// after a pair that is not timed.  False on failure.
+bool time_steps(raishin_model* m, const double* uri, const double* uu, double time, int steps, double* ms) {
+  if (!model_set_state(m, uri, uu, time) || !graph_ready(m)) return false;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  auto go = [&]() -> bool {
+    for (auto& e : ev) HIPCHK(hipEventCreate(&e));
+    HIPCHK(hipGraphLaunch(m->gexec, m->st));
+    const int pairs = steps / 2 + steps % 2;
+    *ms = 1e300;
+    for (int r = 0; r < 3; r++) {
+      HIPCHK(hipEventRecord(ev[0], m->st));
+      for (int q = 0; q < pairs; q++) HIPCHK(hipGraphLaunch(m->gexec, m->st));
+      HIPCHK(hipEventRecord(ev[1], m->st));
+      HIPCHK(hipEventSynchronize(ev[1]));
+      float t = 0.0f;
+      HIPCHK(hipEventElapsedTime(&t, ev[0], ev[1]));
+      *ms = std::min(*ms, (double)t / (2 * pairs));
+    }
+    return true;
+  };
+  const bool ok = go();
+  for (auto e : ev)
+    if (e) (void)hipEventDestroy(e);
+  return ok;
 }
+
+// What replaces the best so far: a gain within the timer's noise does not.
+bool clearly_faster(double ms, double best) { return ms < 0.99 * best; }
 }  // namespace
 
 int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu, double time, int steps) {
@@ -503,8 +519,8 @@ int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu
   double best_ms[TS_N];
   int best[TS_N];
   for (int q = 0; q < TS_N; q++) { best_ms[q] = 1e300; best[q] = 256; }
-  double best_sweeps = 1e300;  // the three sweeps go in one launch: one size for them
-  int sweeps = 256;
+  const bool ppm = m->p.irec == 5;
+  if (ppm && raishin_model_set_sweep_tiles(m, 0, 0, 0) != 0) return -1;
   const unsigned timing = m->timing;
   for (int cand : TUNE_CANDIDATES) {
     int bs[TS_N];
@@ -524,25 +540,39 @@ int raishin_model_autotune(raishin_model* m, const double* uri, const double* uu
       const double avg = cnt[k] ? ms[k] / (double)cnt[k] : 1e300;
       if (avg < best_ms[q]) { best_ms[q] = avg; best[q] = cand; }
     }
-    const double sum = ms[K_SWEEP1] + ms[K_SWEEP2] + ms[K_SWEEP3];
-    if (cnt[K_SWEEP1] && sum < best_sweeps) { best_sweeps = sum; sweeps = cand; }
   }
-  best[TS_SWEEP1] = best[TS_SWEEP2] = best[TS_SWEEP3] = sweeps;
-  if (raishin_model_set_block_sizes(m, best, TS_N) != 0) return -1;
-  // PPM sweep tiles: the fused sweeps with each tile height along j and k,
-  // the fastest per direction (the split form, slower at every measured
-  // size, is left to explicit choice: members of one batch must agree on it)
-  if (m->p.irec == 5) {
-    const int segs[] = {8, 16, 32};
-    double ms[K_NKINDS];
-    double bj = 1e300, bk = 1e300;
-    int sj = segs[0], sk = segs[0];
-    for (int sgm : segs) {
-      if (raishin_model_set_sweep_tiles(m, 0, sgm, sgm) != 0 || !time_kinds(m, uri, uu, time, steps, ms)) return -1;
-      if (ms[K_SWEEP2] < bj) { bj = ms[K_SWEEP2]; sj = sgm; }
-      if (ms[K_SWEEP3] < bk) { bk = ms[K_SWEEP3]; sk = sgm; }
+  // Sweeps that share a launch, and the fused sweeps' tiles: by whole steps as
+  // they are launched (apart, a sweep's tail and the other sweeps' idle lanes
+  // are not those of the launch they share).  The defaults are timed first and
+  // stay unless something is clearly faster: a tuned model is not slower than
+  // an untuned one (mixed 256x128x128 with k tiles of 32 cells 4.09 ms a step,
+  // of the rule's 16 3.98; 64^3 with 64 0.334, the rule's 32 0.343).
+  double least = 1e300, t = 0.0;
+  if (sweeps_one_launch(m->G, m->p.irec)) {
+    int plan[TS_N];
+    for (int q = 0; q < TS_N; q++) plan[q] = 256;
+    if (raishin_model_set_block_sizes(m, plan, TS_N) != 0 || !time_steps(m, uri, uu, time, steps, &least)) return -1;
+    for (int cand : TUNE_CANDIDATES) {
+      best[TS_SWEEP1] = best[TS_SWEEP2] = best[TS_SWEEP3] = cand;
+      if (raishin_model_set_block_sizes(m, best, TS_N) != 0 || !time_steps(m, uri, uu, time, steps, &t)) return -1;
+      if (clearly_faster(t, least)) { least = t; std::copy(best, best + TS_N, plan); }
     }
-    if (raishin_model_set_sweep_tiles(m, 0, sj, sk) != 0) return -1;
+    std::copy(plan, plan + TS_N, best);
+  }
+  if (raishin_model_set_block_sizes(m, best, TS_N) != 0) return -1;
+  if (ppm) {
+    int seg[2] = {0, 0};
+    for (int d = m->G.jfix ? 1 : 0; d < 2; d++) {  // a collapsed model's j sweep has no tile
+      int keep = 0;
+      for (int cand : {8, 16, 32, 64}) {
+        if (!psweep_fills(m->G, 2 + d, cand)) continue;
+        seg[d] = cand;
+        if (raishin_model_set_sweep_tiles(m, 0, seg[0], seg[1]) != 0 || !time_steps(m, uri, uu, time, steps, &t)) return -1;
+        if (clearly_faster(t, least)) { least = t; keep = cand; }
+      }
+      seg[d] = keep;
+    }
+    if (raishin_model_set_sweep_tiles(m, 0, seg[0], seg[1]) != 0) return -1;
   }
   // start again from the given state, as if no step had been taken
   raishin_model_set_state(m, uri, uu, time);

@@ -64,8 +64,8 @@ struct Geo {
   // workgroup size per tuned launch slot (TuneSlot in rh_kernels.hpp);
   // 0 means 256.  Chosen by raishin_model_autotune or set by the caller.
   unsigned short bs[8];
-  // PPM sweeps (irec 5): cells per wave along j and k of the fused sweep's
-  // tile (0: by rule), and ppm_split = 1 for the split form (face values
+  // PPM sweeps (irec 5): cells along j and k of the fused sweep's tile (0: by
+  // rule), and ppm_split = 1 for the split form (face values
   // through HBM in their own kernel).  Chosen by the autotuner or set by the
   // caller (raishin_model_set_sweep_tiles); results never depend on them.
   unsigned short seg[2];

@@ -2459,16 +2459,19 @@ static void psweep_extent(const Geo& G, int dir, long long& along, long long& li
 // along the axis (3 of them overlap the next tile) by bt / tp lines.
 //  D = 1: the whole workgroup along the row, or 16, 32 or 64 cells of several
 //  rows, whichever leaves the fewest idle or overlapping lanes.
-//  D = 2, 3: a wave holds seg cells along the axis by 64 / seg consecutive i
-//  and the workgroup's waves are stacked along the axis.  seg as set by the
-//  caller, else along j the one with the fewest such lanes among 2 to 16, and
-//  along k 4, or 8 where that has fewer and still two waves per SIMD (1024 of
-//  them): along j a tile's cells share their face metric, along k every (i, k)
-//  has its own, read in runs of 64 / seg (seg 4, 8, 16: 256x128x128 0.373,
-//  0.406, 0.370 ms, mixed 0.202, 0.242, 0.250; 64^3, fewer lanes at 8, 28.0,
-//  25.7, 26.1 us; 251x57x77 89, 90, 119 us; one 64x64 row, with half the
-//  workgroups at 8, 12.4, 16.7, 13.4 us).  Never taller than the axis needs (Riemann tubes' four transverse
-//  interfaces), never below the 4 cells that give an interface.
+//  D = 2, 3: a wave holds w cells along the axis by 64 / w consecutive i and
+//  the workgroup's waves are stacked along the axis.  As set by the caller
+//  (Geo::seg, the tile's cells), else along j the w with the fewest such lanes
+//  among 2 to 16, and along k 4, or 8 where that has fewer and still two waves
+//  per SIMD (1024 of them): along j a tile's cells share their face metric,
+//  along k every (i, k) has its own, read in runs of 64 / w (w 4, 8, 16:
+//  256x128x128 0.373, 0.406, 0.370 ms, mixed 0.202, 0.242, 0.250; 64^3, fewer
+//  lanes at 8, 28.0, 25.7, 26.1 us; 251x57x77 89, 90, 119 us; one 64x64 row,
+//  with half the workgroups at 8, 12.4, 16.7, 13.4 us).  Never below a tile of
+//  8 cells, 5 interfaces (64 threads, with a k tile of 4 and one interface:
+//  one 128x128 row 76.7 -> 71.8 us a step, 40x24x40 146.7 -> 136.3), unless
+//  the axis needs no more (Riemann tubes' four transverse interfaces), and
+//  never below the 4 that give an interface.
 static int psweep_tp(const Geo& G, int dir, int bt) {
   long long along, lines, across;
   psweep_extent(G, dir, along, lines, across);
@@ -2481,28 +2484,37 @@ static int psweep_tp(const Geo& G, int dir, int bt) {
       if (tp < bt && lanes(tp, bt / tp) < lanes(best, bt / best)) best = tp;
     return best;
   }
-  const int nw = bt / 64;
-  int seg = G.seg[dir - 2];
-  if (!seg) {
-    if (dir == 2) {
-      seg = 16;
-      for (int sg : {8, 4, 2})
-        if (sg * nw >= 8 && lanes(sg * nw, 64 / sg) < lanes(seg * nw, 64 / seg)) seg = sg;
-    } else {
-      const long long l4 = lanes(4 * nw, 16), l8 = lanes(8 * nw, 8);
-      seg = l8 < l4 && l8 * across >= 2 * 64 * 1024 ? 8 : 4;
-    }
+  const int nw = bt / 64, want = G.seg[dir - 2];
+  int w;
+  if (want) {  // the tallest tile no taller than that
+    for (w = 1; 2 * w * nw <= want;) w *= 2;
+  } else if (dir == 2) {
+    w = 16;
+    for (int q : {8, 4, 2})
+      if (q * nw >= 8 && lanes(q * nw, 64 / q) < lanes(w * nw, 64 / w)) w = q;
+  } else {
+    const long long l4 = lanes(4 * nw, 16), l8 = lanes(8 * nw, 8);
+    w = nw == 1 || (l8 < l4 && l8 * across >= 2 * 64 * 1024) ? 8 : 4;
   }
-  while (seg > 1 && seg * nw / 2 >= 4 && seg * nw / 2 - 3 >= along) seg /= 2;
-  while (seg * nw < 4) seg *= 2;
-  return seg * nw;
+  while (w > 1 && w * nw / 2 >= 4 && w * nw / 2 - 3 >= along) w /= 2;
+  while (w * nw < 4) w *= 2;
+  return w * nw;
 }
 
-// Cells along j or k that a wave of the sweep's tile holds, as a size that can
-// be asked for: where the rule comes to one cell it comes there from two too.
+// The sweep's tile along j or k as a size that can be asked for: its cells, a
+// power of two (three waves make tiles of three quarters of one).
 int psweep_segment(const Geo& G, int dir) {
-  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
-  return std::max(2, psweep_tp(G, dir, bt) / (bt / 64));
+  const int tp = psweep_tp(G, dir, slot_threads(G, TS_SWEEP1 + dir - 1));
+  int seg = 4;
+  while (seg < tp) seg *= 2;
+  return seg;
+}
+
+// Whether the axis fills three quarters of a tile of seg cells along dir.
+bool psweep_fills(const Geo& G, int dir, int seg) {
+  long long along, lines, across;
+  psweep_extent(G, dir, along, lines, across);
+  return 4 * along >= 3 * (seg - 3);
 }
 
 size_t psweep_lds_bytes(int threads, bool mixed) { return (size_t)18 * threads * (mixed ? sizeof(float) : sizeof(double)); }

@@ -204,9 +204,8 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, boo
 // PPM (irec 5) sweep along dir with the face values computed in the same
 // kernel (through LDS): reads W and the direction's PPM width coefficients
 // pc, writes what launch_edges + launch_sweep write to F and CTsrc.
-// seg: cells along j or k per wave of the fused sweep (64 / seg consecutive
-// i per wave; a workgroup's waves are stacked along the axis), a power of two
-// from 2 to 64
+// seg: cells along j or k of the fused sweep's tile (a workgroup; by threads /
+// seg consecutive i), a power of two from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
 hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A, bool mixed, hipStream_t st);
 // The three in one launch (s[d]: the sweep along d + 1), with the CFL
@@ -219,6 +218,7 @@ hipError_t launch_sweep3(const Geo& G, int irec, const SweepArgs s[3], bool mixe
                          hipStream_t st);
 hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st);
 int psweep_segment(const Geo& G, int dir);
+bool psweep_fills(const Geo& G, int dir, int seg);
 size_t psweep_lds_bytes(int threads, bool mixed);
 // f32: CTsrc and F hold floats (the averages are formed in double either way)
 hipError_t launch_fluxct(const Geo& G, const void* CTsrc, void* F1, void* F2, void* F3, bool f32, double* CTd,

@@ -35,3 +35,30 @@ def test_batch_of_mc_and_split_ppm():
     b.close()
     for mm in alone + batched + [w]:
         mm.close()
+
+
+@pytest.mark.parametrize("threads", [64, 128, 256])
+@pytest.mark.parametrize("ni,nj,nk", [(40, 24, 40), (64, 64, 64), (251, 57, 77)])
+def test_untuned_tiles_are_ones_the_autotuner_times(ni, nj, nk, threads):
+    """A tile is its cells along the axis (a workgroup's), in the rule as in
+    what can be asked for, so tuning can keep what an untuned model has."""
+    p = configs.Pram("tile", ni, nj, nk, irec=5, irkt=3).resolved()
+    m = native.Model.from_grid(p, native.setup_grid(p))
+    m.set_block_sizes([threads] * 8)
+    for seg in m.sweep_tiles()["seg_j"], m.sweep_tiles()["seg_k"]:
+        assert seg in (8, 16, 32, 64)
+    m.close()
+
+
+@pytest.mark.parametrize("threads,seg", [(256, 4), (256, 2), (192, 4), (128, 2), (64, 64), (192, 64)])
+def test_smallest_and_tallest_tiles_equal_split(threads, seg):
+    p = configs.Pram("tile", 75, 17, 71, irec=5, irkt=3, cfl=0.4)
+    a, b = make(p), make(p)
+    a.set_sweep_tiles(1, 0, 0)
+    b.set_block_sizes([threads] * 8)
+    b.set_sweep_tiles(0, seg, seg)
+    for s in range(2):
+        assert a.step(1) == b.step(1), s
+    same(a, b, threads)
+    a.close()
+    b.close()
