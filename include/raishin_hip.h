@@ -182,7 +182,9 @@ int raishin_model_get_timing(raishin_model *m, double *ms, long long *launches, 
 /* Workgroup sizes of the tuned launches, in the order: PPM face values,
  * sweep i, sweep j, sweep k, flux-CT, RK update, recov1a, ghosts/floors/
  * caluu1 (8 entries; 0 = 256, else 64..256 in steps of 64).  Sweeps that share
- * a launch take sweep i's.  Results do not depend on them.  get returns the
+ * a launch take sweep i's and are reported with it: PPM's unless split, and the
+ * others' where the metric is symmetric and couples theta to nothing
+ * (Kerr-Schild, Minkowski).  Results do not depend on them.  get returns the
  * sizes in use. */
 int raishin_model_set_block_sizes(raishin_model *m, const int *bs, int n);
 int raishin_model_get_block_sizes(raishin_model *m, int *bs, int n);

@@ -440,6 +440,7 @@ int raishin_model_set_block_sizes(raishin_model* m, const int* bs, int n) {
 int raishin_model_get_block_sizes(raishin_model* m, int* bs, int n) {
   if (!m || !bs || n != TS_N) { set_error("raishin_model_get_block_sizes: expected %d sizes", (int)TS_N); return -1; }
   for (int q = 0; q < TS_N; q++) bs[q] = slot_threads(m->G, q);
+  for (int d = 1; d <= 3; d++) bs[TS_SWEEP1 + d - 1] = sweep_threads(m->G, m->p.irec, d);
   return 0;
 }
 

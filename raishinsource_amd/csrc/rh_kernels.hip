@@ -2326,6 +2326,15 @@ hipError_t launch_edges(const Geo& G, int dir, const double* W, const double* dx
   return hipGetLastError();
 }
 
+// Whether a stage's sweeps share a launch where nothing keeps them apart.
+static bool sweeps_share(const Geo& G, int irec) { return irec == 5 ? !G.ppm_split : G.mk != 0; }
+
+bool sweeps_one_launch(const Geo& G, int irec) { return sweeps_share(G, irec) && (irec == 5 || !g_rec); }
+
+int sweep_threads(const Geo& G, int irec, int dir) {
+  return slot_threads(G, sweeps_share(G, irec) ? TS_SWEEP1 : TS_SWEEP1 + dir - 1);
+}
+
 void record_no_edges(const Geo& G) {
   if (g_rec) record(LK_EDGES, 0, 256, 0, G, AnyArgs{});
 }
@@ -2410,7 +2419,7 @@ static void with_sweep(int variant, F&& f) {
 
 hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, bool mixed, hipStream_t st) {
   const long long n = box(G.nm0, G.ni - G.nm0) * jbox(G, G.nm0, G.nj - G.nm0) * box(G.nm0, G.nk - G.nm0);
-  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
+  const int bt = sweep_threads(G, irec, dir);
   const unsigned nb = nblk(n, bt);
   if (g_rec) {
     AnyArgs a{};
@@ -2504,7 +2513,7 @@ static int psweep_tp(const Geo& G, int dir, int bt) {
 // The sweep's tile along j or k as a size that can be asked for: its cells, a
 // power of two (three waves make tiles of three quarters of one).
 int psweep_segment(const Geo& G, int dir) {
-  const int tp = psweep_tp(G, dir, slot_threads(G, TS_SWEEP1 + dir - 1));
+  const int tp = psweep_tp(G, dir, slot_threads(G, TS_SWEEP1));  // fused sweeps share a launch
   int seg = 4;
   while (seg < tp) seg *= 2;
   return seg;
@@ -2557,7 +2566,7 @@ static long long psweep_args(const Geo& G, int dir, int bt, PSweepArgs& A) {
 }
 
 hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A0, bool mixed, hipStream_t st) {
-  const int bt = slot_threads(G, TS_SWEEP1 + dir - 1);
+  const int bt = sweep_threads(G, 5, dir);
   const bool self = dir == 2 && G.jfix;
   PSweepArgs A = A0;
   const unsigned nb = (unsigned)psweep_args(G, dir, bt, A);
@@ -2587,8 +2596,6 @@ static void with_psweep3(int variant, F&& f) {
     });
   });
 }
-
-bool sweeps_one_launch(const Geo& G, int irec) { return irec == 5 ? !G.ppm_split : G.mk && !g_rec; }
 
 hipError_t launch_sweep3(const Geo& G, int irec, const SweepArgs s[3], bool mixed, const CflArgs* cfl,
                          hipStream_t st) {

@@ -208,12 +208,15 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, boo
 // seg consecutive i), a power of two from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
 hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A, bool mixed, hipStream_t st);
-// The three in one launch (s[d]: the sweep along d + 1), with the CFL
-// reduction of the same primitives when cfl is given; its workgroups' results
-// are then combined by the launch_fluxct that is given the same cfl.
 // Whether a stage's sweeps go in one launch: PPM's (not the split form's)
 // always, the others' where that is built (compact metric tables, no batch).
 bool sweeps_one_launch(const Geo& G, int irec);
+// Workgroup size of the sweep along dir.  Where the sweeps share a launch that
+// is sweep i's, also while they are timed apart or recorded for a batch.
+int sweep_threads(const Geo& G, int irec, int dir);
+// The three in one launch (s[d]: the sweep along d + 1), with the CFL
+// reduction of the same primitives when cfl is given; its workgroups' results
+// are then combined by the launch_fluxct that is given the same cfl.
 hipError_t launch_sweep3(const Geo& G, int irec, const SweepArgs s[3], bool mixed, const CflArgs* cfl,
                          hipStream_t st);
 hipError_t launch_psweep3(const Geo& G, const PSweepArgs s[3], bool mixed, const CflArgs* cfl, hipStream_t st);

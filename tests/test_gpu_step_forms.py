@@ -62,3 +62,35 @@ def test_smallest_and_tallest_tiles_equal_split(threads, seg):
     same(a, b, threads)
     a.close()
     b.close()
+
+
+def general_metric(p):
+    """A model whose metric has not the compact tables' structure: a zero of
+    the centre metric negated, which keeps every value."""
+    p = p.resolved()
+    g = native.setup_grid(p)
+    m = native.setup_metric(p, g)
+    m["gcov"][0, 3] = -0.0
+    mod = native.Model(p, g, m)
+    mod.set_state(native.setup_torus(p, g, native.setup_metric(p, g), seed=1, noise=0.02))
+    return mod
+
+
+def test_sizes_and_tiles_reported_are_those_in_use():
+    """Sweeps that share a launch have one workgroup size, sweep i's: the
+    sizes read back say so, and the tiles are those of that size."""
+    odd = [256, 64, 192, 128, 64, 192, 128, 64]
+    a, b = make(configs.T3D_PPM), make(configs.T3D_PPM)
+    a.set_block_sizes(odd)
+    b.set_block_sizes([256, 64, 64, 64, 64, 192, 128, 64])
+    assert a.block_sizes() == b.block_sizes()
+    assert a.sweep_tiles() == b.sweep_tiles()
+    a.set_sweep_tiles(1, 0, 0)  # the split form's sweeps are launches of their own
+    assert list(a.block_sizes().values()) == odd
+    a.close()
+    b.close()
+    c, d = make(configs.U_MP5), general_metric(configs.U_MP5)
+    for mm, want in ((c, [64, 64, 64]), (d, [64, 192, 128])):
+        mm.set_block_sizes(odd)
+        assert [mm.block_sizes()[k] for k in ("sweep_i", "sweep_j", "sweep_k")] == want
+        mm.close()
