@@ -156,7 +156,8 @@ void raishin_model_set_precision(raishin_model *m, int mode);
  * 5 in-order recovery fix-up; 6 ghosts/floors/caluu1; 7 CFL reduction;
  * 8 PPM face values (irec=5, all three directions); 9 recov1a.
  * Kind 4 includes the recovery where the step does both in one kernel (a
- * symmetric metric); kind 9 then has no launches.  A step that times a sweep
+ * symmetric metric that couples theta to nothing, as Kerr-Schild and Minkowski,
+ * with symmetric Christoffel symbols); kind 9 then has no launches.  A step that times a sweep
  * or the CFL reduction launches them apart, otherwise they share launches.
  * set_timing(1) clears the totals and starts recording; get_timing returns
  * the number of kinds and fills total milliseconds and launch counts. */

@@ -2717,6 +2717,8 @@ static bool with_rkrecov(int variant, F&& f) {
   return true;
 }
 
+bool update_recov_one_launch(const Geo& G, bool chr_sym) { return (G.mk && chr_sym) || g_rec; }
+
 hipError_t launch_update_recov(const Geo& G, int stage, const StageArgs& A, hipStream_t st) {
   const long long n = box(G.nm1 + 1, G.ni - G.nm1) * jbox(G, G.nm1 + 1, G.nj - G.nm1) * box(G.nm1 + 1, G.nk - G.nm1);
   const int bt = slot_threads(G, TS_RK);
@@ -2724,12 +2726,10 @@ hipError_t launch_update_recov(const Geo& G, int stage, const StageArgs& A, hipS
   const int variant = rk_variant(G, stage, A) + 64 * (G.iwvec == 2);
   if (g_rec) { AnyArgs a{}; a.st = A; record(LK_RKRECOV, variant, bt, nb, G, a); return hipSuccess; }
   if (n == 0) return hipSuccess;
-  if (with_rkrecov(variant, [&](auto S, auto T, auto I) {
-        hipLaunchKernelGGL((k_rkrecov<S.value, typename decltype(T)::type, I.value>), dim3(nb), dim3(bt), 0, st, G, A);
-      }))
-    return hipGetLastError();
-  const hipError_t e = launch_update(G, stage, A, st);
-  return e == hipSuccess ? launch_recov(G, A, st) : e;
+  const bool built = with_rkrecov(variant, [&](auto S, auto T, auto I) {
+    hipLaunchKernelGGL((k_rkrecov<S.value, typename decltype(T)::type, I.value>), dim3(nb), dim3(bt), 0, st, G, A);
+  });
+  return built ? hipGetLastError() : hipErrorInvalidValue;
 }
 
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st) {

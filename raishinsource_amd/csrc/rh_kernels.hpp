@@ -231,8 +231,11 @@ hipError_t launch_retype(const void* src, void* dst, long long n, bool to_float,
 // RK update + sources into A.Ukeep (every interior cell), then recov1a into A.Wpre.
 hipError_t launch_update(const Geo& G, int stage, const StageArgs& A, hipStream_t st);
 hipError_t launch_recov(const Geo& G, const StageArgs& A, hipStream_t st);
-// Both, fused where it is built: A.Ukeep then holds only the cells left to
-// launch_recov_carry.
+// Both in one kernel, where that is built (compact metric tables, symmetric
+// Christoffel tables): A.Ukeep then holds only the cells left to
+// launch_recov_carry.  A batch's record is one in any case; its other members
+// get both kernels there, in the update's workgroup size.
+bool update_recov_one_launch(const Geo& G, bool chr_sym);
 hipError_t launch_update_recov(const Geo& G, int stage, const StageArgs& A, hipStream_t st);
 hipError_t launch_recov_carry(const Geo& G, const FixArgs& A, hipStream_t st);
 hipError_t launch_post(const Geo& G, const PostArgs& A, hipStream_t st);

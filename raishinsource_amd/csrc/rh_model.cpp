@@ -578,7 +578,7 @@ bool stage_update(raishin_model* m, int rkstage, const double* W, const double* 
   // the atmosphere of models 7..15 sets the entropy variable to zero whatever
   // the recovery gave (a pow of some 230 instructions)
   A.s5 = !inner || m->p.model < 7 || m->p.model > 15;
-  if (!inner) {
+  if (!inner || !update_recov_one_launch(G, m->chr_sym)) {
     { TimedLaunch t(m, K_UPDATE); HIPCHK(launch_update(G, rkstage, A, m->st)); }
     { TimedLaunch t(m, K_RECOV); HIPCHK(launch_recov(G, A, m->st)); }
   } else {

@@ -64,15 +64,20 @@ def test_smallest_and_tallest_tiles_equal_split(threads, seg):
     b.close()
 
 
-def general_metric(p):
-    """A model whose metric has not the compact tables' structure: a zero of
-    the centre metric negated, which keeps every value."""
+def general_metric(p, table="gcov", mixed=False, seed=1):
+    """A model whose metric has not the compact tables' structure, or whose
+    Christoffel tables are not symmetric: a zero of one table negated, which
+    keeps every value."""
     p = p.resolved()
     g = native.setup_grid(p)
     m = native.setup_metric(p, g)
-    m["gcov"][0, 3] = -0.0
+    uri = native.setup_torus(p, g, m, seed=seed, noise=0.02)
+    at = (0, 3) if table == "gcov" else (3, 2, 3)
+    assert not m[table][at].any()
+    m[table][at] = -0.0
     mod = native.Model(p, g, m)
-    mod.set_state(native.setup_torus(p, g, native.setup_metric(p, g), seed=1, noise=0.02))
+    mod.set_state(uri)
+    mod.set_precision(mixed)
     return mod
 
 
@@ -93,4 +98,41 @@ def test_sizes_and_tiles_reported_are_those_in_use():
     for mm, want in ((c, [64, 64, 64]), (d, [64, 192, 128])):
         mm.set_block_sizes(odd)
         assert [mm.block_sizes()[k] for k in ("sweep_i", "sweep_j", "sweep_k")] == want
+        mm.close()
+
+
+@pytest.mark.parametrize("table", ["gcov", "christ"])
+def test_recovery_timed_where_it_is_a_kernel_of_its_own(table):
+    """Kind 4 (update) and kind 9 (recov) of a model whose step makes a launch
+    of each; the autotuner then has samples of both."""
+    a, b = make(configs.U_PPM, seed=1), general_metric(configs.U_PPM, table)
+    for mm, recov in ((a, 0), (b, 6)):
+        mm.set_timing(True)
+        mm.step(3)
+        t = mm.get_timing()
+        assert t["update"][1] == 6 and t["recov"][1] == recov, t
+    same(a, b, table)
+    a.close()
+    b.close()
+
+
+def test_general_tables_in_a_batch():
+    """Members with general metric tables or asymmetric Christoffel tables (two
+    kernels at the place of the others' one) beside one with neither."""
+    members = [("gcov", False), ("christ", False), ("gcov", True), ("christ", True)]
+    def build():
+        return [general_metric(configs.U_PPM, t, mx, q) for q, (t, mx) in enumerate(members)] + [
+            make(configs.T2D, seed=4), general_metric(replace(configs.T2D, name="t2d_rc2", iwvec=2), "gcov", False, 5)]
+    alone, batched = build(), build()
+    for mm in alone:
+        mm.step(4)
+    b = native.Batch(batched)
+    b.step(1)
+    b.step_graph(1)
+    b.step(1)
+    for q, (x, y) in enumerate(zip(alone, batched)):
+        same(x, y, q)
+    b.set([])
+    b.close()
+    for mm in alone + batched:
         mm.close()
