@@ -2196,13 +2196,6 @@ kb_sweep(const BatchItem* __restrict__ it, int n) {
   const SweepArgs A = it[q].A.s;
   b_sweep<D, IREC, R, ICHA, MK>(G, A, blk);
 }
-template <int D, class R, int ICHA, bool MK>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
-kb_psweep(const BatchItem* __restrict__ it, int n) {
-  RH_BATCH_PROLOGUE
-  const PSweepArgs A = it[q].A.ps;
-  b_psweep<D, R, ICHA, MK>(G, A, blk);
-}
 template <class R, int ICHA, bool MK, bool COLL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, 5>)))
 kb_psweep3(const BatchItem* __restrict__ it, int n) {
@@ -2291,13 +2284,6 @@ static void record(int kind, int variant, int threads, long long nb, const Geo& 
   LaunchRec r;
   r.kind = kind; r.variant = variant; r.threads = threads; r.nb = nb; r.G = G; r.A = A;
   g_rec->push_back(r);
-}
-
-int block_threads(int kind) {
-  switch (kind) {
-    case LK_CARRY: return 1024;
-    default: return 256;
-  }
 }
 
 bool one_group_per_model(int kind) { return kind == LK_CARRY || kind == LK_CFL_FINISH; }
@@ -2571,12 +2557,6 @@ hipError_t launch_psweep(const Geo& G, int dir, const PSweepArgs& A0, bool mixed
   PSweepArgs A = A0;
   const unsigned nb = (unsigned)psweep_args(G, dir, bt, A);
   const int variant = psweep_variant(self ? 0 : dir, mixed, G);
-  if (g_rec) {
-    AnyArgs a{};
-    a.ps = A;
-    record(LK_PSWEEP, variant, bt, nb, G, a);
-    return hipSuccess;
-  }
   if (nb == 0) return hipSuccess;
   const size_t lds = self ? 0 : psweep_lds_bytes(bt, mixed);
   with_psweep(variant, [&](auto D, auto T, auto C, auto K) {
@@ -2817,13 +2797,6 @@ hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* i
         hipLaunchKernelGGL((kb_sweep<D.value, I.value, typename decltype(T)::type, C.value, K.value>), g, b, 0, st, it, n);
       });
       break;
-    case LK_PSWEEP: {
-      const size_t lds = (variant & 3) ? psweep_lds_bytes(threads, (variant & 4) != 0) : 0;
-      with_psweep(variant, [&](auto D, auto T, auto C, auto K) {
-        hipLaunchKernelGGL((kb_psweep<D.value, typename decltype(T)::type, C.value, K.value>), g, b, lds, st, it, n);
-      });
-      break;
-    }
     case LK_PSWEEP3:
       with_psweep3(variant, [&](auto T, auto C, auto K, auto L) {
         hipLaunchKernelGGL((kb_psweep3<typename decltype(T)::type, C.value, K.value, L.value>), g, b,

@@ -141,13 +141,12 @@ inline int slot_threads(const Geo& G, int slot) { return G.bs[slot] ? (int)G.bs[
 // Launch kinds of one step, in the order run_step makes them.
 enum LaunchKind {
   LK_EDGES, LK_SWEEP, LK_FLUXCT, LK_RKRECOV, LK_CARRY, LK_BND, LK_POST, LK_CFL, LK_CFL_FINISH,
-  LK_COPY, LK_PSWEEP, LK_PSWEEP3, LK_N
+  LK_COPY, LK_PSWEEP3, LK_N
 };
 
 union AnyArgs {
   EdgeArgs e;
   SweepArgs s;
-  PSweepArgs ps;
   PSweep3Args ps3;
   CtArgs c;
   StageArgs st;
@@ -182,7 +181,6 @@ void set_recorder(std::vector<LaunchRec>* r);
 // workgroups; for one-workgroup-per-model kinds, n).
 hipError_t launch_batched(int kind, int variant, int threads, const BatchItem* items, int n, long long total_blocks,
                           hipStream_t st);
-int block_threads(int kind);
 // dst[q] = src[q][0] for q < n (the members' times of a batch)
 hipError_t launch_gather_first(const double* const* src, double* dst, int n, hipStream_t st);
 bool one_group_per_model(int kind);
@@ -204,6 +202,7 @@ hipError_t launch_sweep(const Geo& G, int dir, int irec, const SweepArgs& A, boo
 // PPM (irec 5) sweep along dir with the face values computed in the same
 // kernel (through LDS): reads W and the direction's PPM width coefficients
 // pc, writes what launch_edges + launch_sweep write to F and CTsrc.
+// For a model whose sweeps are timed apart; a batch records launch_psweep3.
 // seg: cells along j or k of the fused sweep's tile (a workgroup; by threads /
 // seg consecutive i), a power of two from 2 to 64
 inline bool psweep_seg_ok(int seg) { return seg >= 2 && seg <= 64 && (seg & (seg - 1)) == 0; }
