@@ -125,9 +125,10 @@ void raishin_model_cdtcfl4(raishin_model *m, double *dtcfl, double *dt1, double 
  * doubles in device memory, written in order on the model's stream with
  * dtcfl, dt1, dt2, dt3 (bit-identical to raishin_model_cdtcfl4).  The
  * per-workgroup partials go to one fixed 8 MiB device array per GPU (the
- * library's, held until the process ends) instead of the model's buffers:
- * models of up to 131072 * 256 CFL cells ((imax-2)(jmax-2)(kmax-2) rounded
- * up per 256); larger ones are rejected with an error.  The array needs no
+ * library's, held until the process ends) instead of the model's buffers.
+ * Models of up to 131072 * 256 CFL cells ((imax-2)(jmax-2)(kmax-2) rounded
+ * up per 256) are taken, which is this entry's limit and not the
+ * reduction's (it has 1024 partials at most); larger ones are rejected with an error.  The array needs no
  * clearing (every call writes what it reads); calls that overlap on one GPU
  * race on it, so order them (one stream, or events).  The model's device
  * must be current.  Returns 0, or -1 with raishin_last_error set. */

@@ -13,7 +13,8 @@
 namespace {
 
 // Per-workgroup partials of k_cfl: 4 positions (long long) then 4 minima
-// (double) per workgroup, for at most NOALLOC_CFL_BLOCKS workgroups.
+// (double) per workgroup.  Room for, and the entry's limit, one per 256 cells;
+// launch_cfl uses CFL_GROUPS of them at most.
 constexpr long long NOALLOC_CFL_BLOCKS = 131072;
 constexpr size_t SCRATCH_BYTES = (size_t)NOALLOC_CFL_BLOCKS * 4 * (sizeof(long long) + sizeof(double));
 static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
@@ -45,11 +46,11 @@ extern "C" int raishin_model_cdtcfl4_noalloc(raishin_model* m, double* out) {
     rhm::set_error("raishin_model_cdtcfl4_noalloc: out is not aligned to 8 bytes");
     return -1;
   }
-  const long long nb = cfl_blocks(m->G);
+  const long long nb = cfl_blocks(m->G);  // the limit is by cells, not by what is launched
   if (nb > NOALLOC_CFL_BLOCKS) {
-    rhm::set_error("raishin_model_cdtcfl4_noalloc: the model needs %lld CFL workgroups (%lld cells), over the "
-                   "fixed scratch's %lld; use raishin_model_cdtcfl4",
-                   nb, nb * 256, NOALLOC_CFL_BLOCKS);
+    rhm::set_error("raishin_model_cdtcfl4_noalloc: the model has %lld chunks of 256 CFL cells, over the "
+                   "fixed scratch's limit of %lld; use raishin_model_cdtcfl4",
+                   nb, NOALLOC_CFL_BLOCKS);
     return -1;
   }
   int dev = -1;
