@@ -214,11 +214,13 @@ int raishin_model_set_divb_form(raishin_model *m, int form);
  * whole steps in a graph of two decides on that against the default sizes, on
  * one size for the sweeps and, for PPM, on a tile of 8, 16, 32 or 64 cells
  * along j and along k (where the axis fills three quarters of it): the
- * defaults stay unless something is faster by
- * more than 1% (the split form is never chosen: it is slower
- * at every size measured, and members of a batch must agree on the form);
- * then it sets the state again and clears the counters, so the run
- * starts as if untuned.  Returns 0 or -1. */
+ * defaults stay unless something is faster in each of three runs and by more
+ * than 0.2% in all (the split form is never chosen: it is slower at every size
+ * measured, and members of a batch must agree on the form).  The times are
+ * those of the model alone; a batch's members share a launch only where their
+ * sizes agree, and one of many shapes can be faster untuned.  Then it sets the
+ * state again and clears the counters, so the run starts as if untuned.
+ * Returns 0 or -1. */
 int raishin_model_autotune(raishin_model *m, const double *uri, const double *uu, double time, int steps);
 
 /* Axisymmetric models with one interior phi cell (jmax = 2*nm1+1), periodic
