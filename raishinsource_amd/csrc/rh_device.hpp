@@ -105,10 +105,11 @@ struct MetG {
 // t-phi entry of gcon zero) -- Kerr-Schild and Minkowski: the entries that
 // are left and the derived values, in the arithmetic type R.  The zeros stay
 // in the arithmetic as constants (a product with an infinity is still not a
-// number), so results are those of the general tables bit for bit; 13 planes
-// are read where the general form reads 33 and takes a square root and five
-// divisions (256x128x128: i, j, k sweeps 0.306, 0.330, 0.396 -> 0.288, 0.302,
-// 0.374 ms in FP64, 0.166, 0.198, 0.236 -> 0.136, 0.168, 0.202 ms mixed;
+// number), so results are those of the general tables bit for bit; a face's
+// table is 14 planes and the centre's 20, where the general form has 33 and
+// takes a square root and five divisions besides (256x128x128: i, j, k sweeps
+// 0.306, 0.330, 0.396 -> 0.288, 0.302, 0.374 ms in FP64, 0.166, 0.198, 0.236
+// -> 0.136, 0.168, 0.202 ms mixed;
 // floors 0.305 -> 0.238, recovery 0.184 -> 0.163 ms).
 enum { MK_G00, MK_G01, MK_G02, MK_G11, MK_G12, MK_G22, MK_G33, MK_DETG, MK_ALPHA, MK_RALPHA, MK_BETA1,
        MK_GI3_1, MK_GI3_2, MK_GI3_3, MK_FACE_PLANES,
